@@ -316,6 +316,42 @@ typedef struct gh_adam_tensor {
 int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, float lr, float beta1, float beta2, float eps,
                  int32_t step, void *stream);
 
+/* The same step, which also writes a transposed bf16 copy of a tensor: transposed[c ld + r] =
+ * bf16(param[r][c]) for every r < rows, c < cols (rows a multiple of 8, ld >= rows a multiple
+ * of 8, 16-byte aligned; NULL: none). It is the weight layout of gh_mlp_forward_bf16. packs:
+ * n_tensors entries, or NULL. */
+typedef struct gh_adam_pack {
+  void *transposed;
+  int32_t ld;
+  int32_t reserved;
+} gh_adam_pack;
+int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors, float lr,
+                        float beta1, float beta2, float eps, int32_t step, void *stream);
+
+/* Training passes of a whole dense network (no counterpart in the reference's source, as for
+ * gh_adam_step), for the networks of gh_mlp_forward_bf16 whose input width k_in and padded
+ * output width np (8 or 16) are multiples of 8. At most GH_MLP_TRAIN_MAX_ROWS rows; every
+ * pointer but G and Z 16-byte aligned.
+ * Forward: X: M x k_in bf16 (contiguous); wt, bias as in gh_mlp_forward_bf16; Y[l]: the hidden
+ * activations bf16(relu(Z_l)), M x hidden, kept for the backward pass; Z: FP32 output, columns
+ * 0..n_out-1. Same values as the layer-by-layer gh_gemm_bf16 path, bit for bit.
+ * Backward: w[l] (l >= 1): bf16 weights [K_l][N_l] row-major (N of the last layer = np); G:
+ * dLoss/dZ, M x n_out FP32 with row pitch ldg. dW: the FP32 weight gradients of all layers one
+ * after the other, each K_l x N_l; db: the bias gradients, hidden per hidden layer, then np.
+ * The column sums are taken over the FP32 gradients, the products over their bf16 roundings
+ * (dW: the bits of gh_gemm_bf16). G32, if not NULL, receives the FP32 gradients of the hidden
+ * layers, M x hidden each.
+ * ws: device memory of the bytes gh_mlp_train_workspace gives, free again when the launches have
+ * run. */
+#define GH_MLP_TRAIN_MAX_ROWS 4194240
+int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t n_out,
+                              const void *const *wt, const float *const *bias, void *const *Y, float *Z, int64_t ldz,
+                              void *stream);
+int gh_mlp_train_workspace(int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t np, int64_t *bytes);
+int gh_mlp_train_backward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t n_out,
+                               int32_t np, const void *const *w, const void *const *Y, const float *G, int64_t ldg,
+                               float *dW, float *db, float *const *G32, void *ws, int64_t ws_bytes, void *stream);
+
 /* Learned exit-plane source (replaces the generator call of GANSourceDefaultGenerator.generator,
  * sources/gansources.py:644-684, and its copy/move of the keys, :686-757).
  * gh_gaussian_bf16: out[r*ld + c] = N(0,1) noise in bf16 for rows first_row .. first_row+n_rows-1

@@ -32,6 +32,7 @@
 #include <string>
 
 #include "../../include/gatehip.h"
+#include "splitk.h"
 
 namespace {
 
@@ -39,7 +40,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 64, BN = 64, BK = 32;
+constexpr int BM = gh::GEMM_BM, BN = gh::GEMM_BN, BK = gh::GEMM_BK;
+using gh::splitk_plan;
 constexpr int LDK = BK + 8;  // LDS row pitch in bf16 (16-byte aligned rows, fewer bank conflicts)
 
 __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
@@ -197,21 +199,6 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *__restr
     float acc = 0.0f;
     for (int z = 0; z < S; ++z) acc += part[(int64_t)z * stride + i];
     C32[(int64_t)m * ldc + n] = acc;
-  }
-}
-
-// split-K plan of a GEMM: S slices of kc (a multiple of BK) reduction elements each;
-// S = 1 means no split. Weight gradients (few output tiles, long reduction) are split so
-// that the launch fills the chip; the slices are then summed in a fixed order.
-void splitk_plan(int M, int N, int K, int mode, int &S, int &kc) {
-  const int tiles = ((N + BN - 1) / BN) * ((M + BM - 1) / BM);
-  S = 1;
-  kc = ((K + BK - 1) / BK) * BK;
-  if (mode == GH_EPI_STORE && tiles < 512 && K >= 2048) {
-    S = std::max(1, std::min((K + 511) / 512, std::max(1, 1024 / tiles)));
-    kc = (K + S - 1) / S;
-    kc = (kc + BK - 1) / BK * BK;
-    S = (K + kc - 1) / kc;
   }
 }
 
@@ -834,20 +821,41 @@ extern "C" int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_
 
 // ------------------------------------------------------------------ optimiser
 // One Adam step over every parameter tensor of a network in one launch (the training loop
-// otherwise issues about ten elementwise kernels per tensor). Entry e of the flattened
-// launch belongs to tensor i with offset[i] <= e < offset[i+1]; inside the tensor's
-// valid_rows x valid_cols corner it takes the Adam update (with L2 weight decay added to the
-// gradient when decay != 0), outside it the parameter and both moments stay
-// zero (the padding of the bf16 GEMM operands). The bf16 copy, when given, is the parameter
-// rounded to nearest even, ready for the next forward pass.
+// otherwise issues about ten elementwise kernels per tensor). Inside a tensor's valid_rows x
+// valid_cols corner an entry takes the Adam update (with L2 weight decay added to the
+// gradient when decay != 0), outside it the parameter and both moments stay zero (the
+// padding of the bf16 GEMM operands). The bf16 copy, when given, is the parameter rounded to
+// nearest even, ready for the next forward pass; the transposed copy, when given, holds the
+// same values with the rows of a column contiguous, the layout the fused passes read. A
+// thread of a tensor with a transposed copy takes 8 rows of one column, so that the copy's
+// store is one 16-byte store (2-byte stores at the copy's pitch otherwise).
 namespace {
 constexpr int ADAM_MAX = 32;
 struct AdamArgs {
   gh_adam_tensor t[ADAM_MAX];
-  int64_t offset[ADAM_MAX + 1];
+  gh_adam_pack pack[ADAM_MAX];
+  int64_t offset[ADAM_MAX + 1];   // units: entries, or 8-row strips of one column (transposed copy)
   int n;
   float lr, b1, b2, eps, c1, c2;  // c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
 };
+
+__device__ __forceinline__ float adam_entry(const AdamArgs &a, const gh_adam_tensor &t, int64_t r, int64_t c) {
+  const int64_t j = r * t.cols + c;
+  float p = 0.0f, m = 0.0f, v = 0.0f;
+  if (r < t.valid_rows && c < t.valid_cols) {
+    p = t.param[j];
+    const float g = t.decay != 0.0f ? fmaf(t.decay, p, t.grad[j]) : t.grad[j];
+    m = fmaf(a.b1, t.m[j], (1.0f - a.b1) * g);
+    v = fmaf(a.b2, t.v[j], (1.0f - a.b2) * (g * g));
+    const float mh = m * a.c1, vh = v * a.c2;
+    p -= a.lr * mh / (sqrtf(vh) + a.eps);
+  }
+  t.param[j] = p;
+  t.m[j] = m;
+  t.v[j] = v;
+  if (t.param_bf16) ((__bf16 *)t.param_bf16)[j] = f2bf(p);
+  return p;
+}
 
 __global__ void __launch_bounds__(256) adam_kernel(AdamArgs a) {
   const int64_t total = a.offset[a.n];
@@ -858,25 +866,20 @@ __global__ void __launch_bounds__(256) adam_kernel(AdamArgs a) {
     const gh_adam_tensor &t = a.t[i];
     const int64_t j = e - a.offset[i];
     const int64_t r = j / t.cols, c = j - r * t.cols;
-    float p = 0.0f, m = 0.0f, v = 0.0f;
-    if (r < t.valid_rows && c < t.valid_cols) {
-      p = t.param[j];
-      const float g = t.decay != 0.0f ? fmaf(t.decay, p, t.grad[j]) : t.grad[j];
-      m = fmaf(a.b1, t.m[j], (1.0f - a.b1) * g);
-      v = fmaf(a.b2, t.v[j], (1.0f - a.b2) * (g * g));
-      const float mh = m * a.c1, vh = v * a.c2;
-      p -= a.lr * mh / (sqrtf(vh) + a.eps);
+    if (!a.pack[i].transposed) {
+      (void)adam_entry(a, t, r, c);
+    } else {
+      bf16x8 v;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = f2bf(adam_entry(a, t, 8 * r + k, c));
+      *(bf16x8 *)((__bf16 *)a.pack[i].transposed + c * a.pack[i].ld + 8 * r) = v;
     }
-    t.param[j] = p;
-    t.m[j] = m;
-    t.v[j] = v;
-    if (t.param_bf16) ((__bf16 *)t.param_bf16)[j] = f2bf(p);
   }
 }
 }  // namespace
 
-extern "C" int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, float lr, float beta1, float beta2,
-                            float eps, int32_t step, void *stream) {
+extern "C" int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors,
+                                   float lr, float beta1, float beta2, float eps, int32_t step, void *stream) {
   if (!tensors || n_tensors <= 0 || n_tensors > ADAM_MAX || step <= 0 || !(lr >= 0.0f) || !(beta1 >= 0.0f) ||
       !(beta1 < 1.0f) || !(beta2 >= 0.0f) || !(beta2 < 1.0f) || !(eps > 0.0f))
     return GH_EINVAL;
@@ -889,7 +892,12 @@ extern "C" int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, fl
         t.valid_cols < 0 || t.valid_rows > t.rows || t.valid_cols > t.cols)
       return GH_EINVAL;
     a.t[i] = t;
-    a.offset[i + 1] = a.offset[i] + (int64_t)t.rows * t.cols;
+    if (packs && packs[i].transposed) {
+      const gh_adam_pack &k = packs[i];
+      if (t.rows % 8 != 0 || k.ld < t.rows || k.ld % 8 != 0 || (uintptr_t)k.transposed % 16 != 0) return GH_EINVAL;
+      a.pack[i] = k;
+    }
+    a.offset[i + 1] = a.offset[i] + (int64_t)t.rows * t.cols / (a.pack[i].transposed ? 8 : 1);
   }
   a.lr = lr;
   a.b1 = beta1;
@@ -901,4 +909,9 @@ extern "C" int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, fl
   const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 2048);
   hipLaunchKernelGGL(adam_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+}
+
+extern "C" int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, float lr, float beta1, float beta2,
+                            float eps, int32_t step, void *stream) {
+  return gh_adam_step_packed(tensors, nullptr, n_tensors, lr, beta1, beta2, eps, step, stream);
 }

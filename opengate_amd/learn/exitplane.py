@@ -187,7 +187,10 @@ class ExitPlaneGenerator:
             th = torch.cat([th / th.norm(dim=0, keepdim=True), eye], 1)
             loss = ((torch.sort(o @ th, 0).values - torch.sort(d @ th, 0).values) ** 2).mean()
             loss.backward()
-            dW, db = self.mlp.backward(o.grad)
+            # Adam divides a gradient by its own size, so over a few steps a difference of one
+            # rounding in a bias gradient moves single weights by a tenth of a step: the sums
+            # keep their bits, and with them the weights of a seeded fit
+            dW, db = self.mlp.backward(o.grad, tensor_sums=True)
             self.mlp.step(dW, db)
             losses[it] = loss.detach()
             if log_every and (it % log_every == 0 or it == steps - 1):

@@ -1,15 +1,17 @@
 """Dense MLP trained and evaluated with the library's BF16 MFMA GEMM (gh_gemm_bf16).
 
-Every matrix product of the forward and backward passes runs in the hand-written
-kernel (csrc/mlp.hip) with FP32 accumulation; bias, ReLU and the ReLU derivative are
-fused into its epilogues. PyTorch holds the tensors (device memory, the FP32 master
-weights, the Adam state and the loss), nothing more.
+Every matrix product of the forward and backward passes runs in hand-written kernels with
+FP32 accumulation: networks with equal hidden widths of 128 or 256 take one launch forward
+and three backward (csrc/mlp_train.hip), any other a GEMM launch per product (csrc/mlp.hip)
+with bias, ReLU and the ReLU derivative in its epilogues. PyTorch holds the tensors (device
+memory, the FP32 master weights, the Adam state and the loss), nothing more.
 
 Layer l: Z_l = X_l W_l + b_l (FP32), X_{l+1} = bf16(relu(Z_l)) for hidden layers,
 the last layer is linear. Backward: G_L = dLoss/dZ_L, dW_l = X_l^T G_l,
 db_l = sum_m G_l, G_{l-1} = (G_l W_l^T) * relu'(Z_{l-1}).
 """
 import ctypes as C
+import struct
 
 import numpy as np
 
@@ -22,6 +24,16 @@ def _torch():
     import torch
 
     return torch
+
+
+# the C layouts of gh_adam_tensor and gh_adam_pack
+_ADAM = struct.Struct("=5Q4ifi")
+_PACK = struct.Struct("=Q2i")
+
+
+def _pointers(tensors):
+    """Device addresses of tensors as a C array of pointers."""
+    return struct.pack(f"={len(tensors)}Q", *[t.data_ptr() for t in tensors])
 
 
 def pad8(n):
@@ -52,13 +64,22 @@ class MLP:
 
     # ------------------------------------------------------------------ helpers
     def _refresh(self):
-        """bf16 copies of the weights (kept in place: the optimiser kernel writes them)."""
+        """bf16 copies of the weights (kept in place: the optimiser kernel writes them) and, for
+        the fused kernels, their transposes [N][K] (first layer K -> 32, last layer N -> 16)."""
         torch = _torch()
         if getattr(self, "W16", None) is None or [t.shape for t in self.W16] != [w.shape for w in self.W]:
             self.W16 = [torch.empty(w.shape, device=self.dev, dtype=torch.bfloat16) for w in self.W]
+            self.Wt = None
+            if self.fused_ok():
+                L = len(self.W16)
+                self.Wt = [torch.zeros(self.FUSED_N_OUT if l == L - 1 else w.shape[1],
+                                       self.FUSED_K_IN if l == 0 else w.shape[0], device=self.dev, dtype=torch.bfloat16)
+                           for l, w in enumerate(self.W16)]
         for t, w in zip(self.W16, self.W):
             t.copy_(w)
-        self._fused = None
+        if self.Wt is not None:
+            for t, w in zip(self.Wt, self.W16):
+                t[:w.shape[1], :w.shape[0]] = w.t()
 
     def _stream(self):
         return C.c_void_p(_torch().cuda.current_stream().cuda_stream)
@@ -88,6 +109,8 @@ class MLP:
         else:
             X = torch.zeros(M, self.psizes[0], device=self.dev, dtype=torch.bfloat16)
             X[:, : self.sizes[0]] = x.to(torch.bfloat16)
+        if self._train_fused(X):
+            return self._forward_fused(X, keep)
         xs, zs = [X], []
         L = len(self.W)
         for l in range(L):
@@ -125,6 +148,7 @@ class MLP:
 
     # ------------------------------------------------------------------ fused inference
     FUSED_K_IN, FUSED_N_OUT, FUSED_MAX_LAYERS = 32, 16, 8
+    TRAIN_MAX_ROWS = 4194240  # GH_MLP_TRAIN_MAX_ROWS
 
     def fused_ok(self):
         """gh_mlp_forward_bf16 handles 2..8 layers with equal hidden widths of 128 or 256,
@@ -133,45 +157,87 @@ class MLP:
         return (2 <= len(self.W) <= self.FUSED_MAX_LAYERS and len(hidden) == 1 and hidden <= {128, 256}
                 and self.psizes[0] <= self.FUSED_K_IN and self.psizes[-1] <= self.FUSED_N_OUT)
 
-    def _fused_weights(self):
-        """Transposed, padded bf16 weights (first layer K -> 32, last layer N -> 16) and
-        biases (last layer -> 16), rebuilt after each optimiser step."""
+    def _fused_args(self):
+        """Pointer arrays (bytes) of the transposed weights and the biases; the tensors they
+        point to stay referenced by the returned list."""
+        bs = [b if b.is_contiguous() and b.data_ptr() % 16 == 0 else b.clone(memory_format=_torch().contiguous_format)
+              for b in self.b]
+        return _pointers(self.Wt), _pointers(bs), bs
+
+    def _train_fused(self, X):
+        """gh_mlp_train_* take the network and this batch."""
+        return self.Wt is not None and 1 <= X.shape[0] <= self.TRAIN_MAX_ROWS and X.data_ptr() % 16 == 0
+
+    def _forward_fused(self, X, keep):
         torch = _torch()
-        if self._fused is None:
-            L = len(self.W16)
-            wts, bs = [], []
-            for l, w16 in enumerate(self.W16):
-                K, N = w16.shape
-                Kp = self.FUSED_K_IN if l == 0 else K
-                Np = self.FUSED_N_OUT if l == L - 1 else N
-                t = torch.zeros(Np, Kp, device=self.dev, dtype=torch.bfloat16)
-                t[:N, :K] = w16.t()
-                wts.append(t.contiguous())
-                b = torch.zeros(Np, device=self.dev)
-                b[:N] = self.b[l]
-                bs.append(b)
-            self._fused = (wts, bs)
-        return self._fused
+        M, L = X.shape[0], len(self.W)
+        Z = torch.empty(M, self.psizes[-1], device=self.dev, dtype=torch.float32)
+        if not keep:
+            return self.infer_fused(X, Z)[:, : self.sizes[-1]]
+        Y = torch.empty(L - 1, M, self.psizes[1], device=self.dev, dtype=torch.bfloat16)
+        wp, bp, hold = self._fused_args()
+        rc = self.lib.gh_mlp_train_forward_bf16(X.data_ptr(), M, L, self.psizes[0], self.psizes[1], self.sizes[-1],
+                                                wp, bp, _pointers(Y), Z.data_ptr(), Z.stride(0), self._stream())
+        del hold
+        if rc != 0:
+            raise RuntimeError(f"gh_mlp_train_forward_bf16 failed ({rc})")
+        self._xs, self._zs = [X, *Y], None
+        return Z[:, : self.sizes[-1]]
+
+    def _backward_fused(self, grad_out, tensor_sums):
+        torch = _torch()
+        X, Y, L = self._xs[0], self._xs[1:], len(self.W)
+        M, k_in, hidden, n_out, n_pad = X.shape[0], self.psizes[0], self.psizes[1], self.sizes[-1], self.psizes[-1]
+        G, G32 = grad_out, None
+        if tensor_sums:
+            G = torch.zeros(M, n_pad, device=self.dev, dtype=torch.float32)
+            G[:, :n_out] = grad_out
+            G32 = torch.empty(L - 1, M, hidden, device=self.dev, dtype=torch.float32)
+        elif G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != X.device or G.stride(1) != 1:
+            G = torch.empty(M, n_out, device=self.dev, dtype=torch.float32)
+            G[:] = grad_out
+        shapes = [tuple(w.shape) for w in self.W]
+        flat = torch.empty(sum(k * n for k, n in shapes), device=self.dev, dtype=torch.float32)
+        dbf = torch.empty((L - 1) * hidden + n_pad, device=self.dev, dtype=torch.float32)
+        size = C.c_int64()
+        rc = self.lib.gh_mlp_train_workspace(M, L, k_in, hidden, n_pad, C.byref(size))
+        if rc != 0:
+            raise RuntimeError(f"gh_mlp_train_workspace failed ({rc})")
+        ws = torch.empty(size.value, device=self.dev, dtype=torch.uint8)
+        rc = self.lib.gh_mlp_train_backward_bf16(X.data_ptr(), M, L, k_in, hidden, n_out, n_pad, _pointers(self.W16),
+                                                 _pointers(Y), G.data_ptr(), G.stride(0), flat.data_ptr(),
+                                                 dbf.data_ptr(), None if G32 is None else _pointers(G32),
+                                                 ws.data_ptr(), size.value, self._stream())
+        if rc != 0:
+            raise RuntimeError(f"gh_mlp_train_backward_bf16 failed ({rc})")
+        dW, o = [], 0
+        for k, n in shapes:
+            dW.append(flat[o:o + k * n].view(k, n))
+            o += k * n
+        if tensor_sums:
+            return dW, [g.sum(0) for g in (*G32, G)]
+        return dW, list(dbf.split([n for _, n in shapes]))
 
     def infer_fused(self, X, out):
         """All layers in one kernel (gh_mlp_forward_bf16): X (M, in padded) bf16 with row
         pitch X.stride(0), out (M, >= out) FP32 with row pitch out.stride(0); only the
         first sizes[-1] columns of out are written. Same values as infer()."""
-        wts, bs = self._fused_weights()
-        L = len(wts)
-        wp = (C.c_void_p * L)(*[t.data_ptr() for t in wts])
-        bp = (C.POINTER(C.c_float) * L)(*[C.cast(C.c_void_p(t.data_ptr()), C.POINTER(C.c_float)) for t in bs])
-        rc = self.lib.gh_mlp_forward_bf16(C.c_void_p(X.data_ptr()), X.stride(0), X.shape[0], L, self.psizes[0],
-                                          self.psizes[1], self.sizes[-1], wp, bp,
-                                          C.cast(C.c_void_p(out.data_ptr()), C.POINTER(C.c_float)),
-                                          out.stride(0), self._stream())
+        wp, bp, hold = self._fused_args()
+        rc = self.lib.gh_mlp_forward_bf16(X.data_ptr(), X.stride(0), X.shape[0], len(self.W), self.psizes[0],
+                                          self.psizes[1], self.sizes[-1], wp, bp, out.data_ptr(), out.stride(0),
+                                          self._stream())
+        del hold
         if rc != 0:
             raise RuntimeError(f"gh_mlp_forward_bf16 failed ({rc})")
         return out
 
-    def backward(self, grad_out):
-        """grad_out: dLoss/dOutput (M, out) FP32. Returns [dW...], [db...] (FP32, padded)."""
+    def backward(self, grad_out, tensor_sums=False):
+        """grad_out: dLoss/dOutput (M, out) FP32. Returns [dW...], [db...] (FP32, padded).
+        tensor_sums: take the bias gradients as PyTorch's column sums of the FP32 gradients,
+        the bits of the layer-by-layer path, instead of the kernels' own sums (2e-7 apart)."""
         torch = _torch()
+        if self._zs is None:
+            return self._backward_fused(grad_out, tensor_sums)
         M = grad_out.shape[0]
         L = len(self.W)
         G32 = torch.zeros(M, self.psizes[-1], device=self.dev, dtype=torch.float32)
@@ -196,26 +262,28 @@ class MLP:
 
     def step(self, dW, db):
         """Adam update of the FP32 master weights and biases in one kernel (gh_adam_step),
-        which also keeps the padding at zero and writes the bf16 weight copies."""
+        which also keeps the padding at zero and writes the bf16 weight copies (both layouts)."""
         self.t += 1
         params = self.W + self.b
         grads = list(dW) + list(db)
         valid = [(k, n) for k, n in zip(self.sizes[:-1], self.sizes[1:])] + [(1, n) for n in self.sizes[1:]]
-        tab = (A.AdamTensor * len(params))()
+        tab, packs = [], []
+        L = len(self.W)
         for i, (p, g, (vr, vc)) in enumerate(zip(params, grads, valid)):
             if g.shape != p.shape or not g.is_contiguous() or g.dtype != p.dtype:
                 raise ValueError("gradient shape / layout differs from its parameter")
             rows, cols = (p.shape[0], p.shape[1]) if p.dim() == 2 else (1, p.shape[0])
-            is_w = i < len(self.W)
-            tab[i] = A.AdamTensor(p.data_ptr(), g.data_ptr(), self.m[i].data_ptr(), self.v[i].data_ptr(),
-                                  self.W16[i].data_ptr() if is_w else None, rows, cols, vr, vc,
-                                  float(self.wd) if is_w else 0.0, 0)
+            is_w = i < L
+            tab.append(_ADAM.pack(p.data_ptr(), g.data_ptr(), self.m[i].data_ptr(), self.v[i].data_ptr(),
+                                  self.W16[i].data_ptr() if is_w else 0, rows, cols, vr, vc,
+                                  float(self.wd) if is_w else 0.0, 0))
+            t = self.Wt[i] if is_w and self.Wt is not None else None
+            packs.append(_PACK.pack(0, 0, 0) if t is None else _PACK.pack(t.data_ptr(), t.shape[1], 0))
         b1, b2 = self.betas
-        rc = self.lib.gh_adam_step(tab, len(params), float(self.lr), float(b1), float(b2), float(self.eps), self.t,
-                                   self._stream())
+        rc = self.lib.gh_adam_step_packed(b"".join(tab), b"".join(packs), len(params), float(self.lr), float(b1),
+                                          float(b2), float(self.eps), self.t, self._stream())
         if rc != 0:
-            raise RuntimeError(f"gh_adam_step failed ({rc})")
-        self._fused = None
+            raise RuntimeError(f"gh_adam_step_packed failed ({rc})")
 
     def state_dict(self):
         return {"sizes": self.sizes, "W": [w.cpu() for w in self.W], "b": [b.cpu() for b in self.b]}
