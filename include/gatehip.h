@@ -297,6 +297,12 @@ int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers,
                         int32_t n_out, const void *const *wt, const float *const *bias, float *Z, int64_t ldz,
                         void *stream);
 
+/* The same with wt[l] in fragment order (see gh_adam_step_packed) and 16-byte aligned bias[l] of
+ * the hidden layers. */
+int gh_mlp_forward_packed_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
+                               int32_t n_out, const void *const *wt, const float *const *bias, float *Z, int64_t ldz,
+                               void *stream);
+
 /* Training: one Adam step (Kingma & Ba) over all parameter tensors of a network in one
  * launch. No counterpart in the reference's source: its networks come trained from the
  * external gaga / garf packages (loaded in sources/gansources.py and actors/arfactors.py);
@@ -316,15 +322,21 @@ typedef struct gh_adam_tensor {
 int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, float lr, float beta1, float beta2, float eps,
                  int32_t step, void *stream);
 
-/* The same step, which also writes a transposed bf16 copy of a tensor: transposed[c ld + r] =
- * bf16(param[r][c]) for every r < rows, c < cols (rows a multiple of 8, ld >= rows a multiple
- * of 8, 16-byte aligned; NULL: none). It is the weight layout of gh_mlp_forward_bf16. packs:
- * n_tensors entries, or NULL. */
+/* Fragment order of a bf16 matrix [N][K], N a multiple of 16 and K of 32: element (n, k) at
+ * ((n/16 * K/32 + k/32) * 64 + (k%32)/8 * 16 + n%16) * 8 + k%8, the order in which a wave loads
+ * its MFMA fragments. Of a weight tensor W [K][N] (rows x cols), the forward copy is W^T [N][K]
+ * and the backward copy W [K][N], in fragment order, the reduction dimension padded with zeros.
+ *
+ * The same Adam step, which also writes these copies of a tensor: element (c, r) of `forward`
+ * (K = forward_k >= rows) and (r, c) of `backward` (K = backward_k >= cols; NULL: none) =
+ * bf16(param[r][c]); rows a multiple of 8, 16-byte aligned. forward NULL: no copies. packs:
+ * n_tensors entries, or NULL. gh_pack_weights writes the copies (param_bf16 too) of the
+ * parameters as they are; grad, m and v are not read. */
 typedef struct gh_adam_pack {
-  void *transposed;
-  int32_t ld;
-  int32_t reserved;
+  void *forward, *backward;
+  int32_t forward_k, backward_k;
 } gh_adam_pack;
+int gh_pack_weights(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors, void *stream);
 int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors, float lr,
                         float beta1, float beta2, float eps, int32_t step, void *stream);
 
@@ -332,23 +344,25 @@ int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs
  * gh_adam_step), for the networks of gh_mlp_forward_bf16 whose input width k_in and padded
  * output width np (8 or 16) are multiples of 8. At most GH_MLP_TRAIN_MAX_ROWS rows; every
  * pointer but G and Z 16-byte aligned.
- * Forward: X: M x k_in bf16 (contiguous); wt, bias as in gh_mlp_forward_bf16; Y[l]: the hidden
- * activations bf16(relu(Z_l)), M x hidden, kept for the backward pass; Z: FP32 output, columns
- * 0..n_out-1. Same values as the layer-by-layer gh_gemm_bf16 path, bit for bit.
- * Backward: w[l] (l >= 1): bf16 weights [K_l][N_l] row-major (N of the last layer = np); G:
- * dLoss/dZ, M x n_out FP32 with row pitch ldg. dW: the FP32 weight gradients of all layers one
- * after the other, each K_l x N_l; db: the bias gradients, hidden per hidden layer, then np.
- * The column sums are taken over the FP32 gradients, the products over their bf16 roundings
- * (dW: the bits of gh_gemm_bf16). G32, if not NULL, receives the FP32 gradients of the hidden
- * layers, M x hidden each.
- * ws: device memory of the bytes gh_mlp_train_workspace gives, free again when the launches have
- * run. */
+ * The kept matrices are in tiles of 16 rows, tile t at 16 t C for C columns, each in fragment
+ * order (N = 16 rows, K = C), padded with zeros to Mp = M rounded up to 32 rows.
+ * Forward: X: M x k_in bf16 (contiguous); wt, bias as in gh_mlp_forward_packed_bf16; kept: Xt, the
+ * input in 32 columns (Mp x 32), and Y[l], the hidden activations bf16(relu(Z_l)) (Mp x hidden);
+ * Z: FP32 output, columns 0..n_out-1. Same values as the layer-by-layer gh_gemm_bf16 path, bit
+ * for bit.
+ * Backward: Xt, Y: as kept; w[l] (l >= 1): W_l [K_l][N_l] in fragment order (N of the last layer
+ * padded to 32); G: dLoss/dZ, M x n_out FP32 with row pitch ldg. dW: the FP32 weight gradients of
+ * all layers one after the other, each K_l x N_l; db: the bias gradients, hidden per hidden
+ * layer, then np. The column sums are taken over the FP32 gradients, the products over their
+ * bf16 roundings (dW: the bits of gh_gemm_bf16). G32, if not NULL, receives the FP32 gradients of
+ * the hidden layers, M x hidden row-major each. ws: device memory of the bytes
+ * gh_mlp_train_workspace gives, free again when the launches have run. */
 #define GH_MLP_TRAIN_MAX_ROWS 4194240
 int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t n_out,
-                              const void *const *wt, const float *const *bias, void *const *Y, float *Z, int64_t ldz,
-                              void *stream);
+                              const void *const *wt, const float *const *bias, void *Xt, void *const *Y, float *Z,
+                              int64_t ldz, void *stream);
 int gh_mlp_train_workspace(int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t np, int64_t *bytes);
-int gh_mlp_train_backward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t n_out,
+int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden, int32_t n_out,
                                int32_t np, const void *const *w, const void *const *Y, const float *G, int64_t ldg,
                                float *dW, float *db, float *const *G32, void *ws, int64_t ws_bytes, void *stream);
 
@@ -366,6 +380,15 @@ int gh_gaussian_bf16(uint64_t seed, uint64_t first_row, int64_t n_rows, int32_t 
 int gh_exitplane_decode(const float *Z, int64_t ldz, int64_t n, const float *qtab, int32_t n_knots, float g_max,
                         const float focal[3], float plane_z, const float offset[3], float weight,
                         float *const out[8], void *stream);
+
+/* Both around gh_mlp_forward_packed_bf16 (k_in = n_noise, hidden = 256, n_out = 6): photons of
+ * noise rows first .. first + n - 1, the bits of the three calls. Z: device work memory of
+ * z_rows x 8 floats; z_rows >= min(n, 65536), more for fewer launches (up to 32768 photons need
+ * none: 0, NULL). */
+int gh_exitplane_generate(uint64_t seed, uint64_t first, int64_t n, int32_t n_noise, int32_t n_layers, int32_t hidden,
+                          const void *const *wt, const float *const *bias, const float *qtab, int32_t n_knots,
+                          float g_max, const float focal[3], float plane_z, const float offset[3], float weight,
+                          float *const out[8], float *Z, int64_t z_rows, void *stream);
 
 /* SPECT heads for the learned collimator-detector response (ARFActor, actors/arfactors.py:140-463:
  * apply / arf_build_image_from_projected_points, and GateARFActor::SteppingAction,

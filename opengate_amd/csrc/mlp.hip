@@ -32,13 +32,12 @@
 #include <string>
 
 #include "../../include/gatehip.h"
+#include "mlp_rows.h"
 #include "splitk.h"
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
+using namespace mlp;
 
 constexpr int BM = gh::GEMM_BM, BN = gh::GEMM_BN, BK = gh::GEMM_BK;
 using gh::splitk_plan;
@@ -378,9 +377,6 @@ extern "C" int gh_gemm_bf16_noalloc(const void *A, int64_t sam, int64_t sak, con
 // is the same as the layer-by-layer GEMM path, so both give bit-identical outputs.
 namespace {
 
-constexpr int MAXL = 8;          // layers
-constexpr int K0 = 32;           // first-layer input width (padded)
-constexpr int NOUT = 16;         // last-layer output width (padded)
 // 16-row tiles per workgroup, per hidden width (measured best on MI355X)
 #ifndef GH_MLP_RT128
 #define GH_MLP_RT128 8           // 128 rows
@@ -389,19 +385,17 @@ constexpr int NOUT = 16;         // last-layer output width (padded)
 #define GH_MLP_SB 1              // one activation buffer, overwritten after a barrier
 #endif
 
-struct MlpArgs {
-  const __bf16 *wt[MAXL];        // [N_l][K_l]
-  const float *bias[MAXL];       // [N_l]
-  int n_layers;
-  int k_in;                      // valid input columns (<= K0)
-  int n_out;                     // valid output columns (<= NOUT)
-  int x_vec;                     // 1: input rows 16-byte aligned (16-byte loads)
-};
-
 template <int H, int RT, int SB>
 constexpr size_t mlp_lds_bytes() { return (SB ? 1ull : 2ull) * (16 * RT) * (H + 8) * sizeof(__bf16); }
 
-template <int H, int RT, int SB>
+// address of a lane's fragment (16-column tile ct, k step ks) of weights [N][K = 32 nk]
+template <bool PACKED>
+__device__ __forceinline__ const __bf16 *weight_frag(const __bf16 *W, int ct, int ks, int nk, int lane) {
+  return PACKED ? W + ((ct * nk + ks) * 64 + lane) * 8
+                : W + (int64_t)(ct * 16 + (lane & 15)) * (nk * 32) + ks * 32 + (lane >> 4) * 8;
+}
+
+template <int H, int RT, int SB, bool PACKED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) mlp_forward_kernel(const __bf16 *__restrict__ X, int64_t ldx, int64_t M,
                                                           MlpArgs a, float *__restrict__ Z, int64_t ldz) {
   constexpr int P = H + 8;                 // LDS row pitch (bf16)
@@ -461,12 +455,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
       const int nk = K / 32;
       const __bf16 *wrow[CT];
 #pragma unroll
-      for (int j = 0; j < CT; ++j) wrow[j] = W + (int64_t)(n0 + j * 16 + fr) * K + fk;
+      for (int j = 0; j < CT; ++j) wrow[j] = weight_frag<PACKED>(W, wave * CT + j, 0, nk, lane);
       const __bf16 *arow = in + fr * P + fk;
       bf16x8 bA[CT], bB[CT], aA[RT], aB[RT];
       auto load = [&](bf16x8 *b, bf16x8 *af, int ks) {
 #pragma unroll
-        for (int j = 0; j < CT; ++j) b[j] = *(const bf16x8 *)(wrow[j] + ks * 32);
+        for (int j = 0; j < CT; ++j) b[j] = *(const bf16x8 *)(wrow[j] + ks * (PACKED ? 512 : 32));
 #pragma unroll
         for (int i = 0; i < RT; ++i) af[i] = *(const bf16x8 *)(arow + i * 16 * P + ks * 32);
       };
@@ -515,7 +509,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
       if (l + 2 < a.n_layers) {
         const __bf16 *Wn = a.wt[l + 1];
 #pragma unroll
-        for (int j = 0; j < CT; ++j) wpre[j] = *(const bf16x8 *)(Wn + (int64_t)(n0 + j * 16 + fr) * H + fk);
+        for (int j = 0; j < CT; ++j) wpre[j] = *(const bf16x8 *)weight_frag<PACKED>(Wn, wave * CT + j, 0, H / 32, lane);
         have_pre = true;
       }
       // with one buffer, every wave must be done reading the layer input before any
@@ -544,7 +538,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
       // weights loaded at once (one L2 latency instead of one per k step)
       bf16x8 wout[H / 32];
 #pragma unroll
-      for (int k = 0; k < H / 32; ++k) wout[k] = *(const bf16x8 *)(W + (int64_t)fr * H + k * 32 + fk);
+      for (int k = 0; k < H / 32; ++k) wout[k] = *(const bf16x8 *)weight_frag<PACKED>(W, 0, k, H / 32, lane);
       constexpr int NTW = (RT + 3) / 4;
       floatx4 acc[NTW];
 #pragma unroll
@@ -602,25 +596,31 @@ constexpr size_t W8_LDS = W8_ACT + 2 * W8_STAGE;           // 163 840 bytes
 // element (r, k) of the swizzled activation tile
 __device__ __forceinline__ int w8_at(int r, int k) { return r * W8_P + ((((k >> 3) ^ (r & 15)) << 3) | (k & 7)); }
 
-// k step ks of a 256-column weight matrix Wt[n][k] (row length K) into a stage: 16-byte
-// slot s holds k group s / 256 (8 values) of column s % 256, so that the 16 lanes of an
-// MFMA fragment read (16 consecutive columns, one k group) read 256 consecutive bytes.
-// Each of the 512 threads moves two slots; lane i of an instruction writes its 16 bytes
-// at the instruction's LDS base + 16 i.
+// k step ks of a 256-column weight matrix [n][k] (row length K) into a stage of 1024 16-byte
+// slots; each of the 512 threads moves two slots, lane i of an instruction writing its 16
+// bytes at the instruction's LDS base + 16 i. Fragment order: fragment ct (the 64 lanes of an
+// MFMA operand) in slots 64 ct .. 64 ct + 63, 1 KiB pieces on both sides. Rows: slot s holds k
+// group s / 256 (8 values) of column s % 256, so that the 16 lanes of an MFMA fragment read (16
+// consecutive columns, one k group) read 256 consecutive bytes.
+template <bool PACKED>
 __device__ __forceinline__ void w8_stage_load(unsigned char *stage, const __bf16 *W, int K, int ks, int tid) {
   const int lane = tid & 63, wave = tid >> 6;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int s = i * 512 + wave * 64 + lane;
-    const int n = s & 255, kg = s >> 8;
-    const __bf16 *src = W + (int64_t)n * K + ks * 32 + kg * 8;
+    const __bf16 *src = PACKED ? weight_frag<true>(W, s >> 6, ks, K / 32, lane)
+                               : W + (int64_t)(s & 255) * K + ks * 32 + (s >> 8) * 8;
     unsigned char *dst = stage + (size_t)(i * 512 + wave * 64) * 16;
     __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
   }
 }
 
+// NOISE: the input tile is generator noise, made here: the 16-byte-per-row input would be
+// written and read through HBM otherwise, and its load latency is longer than the Philox block
+// and Box-Muller of a thread
+template <bool PACKED, bool NOISE>
 __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__ X, int64_t ldx, int64_t M,
-                                                      MlpArgs a, float *__restrict__ Z, int64_t ldz) {
+                                                      MlpArgs a, MlpGenerate gen, float *__restrict__ Z, int64_t ldz) {
   constexpr int H = 256, RT = W8_RT, CT = 4, ROWS = W8_ROWS;
   extern __shared__ __align__(16) unsigned char mlp_lds[];
   __bf16 *act = (__bf16 *)mlp_lds;
@@ -633,8 +633,24 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
   // step ks of a hidden layer stage (ks + 1) % 2. Every stage index and weight offset below
   // is a compile-time constant; only the layer's weight pointers are read per layer.
   auto stage = [&](int g) { return mlp_lds + W8_ACT + (size_t)(g & 1) * W8_STAGE; };
-  w8_stage_load(stage(0), a.wt[0], K0, 0, tid);  // the input layer's weights load while the input tile does
-  if (a.x_vec) {
+  w8_stage_load<PACKED>(stage(0), a.wt[0], K0, 0, tid);  // the input layer's weights load while the input tile does
+  if (NOISE) {
+    // 4 columns per thread and turn
+    for (int i = tid; i < ROWS * (K0 / 4); i += 512) {
+      const int r = i % ROWS, c = i / ROWS * 4;
+      bf16x4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = (__bf16)0.0f;
+      if (c < gen.n_cols) {
+        float g[4];
+        ep::noise4(gen.first + (uint64_t)(row0 + r), (uint32_t)(c >> 2), gen.k0, gen.k1, g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < gen.n_cols) v[j] = (__bf16)g[j];
+      }
+      *(bf16x4 *)(act + w8_at(r, c)) = v;
+    }
+  } else if (a.x_vec) {
     for (int i = tid; i < ROWS * (K0 / 8); i += 512) {
       const int r = i / (K0 / 8), q = (i - r * (K0 / 8)) * 8;
       const int64_t gr = row0 + r;
@@ -671,7 +687,7 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
     auto loadB = [&](bf16x8 *b, int g) {
       const unsigned char *st = stage(g);
 #pragma unroll
-      for (int j = 0; j < CT; ++j) b[j] = *(const bf16x8 *)(st + (size_t)((lane >> 4) * 256 + cg * 64 + j * 16 + fr) * 16);
+      for (int j = 0; j < CT; ++j) b[j] = *(const bf16x8 *)(st + (size_t)(PACKED ? (cg * 4 + j) * 64 + lane : (lane >> 4) * 256 + cg * 64 + j * 16 + fr) * 16);
     };
     // this layer's weights and, when the next layer is a hidden one, the next layer's (its
     // first step is staged during this layer's second-to-last step)
@@ -684,9 +700,9 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();  // the layer input is complete, and so are the weights of its first step
       if (NK == 1) {
-        if (Wn) w8_stage_load(stage(1), Wn, H, 0, tid);
+        if (Wn) w8_stage_load<PACKED>(stage(1), Wn, H, 0, tid);
       } else {
-        w8_stage_load(stage(stg(1)), Wl, H, 1, tid);
+        w8_stage_load<PACKED>(stage(stg(1)), Wl, H, 1, tid);
       }
       loadB(bA, stg(0));
       loadA(aA, 0);
@@ -699,8 +715,8 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
 #pragma unroll
           for (int j = 0; j < CT; ++j) asm volatile("" : "+v"(bCur[j]) :: "memory");
           // refill the stage that step ks used (its fragments were read one step earlier)
-          if (ks + 2 < NK) w8_stage_load(stage(stg(ks + 2)), Wl, H, ks + 2, tid);
-          else if (Wn) w8_stage_load(stage(1), Wn, H, 0, tid);
+          if (ks + 2 < NK) w8_stage_load<PACKED>(stage(stg(ks + 2)), Wl, H, ks + 2, tid);
+          else if (Wn) w8_stage_load<PACKED>(stage(1), Wn, H, 0, tid);
           loadB(bNext, stg(ks + 1));
           loadA(aNext, ks + 1);
         }
@@ -741,7 +757,7 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
   const float *__restrict__ bias = a.bias[l];
   bf16x8 wout[H / 32];
 #pragma unroll
-  for (int k = 0; k < H / 32; ++k) wout[k] = *(const bf16x8 *)(W + (int64_t)fr * H + k * 32 + fk);
+  for (int k = 0; k < H / 32; ++k) wout[k] = *(const bf16x8 *)weight_frag<PACKED>(W, 0, k, H / 32, lane);
   constexpr int NT = 2 * RT, NTW = (NT + 7) / 8;
   floatx4 acc[NTW];
 #pragma unroll
@@ -773,38 +789,40 @@ __global__ void __launch_bounds__(512) mlp_forward_w8(const __bf16 *__restrict__
   }
 }
 
-template <int H>
+template <bool PACKED, bool NOISE>
+int launch_w8(const __bf16 *X, int64_t ldx, int64_t M, const MlpArgs &a, const MlpGenerate &gen, float *Z, int64_t ldz,
+              hipStream_t st) {
+  const void *fn = (const void *)&mlp_forward_w8<PACKED, NOISE>;
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)W8_LDS) != hipSuccess)
+    return GH_EHIP;
+  const dim3 grid((unsigned)((M + W8_ROWS - 1) / W8_ROWS));
+  hipLaunchKernelGGL((mlp_forward_w8<PACKED, NOISE>), grid, dim3(512), W8_LDS, st, X, ldx, M, a, gen, Z, ldz);
+  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+}
+
+template <int H, bool PACKED>
 int launch_mlp(const __bf16 *X, int64_t ldx, int64_t M, const MlpArgs &a, float *Z, int64_t ldz, hipStream_t st) {
   if constexpr (H == 256) {
-    const void *fn = (const void *)&mlp_forward_w8;
-    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)W8_LDS) != hipSuccess)
-      return GH_EHIP;
-    const dim3 grid((unsigned)((M + W8_ROWS - 1) / W8_ROWS));
-    hipLaunchKernelGGL(mlp_forward_w8, grid, dim3(512), W8_LDS, st, X, ldx, M, a, Z, ldz);
-    return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+    return launch_w8<PACKED, false>(X, ldx, M, a, {}, Z, ldz, st);
   } else {
     constexpr int RT = GH_MLP_RT128, SB = GH_MLP_SB;
     constexpr size_t lds = mlp_lds_bytes<H, RT, SB>();
-    const void *fn = (const void *)&mlp_forward_kernel<H, RT, SB>;
+    const void *fn = (const void *)&mlp_forward_kernel<H, RT, SB, PACKED>;
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return GH_EHIP;
     const dim3 grid((unsigned)((M + 16 * RT - 1) / (16 * RT)));
-    hipLaunchKernelGGL((mlp_forward_kernel<H, RT, SB>), grid, dim3(256), lds, st, X, ldx, M, a, Z, ldz);
+    hipLaunchKernelGGL((mlp_forward_kernel<H, RT, SB, PACKED>), grid, dim3(256), lds, st, X, ldx, M, a, Z, ldz);
     return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
   }
 }
 
-}  // namespace
-
-extern "C" int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers, int32_t k_in,
-                                   int32_t hidden, int32_t n_out, const void *const *wt, const float *const *bias,
-                                   float *Z, int64_t ldz, void *stream) {
+int mlp_forward_args(const void *X, int64_t ldx, int64_t M, int n_layers, int k_in, int hidden, int n_out,
+                     const void *const *wt, const float *const *bias, const float *Z, int64_t ldz, MlpArgs &a) {
   if (!X || !wt || !bias || !Z || M < 0 || n_layers < 2 || n_layers > MAXL || k_in <= 0 || k_in > K0 ||
       n_out <= 0 || n_out > NOUT || ldz < n_out || ldx < k_in)
     return GH_EINVAL;
   if (hidden != 128 && hidden != 256) return GH_EINVAL;
-  MlpArgs a{};
   a.n_layers = n_layers;
   a.k_in = k_in;
   a.n_out = n_out;
@@ -813,10 +831,107 @@ extern "C" int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_
     a.wt[l] = (const __bf16 *)wt[l];
     a.bias[l] = bias[l];
   }
-  if (M == 0) return GH_OK;
   a.x_vec = ((uintptr_t)X % 16 == 0 && ldx % 8 == 0) ? 1 : 0;
-  if (hidden == 256) return launch_mlp<256>((const __bf16 *)X, ldx, M, a, Z, ldz, (hipStream_t)stream);
-  return launch_mlp<128>((const __bf16 *)X, ldx, M, a, Z, ldz, (hipStream_t)stream);
+  return GH_OK;
+}
+
+template <int H, int MODE>
+int launch_rows(const __bf16 *X, int64_t ldx, int64_t M, const MlpArgs &a, const MlpGenerate &gen, float *Z,
+                int64_t ldz, hipStream_t st) {
+  const MlpKeep keep{};
+  switch (row_tiles(M)) {
+    case 1: return launch_rows_forward<H, 1, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+    case 2: return launch_rows_forward<H, 2, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+    default: return launch_rows_forward<H, 4, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+  }
+}
+
+// Which form takes M rows. Width 256: the row-tile form covers 16384 rows per round of 256 CUs in
+// 12.5 us, the 8-wave form 65536 in 31 us (1190 TFLOP/s, against 690): measured 13.3 : 30.8 us
+// at 16384 rows, 24.9 : 30.3 at 32768, 33.3 : 30.4 at 40960. Beyond a round, a remainder of at
+// most two rounds of the row form goes there (81920 rows: 45 us instead of 59). Width 128: the
+// row form up to one round of it at 64 rows on four workgroups per CU (8.1 : 9.2 us at 49152
+// rows), 9.4 : 9.3 at 57344, 459 : 448 at 4.2M.
+constexpr int64_t ROWS_MAX_256 = 32768, ROUND_256 = 65536, ROWS_MAX_128 = 57344;
+
+}  // namespace
+
+extern "C" int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers, int32_t k_in,
+                                   int32_t hidden, int32_t n_out, const void *const *wt, const float *const *bias,
+                                   float *Z, int64_t ldz, void *stream) {
+  MlpArgs a{};
+  const int rc = mlp_forward_args(X, ldx, M, n_layers, k_in, hidden, n_out, wt, bias, Z, ldz, a);
+  if (rc != GH_OK || M == 0) return rc;
+  const __bf16 *x = (const __bf16 *)X;
+  hipStream_t st = (hipStream_t)stream;
+  return hidden == 256 ? launch_mlp<256, false>(x, ldx, M, a, Z, ldz, st)
+                       : launch_mlp<128, false>(x, ldx, M, a, Z, ldz, st);
+}
+
+extern "C" int gh_mlp_forward_packed_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers, int32_t k_in,
+                                          int32_t hidden, int32_t n_out, const void *const *wt,
+                                          const float *const *bias, float *Z, int64_t ldz, void *stream) {
+  MlpArgs a{};
+  const int rc = mlp_forward_args(X, ldx, M, n_layers, k_in, hidden, n_out, wt, bias, Z, ldz, a);
+  if (rc != GH_OK) return rc;
+  for (int l = 0; l < n_layers; ++l)
+    if ((uintptr_t)wt[l] % 16 != 0 || (l < n_layers - 1 && (uintptr_t)bias[l] % 16 != 0)) return GH_EINVAL;
+  if (M == 0) return GH_OK;
+  const __bf16 *x = (const __bf16 *)X;
+  hipStream_t st = (hipStream_t)stream;
+  if (hidden == 256) {
+    const int64_t rest = M % ROUND_256;
+    const int64_t n = rest <= ROWS_MAX_256 ? M - rest : M;
+    if (n > 0) {
+      const int r = launch_mlp<256, true>(x, ldx, n, a, Z, ldz, st);
+      if (r != GH_OK || n == M) return r;
+    }
+    return launch_rows<256, ROWS_INFER>(x + n * ldx, ldx, M - n, a, {}, Z + n * ldz, ldz, st);
+  }
+  return M <= ROWS_MAX_128 ? launch_rows<128, ROWS_INFER>(x, ldx, M, a, {}, Z, ldz, st)
+                           : launch_mlp<128, true>(x, ldx, M, a, Z, ldz, st);
+}
+
+// The whole exit-plane source: noise rows, network, decoder. At most ROWS_MAX_256 photons (or
+// what a round of the 8-wave form leaves over) take one launch per row tile, noise to photons;
+// more take the 8-wave form, which makes its noise, and the decoder as a launch of its own (its
+// table lookups would leave the matrix cores of a CU idle for a tenth of the time there).
+extern "C" int gh_exitplane_generate(uint64_t seed, uint64_t first, int64_t n, int32_t n_noise, int32_t n_layers,
+                                     int32_t hidden, const void *const *wt, const float *const *bias,
+                                     const float *qtab, int32_t n_knots, float g_max, const float focal[3],
+                                     float plane_z, const float offset[3], float weight, float *const out[8], float *Z,
+                                     int64_t z_rows, void *stream) {
+  if (!qtab || !focal || !offset || !out || n < 0 || n_knots < 2 || !(g_max > 0.0f) || hidden != 256 || n_noise <= 0 ||
+      n_noise > K0 || z_rows < 0 || (z_rows > 0 && !Z))
+    return GH_EINVAL;
+  for (int k = 0; k < 8; ++k)
+    if (!out[k]) return GH_EINVAL;
+  MlpArgs a{};
+  const float dummy = 0.0f;
+  const int rc = mlp_forward_args(&dummy, K0, n, n_layers, n_noise, hidden, 6, wt, bias, &dummy, 8, a);
+  if (rc != GH_OK) return rc;
+  for (int l = 0; l < n_layers; ++l)
+    if ((uintptr_t)wt[l] % 16 != 0 || (l < n_layers - 1 && (uintptr_t)bias[l] % 16 != 0)) return GH_EINVAL;
+  MlpGenerate gen{(uint32_t)seed, (uint32_t)(seed >> 32), first, (int)n_noise,
+                  {qtab, (int)n_knots, (float)(n_knots - 1) / (2.0f * g_max), g_max,
+                   {focal[0], focal[1], focal[2], plane_z, offset[0], offset[1], offset[2], weight}, {}}};
+  hipStream_t st = (hipStream_t)stream;
+  for (int64_t c0 = 0; c0 < n;) {
+    const int64_t left = n - c0;
+    for (int k = 0; k < 8; ++k) gen.d.out[k] = out[k] + c0;
+    gen.first = first + (uint64_t)c0;
+    if (left <= ROWS_MAX_256) return launch_rows<256, ROWS_GENERATE>(nullptr, 0, left, a, gen, nullptr, 0, st);
+    int64_t m = std::min(left, z_rows);
+    if (m < left) m -= m % ROUND_256;  // whole rounds but for the last launch
+    else if (m % ROUND_256 <= ROWS_MAX_256 && m > ROUND_256) m -= m % ROUND_256;
+    if (m <= 0) return GH_EINVAL;  // z_rows too small
+    int r = launch_w8<true, true>(nullptr, 0, m, a, gen, Z, 8, st);
+    if (r != GH_OK) return r;
+    r = gh_exitplane_decode(Z, 8, m, qtab, n_knots, g_max, focal, plane_z, offset, weight, gen.d.out, stream);
+    if (r != GH_OK) return r;
+    c0 += m;
+  }
+  return GH_OK;
 }
 
 // ------------------------------------------------------------------ optimiser
@@ -825,38 +940,64 @@ extern "C" int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_
 // valid_cols corner an entry takes the Adam update (with L2 weight decay added to the
 // gradient when decay != 0), outside it the parameter and both moments stay zero (the
 // padding of the bf16 GEMM operands). The bf16 copy, when given, is the parameter rounded to
-// nearest even, ready for the next forward pass; the transposed copy, when given, holds the
-// same values with the rows of a column contiguous, the layout the fused passes read. A
-// thread of a tensor with a transposed copy takes 8 rows of one column, so that the copy's
-// store is one 16-byte store (2-byte stores at the copy's pitch otherwise).
+// nearest even, ready for the next forward pass; the packed copies, when given, hold the same
+// values in the fragment order that the fused passes read. A thread of a tensor with packed
+// copies takes 8 rows of one column: a 16-byte store into the forward copy, and 2-byte stores
+// of 8 consecutive lanes side by side into the backward copy.
 namespace {
 constexpr int ADAM_MAX = 32;
 struct AdamArgs {
   gh_adam_tensor t[ADAM_MAX];
   gh_adam_pack pack[ADAM_MAX];
-  int64_t offset[ADAM_MAX + 1];   // units: entries, or 8-row strips of one column (transposed copy)
+  int64_t offset[ADAM_MAX + 1];   // units: entries, or 8-row strips of one column (packed copies)
   int n;
   float lr, b1, b2, eps, c1, c2;  // c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
 };
 
-__device__ __forceinline__ float adam_entry(const AdamArgs &a, const gh_adam_tensor &t, int64_t r, int64_t c) {
-  const int64_t j = r * t.cols + c;
-  float p = 0.0f, m = 0.0f, v = 0.0f;
-  if (r < t.valid_rows && c < t.valid_cols) {
-    p = t.param[j];
-    const float g = t.decay != 0.0f ? fmaf(t.decay, p, t.grad[j]) : t.grad[j];
-    m = fmaf(a.b1, t.m[j], (1.0f - a.b1) * g);
-    v = fmaf(a.b2, t.v[j], (1.0f - a.b2) * (g * g));
-    const float mh = m * a.c1, vh = v * a.c2;
-    p -= a.lr * mh / (sqrtf(vh) + a.eps);
+// N entries of one column, rows r0..; every load first, so that their latencies overlap
+template <int N>
+__device__ __forceinline__ void adam_entries(const AdamArgs &a, const gh_adam_tensor &t, int64_t r0, int64_t c,
+                                             float (&p)[N]) {
+  float g[N], m[N], v[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    const int64_t j = (r0 + q) * t.cols + c;
+    p[q] = t.param[j];
+    g[q] = t.grad[j];
+    m[q] = t.m[j];
+    v[q] = t.v[j];
   }
-  t.param[j] = p;
-  t.m[j] = m;
-  t.v[j] = v;
-  if (t.param_bf16) ((__bf16 *)t.param_bf16)[j] = f2bf(p);
-  return p;
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    const int64_t j = (r0 + q) * t.cols + c;
+    const bool in = r0 + q < t.valid_rows && c < t.valid_cols;
+    const float gg = t.decay != 0.0f ? fmaf(t.decay, p[q], g[q]) : g[q];
+    m[q] = fmaf(a.b1, m[q], (1.0f - a.b1) * gg);
+    v[q] = fmaf(a.b2, v[q], (1.0f - a.b2) * (gg * gg));
+    const float mh = m[q] * a.c1, vh = v[q] * a.c2;
+    p[q] -= a.lr * mh / (sqrtf(vh) + a.eps);
+    if (!in) p[q] = m[q] = v[q] = 0.0f;
+    t.param[j] = p[q];
+    t.m[j] = m[q];
+    t.v[j] = v[q];
+    if (t.param_bf16) ((__bf16 *)t.param_bf16)[j] = f2bf(p[q]);
+  }
 }
 
+// element (n, k) of a matrix [N][K] in fragment order
+__device__ __forceinline__ int64_t frag_at(int64_t n, int64_t k, int K) {
+  return (((n >> 4) * (K >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (n & 15)) * 8 + (k & 7);
+}
+
+__device__ __forceinline__ void pack_strip(const gh_adam_pack &k, int64_t r, int64_t c, const bf16x8 &v) {
+  *(bf16x8 *)((__bf16 *)k.forward + frag_at(c, 8 * r, k.forward_k)) = v;
+  if (k.backward)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) ((__bf16 *)k.backward)[frag_at(8 * r + q, c, k.backward_k)] = v[q];
+}
+
+// UPDATE: the Adam step; otherwise only the bf16 copies of the parameters as they are
+template <bool UPDATE>
 __global__ void __launch_bounds__(256) adam_kernel(AdamArgs a) {
   const int64_t total = a.offset[a.n];
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
@@ -866,49 +1007,83 @@ __global__ void __launch_bounds__(256) adam_kernel(AdamArgs a) {
     const gh_adam_tensor &t = a.t[i];
     const int64_t j = e - a.offset[i];
     const int64_t r = j / t.cols, c = j - r * t.cols;
-    if (!a.pack[i].transposed) {
-      (void)adam_entry(a, t, r, c);
+    const gh_adam_pack &k = a.pack[i];
+    if (!k.forward) {
+      float p[1];
+      if (UPDATE) adam_entries<1>(a, t, r, c, p);
+      else if (t.param_bf16) ((__bf16 *)t.param_bf16)[j] = f2bf(t.param[j]);
     } else {
+      float p[8];
+      if (UPDATE) {
+        adam_entries<8>(a, t, 8 * r, c, p);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          p[q] = t.param[(8 * r + q) * t.cols + c];
+          if (t.param_bf16) ((__bf16 *)t.param_bf16)[(8 * r + q) * t.cols + c] = f2bf(p[q]);
+        }
+      }
       bf16x8 v;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = f2bf(adam_entry(a, t, 8 * r + k, c));
-      *(bf16x8 *)((__bf16 *)a.pack[i].transposed + c * a.pack[i].ld + 8 * r) = v;
+      for (int q = 0; q < 8; ++q) v[q] = f2bf(p[q]);
+      pack_strip(k, r, c, v);
     }
   }
 }
-}  // namespace
 
-extern "C" int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors,
-                                   float lr, float beta1, float beta2, float eps, int32_t step, void *stream) {
-  if (!tensors || n_tensors <= 0 || n_tensors > ADAM_MAX || step <= 0 || !(lr >= 0.0f) || !(beta1 >= 0.0f) ||
-      !(beta1 < 1.0f) || !(beta2 >= 0.0f) || !(beta2 < 1.0f) || !(eps > 0.0f))
-    return GH_EINVAL;
-  AdamArgs a{};
-  a.n = n_tensors;
+// tensors and copies of a launch into a; state: gradients and moments are needed
+int adam_tensors(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int n, bool state, AdamArgs &a) {
+  if (!tensors || n <= 0 || n > ADAM_MAX) return GH_EINVAL;
+  a.n = n;
   a.offset[0] = 0;
-  for (int i = 0; i < n_tensors; ++i) {
+  for (int i = 0; i < n; ++i) {
     const gh_adam_tensor &t = tensors[i];
-    if (!t.param || !t.grad || !t.m || !t.v || t.rows <= 0 || t.cols <= 0 || t.valid_rows < 0 ||
+    if (!t.param || (state && (!t.grad || !t.m || !t.v)) || t.rows <= 0 || t.cols <= 0 || t.valid_rows < 0 ||
         t.valid_cols < 0 || t.valid_rows > t.rows || t.valid_cols > t.cols)
       return GH_EINVAL;
     a.t[i] = t;
-    if (packs && packs[i].transposed) {
+    if (packs && packs[i].forward) {
       const gh_adam_pack &k = packs[i];
-      if (t.rows % 8 != 0 || k.ld < t.rows || k.ld % 8 != 0 || (uintptr_t)k.transposed % 16 != 0) return GH_EINVAL;
+      if (t.rows % 8 != 0 || k.forward_k < t.rows || k.forward_k % 32 != 0 || (uintptr_t)k.forward % 16 != 0 ||
+          (k.backward && (k.backward_k < t.cols || k.backward_k % 32 != 0)))
+        return GH_EINVAL;
       a.pack[i] = k;
     }
-    a.offset[i + 1] = a.offset[i] + (int64_t)t.rows * t.cols / (a.pack[i].transposed ? 8 : 1);
+    a.offset[i + 1] = a.offset[i] + (int64_t)t.rows * t.cols / (a.pack[i].forward ? 8 : 1);
   }
+  return GH_OK;
+}
+
+template <bool UPDATE>
+int launch_adam(const AdamArgs &a, hipStream_t st) {
+  const unsigned grid = (unsigned)std::min<int64_t>((a.offset[a.n] + 255) / 256, 2048);
+  hipLaunchKernelGGL(adam_kernel<UPDATE>, dim3(grid), dim3(256), 0, st, a);
+  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+}
+}  // namespace
+
+extern "C" int gh_pack_weights(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors,
+                               void *stream) {
+  AdamArgs a{};
+  const int rc = adam_tensors(tensors, packs, n_tensors, false, a);
+  return rc != GH_OK ? rc : launch_adam<false>(a, (hipStream_t)stream);
+}
+
+extern "C" int gh_adam_step_packed(const gh_adam_tensor *tensors, const gh_adam_pack *packs, int32_t n_tensors,
+                                   float lr, float beta1, float beta2, float eps, int32_t step, void *stream) {
+  if (step <= 0 || !(lr >= 0.0f) || !(beta1 >= 0.0f) || !(beta1 < 1.0f) || !(beta2 >= 0.0f) || !(beta2 < 1.0f) ||
+      !(eps > 0.0f))
+    return GH_EINVAL;
+  AdamArgs a{};
+  const int rc = adam_tensors(tensors, packs, n_tensors, true, a);
+  if (rc != GH_OK) return rc;
   a.lr = lr;
   a.b1 = beta1;
   a.b2 = beta2;
   a.eps = eps;
   a.c1 = (float)(1.0 / (1.0 - std::pow((double)beta1, (double)step)));
   a.c2 = (float)(1.0 / (1.0 - std::pow((double)beta2, (double)step)));
-  const int64_t total = a.offset[n_tensors];
-  const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 2048);
-  hipLaunchKernelGGL(adam_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream, a);
-  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+  return launch_adam<true>(a, (hipStream_t)stream);
 }
 
 extern "C" int gh_adam_step(const gh_adam_tensor *tensors, int32_t n_tensors, float lr, float beta1, float beta2,

@@ -23,17 +23,17 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------ input gradients
 // G_l = dLoss/dZ_l. G_{L-1} is the caller's; G_{l-1} = (G_l W_l^T) * relu'(Z_{l-1}), the
 // derivative taken from the kept activation (bf16(relu(z)) > 0 where z > 0). Same tile, same
-// register-held weights as the forward kernel; W_l [K][N] is read as it is (its rows are the
-// outputs of this product). The bias gradients are column sums of the FP32 gradients before
+// register-held weights as the forward kernel (the rows of W_l [K][N] are the outputs of this
+// product). The bias gradients are column sums of the FP32 gradients before
 // their rounding to bf16: each workgroup writes the sums of its rows.
 struct BackArgs {
-  const __bf16 *w[MAXL];  // layer l >= 1: [K_l][N_l], N_l contiguous (N of the last layer: np)
-  const __bf16 *y[MAXL];  // kept activations
-  __bf16 *g[MAXL];        // out: G_l for l <= L-2, M x H
-  __bf16 *g_out;          // out: bf16(G_{L-1}), M x 16, zeros from n_out on
+  const __bf16 *w[MAXL];  // layer l >= 1: W_l [K_l][N_l] in fragment order (N of the last layer: 32)
+  const __bf16 *y[MAXL];  // kept activations (MlpKeep order)
+  __bf16 *g[MAXL];        // out: G_l for l <= L-2, in the same order
+  __bf16 *g_out;          // out: bf16(G_{L-1}), 32 columns, in the same order
   float *g32[MAXL];       // out, optional: the FP32 gradients of the hidden layers, M x H
   float *db;              // out: [workgroup][(L-1) H + 16] partial sums (layer 0 first)
-  int n_layers, n_out, np;
+  int n_layers, n_out;
 };
 
 template <int H, int RT>
@@ -43,28 +43,27 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
   extern __shared__ __align__(16) unsigned char mlp_lds[];
   __shared__ float s_last[ROW_THREADS / 64][NOUT];
   __bf16 *in = (__bf16 *)mlp_lds, *out = in + ROWS * H;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int fr = lane & 15, g = lane >> 4, fk = g * 8;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, g = lane >> 4;
   const int n0 = wave * 16 * CT;
   const int64_t row0 = (int64_t)blockIdx.x * ROWS;
   const int L = a.n_layers;
   float *db = a.db + (int64_t)blockIdx.x * ((L - 1) * H + NOUT);
-  bf16x8 w0[1][CT], wA[NK][CT], wB[NK][CT];
+  bf16x8 w0[CT], w[NK][CT];
 #pragma unroll
-  for (int j = 0; j < CT; ++j)
-    w0[0][j] = fk < a.np ? *(const bf16x8 *)(a.w[L - 1] + (int64_t)(n0 + j * 16 + fr) * a.np + fk) : bf16x8_zero();
+  for (int j = 0; j < CT; ++j) w0[j] = *(const bf16x8 *)(a.w[L - 1] + ((wave * CT + j) * 64 + lane) * 8);
   // output gradient tile: bf16, padded to 32 columns
   for (int u = tid; u < ROWS * 4; u += ROW_THREADS) {
     const int r = u >> 2, q = (u & 3) * 8;
     const int64_t gr = row0 + r;
     bf16x8 v = bf16x8_zero();
-    if (gr < M && q < NOUT) {
+    if (gr < M) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (q + j < a.n_out) v[j] = (__bf16)G[gr * ldg + q + j];
-      *(bf16x8 *)(a.g_out + gr * NOUT + q) = v;
     }
     *(bf16x8 *)(in + (((r >> 4) * NK) * 64 + (u & 3) * 16 + (r & 15)) * 8) = v;
+    if (gr < padded_rows(M)) *(bf16x8 *)(a.g_out + row0 * K0 + ((r >> 4) * 64 + (u & 3) * 16 + (r & 15)) * 8) = v;
   }
   {
     // its column sums: thread (row tid / 16, column tid % 16), then lanes, then waves
@@ -77,10 +76,7 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
   }
   floatx4 acc[RT][CT];
   bf16x4 y[RT][CT];
-  auto fetch_w = [&](bf16x8(&w)[NK][CT], int l) {
-    if (l >= 1) rows_weights<CT, NK>(w, a.w[l], H, n0, 16, fr, fk);
-    __builtin_amdgcn_sched_barrier(0);
-  };
+  auto tiles = [&](int l) { return a.w[max(l, 1)] + wave * CT * NK * 512 + lane * 8; };
   auto fetch_y = [&](int l) {
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -89,7 +85,7 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
         const int64_t row = row0 + i * 16 + fr;
 #pragma unroll
         for (int r = 0; r < 4; ++r) y[i][j][r] = (__bf16)0.0f;
-        if (row < M) y[i][j] = *(const bf16x4 *)(a.y[l] + row * H + n0 + j * 16 + g * 4);
+        if (row < M) y[i][j] = *(const bf16x4 *)(a.y[l] + row0 * H + rows_at<NK>(i, fr, n0 + j * 16 + g * 4));
       }
   };
   // times the ReLU derivative; column sums; bf16 to the other buffer and to memory
@@ -109,11 +105,10 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
           v[r] = (__bf16)z[r];
         }
         *(bf16x4 *)(out + rows_at<NK>(i, fr, c)) = v;
+        // (rows from M on are exact zeros: their output gradients are)
         const int64_t row = row0 + i * 16 + fr;
-        if (row < M) {
-          *(bf16x4 *)(a.g[l] + row * H + c) = v;
-          if (a.g32[l]) *(floatx4 *)(a.g32[l] + row * H + c) = z;
-        }
+        if (row < padded_rows(M)) *(bf16x4 *)(a.g[l] + row0 * H + rows_at<NK>(i, fr, c)) = v;
+        if (a.g32[l] && row < M) *(floatx4 *)(a.g32[l] + row * H + c) = z;
       }
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1)
@@ -124,13 +119,8 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
     __syncthreads();
     __bf16 *t = in; in = out; out = t;
   };
-  auto hidden = [&](int l, bf16x8(&w)[NK][CT]) {  // G_{l-1} from G_l
-    rows_zero<RT, CT>(acc);
-    rows_mma<RT, CT, NK, NK, NK>(acc, w, in, lane);
-    finish(l - 1);
-  };
   fetch_y(L - 2);
-  fetch_w(wA, L - 2);
+  if (L > 2) rows_weights<CT, NK>(w, tiles(L - 2), NK * 512);
   __syncthreads();
   if (tid < NOUT) {
     float s = 0.0f;
@@ -139,33 +129,33 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_backward(const float *__
     db[(L - 1) * H + tid] = s;
   }
   rows_zero<RT, CT>(acc);
-  rows_mma<RT, CT, 1, NK, 1>(acc, w0, in, lane);
+  rows_mma0<RT, CT, NK>(acc, w0, in, lane);
   finish(L - 2);
-  for (int l = L - 2; l >= 1; l -= 2) {
+  for (int l = L - 2; l >= 1; --l) {  // G_{l-1} from G_l
     fetch_y(l - 1);
-    fetch_w(wB, l - 1);
-    hidden(l, wA);
-    if (l == 1) break;
-    fetch_y(l - 2);
-    fetch_w(wA, l - 2);
-    hidden(l - 1, wB);
+    rows_zero<RT, CT>(acc);
+    rows_mma<RT, CT, NK>(acc, w, in, lane, tiles(l - 1), NK * 512);
+    finish(l - 1);
   }
 }
 
 // ------------------------------------------------------------------ weight gradients
-// dW_l = X_l^T G_l: reductions over the batch of two row-major matrices. All layers in one
-// launch: blockIdx.x is an output tile of some layer, blockIdx.y a slice of the rows. The slices
-// are those of gh_gemm_bf16 for the same product (its rule: 512 rows from 2048 rows on, 32
-// slices and 256 workgroups for the four inner layers at 16384 rows), so the sums have the
-// same bits. 32 rows
-// of both operands are staged in LDS per step, loaded into registers one step ahead; the
-// fragments (8 consecutive rows of one column) are read with the transposing LDS read
-// (ds_read_b64_tr_b16: lane s of 16 names 4 columns of row s / 4, lane i receives 4 rows of
-// column i), with the 32-byte chunks of a row XOR-swizzled so that the 8 rows of a half wave
-// fall into different banks.
+// dW_l = X_l^T G_l: reductions over the batch of two matrices in MlpKeep order (tiles of 16
+// rows; the input and the output gradient padded to 32 columns, all to a multiple of 32 rows
+// with zeros). All layers in one launch: blockIdx.x is an output tile of some layer, blockIdx.y
+// a slice of the rows. The slices are those of gh_gemm_bf16 for the same product (its rule: 512
+// rows from 2048 rows on, 32 slices and 256 workgroups for the four inner layers at 16384
+// rows), so the sums have the same bits. A step of 32 rows (512 MFMA cycles) is shorter than the
+// latency of its 24 KiB: the steps come through a ring of three LDS stages (two workgroups of
+// 72 KiB per CU), two in flight, by direct global-to-LDS loads of 1 KiB blocks. The fragments (8 consecutive rows of one
+// column) are read with the transposing LDS read (ds_read_b64_tr_b16: lane s of 16 names 4
+// columns of row s / 4, lane i receives 4 rows of column i); the 16-byte units of odd column
+// groups sit at row ^ 4, so that the 8 rows and 2 groups of a half wave fall into different
+// banks.
 struct DwLayer {
-  const __bf16 *A, *B;  // X_l (M x ka, pitch lda) and G_l (M x nb, pitch ldb)
-  int lda, ldb, ka, nb;
+  const __bf16 *A, *B;  // X_l and G_l
+  int na, nb32;         // 32-column blocks per row tile of A and B
+  int ka, nb;           // valid columns of A and B: dW_l is ka x nb
   int rows, slices;     // rows of a slice, number of slices
   float *part;          // [slice][ka nb] partial sums
   int64_t off;          // offset of the layer's ka x nb block in the result
@@ -176,88 +166,87 @@ struct DwArgs {
   int64_t M, n_elems;   // elements of the result
 };
 
-constexpr int DW_THREADS = 512;
+constexpr int DW_THREADS = 512, DW_STAGES = 3;
 
-__device__ __forceinline__ int dw_swizzle(int row, int units) {
-  return (((row & 3) | ((row >> 1) & 4)) << 1) & (units - 1);
+// 16 bytes per lane to LDS at p + 16 lane, p wave-uniform. In asm, so that the compiler does
+// not put its own wait for every load in flight in front of each LDS read and barrier: the
+// caller waits (vmcnt) and then meets a barrier before it reads. No vector register is
+// written; m0 is set where it is used, as the compiler does for its own loads.
+__device__ __forceinline__ void lds_load(const void *p, const void *src) {
+  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
+               : "memory");
 }
 
-// output tile [a0, a0 + TA) x [0, TB) over the waves WA x WB
-template <int TA, int TB, int WA, int WB>
+// output tile [a0, a0 + TA) x [0, TB) over the waves WA x WB, FA x FB fragments each
+template <int TA, int TB, int WA, int WB, int FA, int FB>
 __device__ __forceinline__ void dw_tile(const DwLayer &d, int a0, int64_t r0, int64_t r1, float *part,
                                         unsigned char *lds) {
-  constexpr int UA = TA / 8, UB = TB / 8, UNITS = 32 * (UA + UB), NU = (UNITS + DW_THREADS - 1) / DW_THREADS;
-  constexpr int FA = TA / 16 / WA, FB = TB / 16 / WB, STAGE = 32 * (TA + TB);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int BA = TA / 32, BB = TB / 32, BLOCKS = 2 * (BA + BB), PER_WAVE = (BLOCKS + 7) / 8;
+  constexpr int STAGE = BLOCKS * 512;  // elements
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wa = wave / WB, wb = wave % WB;
   const int s = lane & 15, g = lane >> 4;
   __bf16 *buf = (__bf16 *)lds;
-  bf16x8 reg[NU];
-  auto load = [&](int64_t row) {
+  const int swz = ((lane >> 4) & 1) << 2;  // of the unit (column group lane / 16, row lane % 16)
+  const int steps = (int)((r1 - r0 + 31) >> 5);
+  // block b of a stage: row tile b / (BA + BB), then A's blocks, then B's; a wave without a
+  // PER_WAVE-th block loads an earlier one again, so that every wave waits for the same count
+  const __bf16 *src[PER_WAVE];
+  int stride[PER_WAVE];  // per step
 #pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      const int u = tid + k * DW_THREADS;
-      reg[k] = bf16x8_zero();
-      if (u < 32 * UA) {
-        const int64_t r = row + u / UA;
-        const int c = a0 + (u % UA) * 8;
-        if (r < r1 && c < d.ka) reg[k] = *(const bf16x8 *)(d.A + r * d.lda + c);
-      } else if (u < UNITS) {
-        const int64_t r = row + (u - 32 * UA) / UB;
-        const int c = ((u - 32 * UA) % UB) * 8;
-        if (r < r1 && c < d.nb) reg[k] = *(const bf16x8 *)(d.B + r * d.ldb + c);
-      }
-    }
-  };
-  auto store = [&](__bf16 *b) {
+  for (int k = 0; k < PER_WAVE; ++k) {
+    const int b = (wave + 8 * k) % BLOCKS;
+    const int64_t tile = (r0 >> 4) + b / (BA + BB);
+    const int q = b % (BA + BB);
+    src[k] = (q < BA ? d.A + (tile * d.na + (a0 >> 5) + q) * 512 : d.B + (tile * d.nb32 + (q - BA)) * 512) +
+             (lane ^ swz) * 8;
+    stride[k] = (q < BA ? d.na : d.nb32) * 1024;
+  }
+  auto load = [&](int t) {
+    const __bf16 *stage = buf + (t % DW_STAGES) * STAGE;
 #pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      const int u = tid + k * DW_THREADS;
-      if (u < 32 * UA) {
-        const int r = u / UA, c = u % UA;
-        *(bf16x8 *)(b + r * TA + ((c ^ dw_swizzle(r, UA)) << 3)) = reg[k];
-      } else if (u < UNITS) {
-        const int r = (u - 32 * UA) / UB, c = (u - 32 * UA) % UB;
-        *(bf16x8 *)(b + 32 * TA + r * TB + ((c ^ dw_swizzle(r, UB)) << 3)) = reg[k];
-      }
-    }
+    for (int k = 0; k < PER_WAVE; ++k)
+      lds_load(stage + ((wave + 8 * k) % BLOCKS) * 512, src[k] + (int64_t)t * stride[k]);
   };
-  // fragment of 16 columns from c0 of a staged operand of T columns
-  auto frag = [&](const __bf16 *b, int T, int c0) {
+  // fragment of 16 columns from c0 of a staged operand whose first block is b0
+  auto frag = [&](const __bf16 *stage, int b0, int c0) {
     union { bf16x8 v; s16x4 h[2]; } f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int row = 8 * g + 4 * h + (s >> 2);
-      const int unit = (c0 >> 3) + ((s & 3) >> 1);
-      const __bf16 *p = b + row * T + ((unit ^ dw_swizzle(row, T / 8)) << 3) + (s & 1) * 4;
+      const int row = 8 * (g & 1) + 4 * h + (s >> 2);  // in row tile g / 2
+      const int c = c0 + 4 * (s & 3), kg = (c >> 3) & 3;
+      const __bf16 *p = stage + ((g >> 1) * (BA + BB) + b0 + (c >> 5)) * 512 +
+                        (kg * 16 + (row ^ ((kg & 1) << 2))) * 8 + (c & 4);
       f.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
     }
     return f.v;
   };
   floatx4 acc[FA][FB];
   rows_zero<FA, FB>(acc);
-  load(r0);
-  store(buf);
-  if (r0 + 32 < r1) load(r0 + 32);
-  __syncthreads();
-  int cur = 0;
-  for (int64_t r = r0; r < r1; r += 32) {
-    const __bf16 *b = buf + cur * STAGE;
+#pragma unroll
+  for (int t = 0; t < DW_STAGES - 1; ++t)
+    if (t < steps) load(t);
+  for (int t = 0; t < steps; ++t) {
+    // this wave's blocks of step t have arrived (loads return in order; the next step's in
+    // flight) and its LDS reads of step t - 1 are done; after the barrier that holds for
+    // every wave, and the next load may refill the stage of step t - 1
+    if (t + 1 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER_WAVE) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + DW_STAGES - 1 < steps) load(t + DW_STAGES - 1);
+    const __bf16 *stage = buf + (t % DW_STAGES) * STAGE;
     bf16x8 af[FA], bf[FB];
 #pragma unroll
-    for (int i = 0; i < FA; ++i) af[i] = frag(b, TA, (wa * FA + i) * 16);
+    for (int i = 0; i < FA; ++i) af[i] = frag(stage, 0, (wa * FA + i) * 16);
 #pragma unroll
-    for (int j = 0; j < FB; ++j) bf[j] = frag(b + 32 * TA, TB, (wb * FB + j) * 16);
-    // the other buffer was last read before the barrier that ended the step before
-    if (r + 32 < r1) store(buf + (cur ^ 1) * STAGE);
-    if (r + 64 < r1) load(r + 64);
+    for (int j = 0; j < FB; ++j) bf[j] = frag(stage, BA, (wb * FB + j) * 16);
 #pragma unroll
     for (int i = 0; i < FA; ++i)
 #pragma unroll
       for (int j = 0; j < FB; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-    cur ^= 1;
   }
 #pragma unroll
   for (int i = 0; i < FA; ++i)
@@ -274,8 +263,7 @@ __device__ __forceinline__ void dw_tile(const DwLayer &d, int a0, int64_t r0, in
 
 template <int H>
 __global__ void __launch_bounds__(DW_THREADS) mlp_weight_grad(DwArgs a) {
-  __shared__ __align__(16) unsigned char lds[2 * 32 * (128 + H) * sizeof(__bf16)];
-  static_assert(128 + H >= H + 32, "the thin tiles fit the same stages");
+  extern __shared__ __align__(16) unsigned char lds[];  // DW_STAGES stages of 32 rows x (128 + H) columns
   constexpr int TILES = H / 128;  // tiles of an inner layer: 128 of its rows, all columns
   const int inner = (a.n_layers - 2) * TILES;
   const int b = blockIdx.x;
@@ -285,9 +273,9 @@ __global__ void __launch_bounds__(DW_THREADS) mlp_weight_grad(DwArgs a) {
   const int64_t r0 = (int64_t)blockIdx.y * d.rows;
   const int64_t r1 = min(a.M, r0 + d.rows);
   float *part = d.part + (int64_t)blockIdx.y * d.ka * d.nb;
-  if (b < inner) dw_tile<128, H, 2, 4>(d, (b % TILES) * 128, r0, r1, part, lds);
-  else if (b == inner) dw_tile<K0, H, 1, 8>(d, 0, r0, r1, part, lds);
-  else dw_tile<H, NOUT, 8, 1>(d, 0, r0, r1, part, lds);
+  if (b < inner) dw_tile<128, H, 2, 4, 4, H / 64>(d, (b % TILES) * 128, r0, r1, part, lds);
+  else if (b == inner) dw_tile<K0, H, 1, 8, 2, H / 128>(d, 0, r0, r1, part, lds);
+  else dw_tile<H, K0, 8, 1, H / 128, 1>(d, 0, r0, r1, part, lds);
 }
 
 // dW = sum of the slices in order; db = sum of the workgroups' column sums (blocks from
@@ -340,9 +328,10 @@ Sizes train_sizes(int64_t M, int L, int k_in, int H, int np, DwLayer *layer = nu
   Sizes z{};
   for (int l = 0; l < L; ++l) {
     DwLayer d{};
-    d.lda = d.ka = l == 0 ? k_in : H;
-    d.ldb = l == L - 1 ? NOUT : H;
+    d.ka = l == 0 ? k_in : H;
+    d.na = l == 0 ? 1 : H / 32;
     d.nb = l == L - 1 ? np : H;
+    d.nb32 = l == L - 1 ? 1 : H / 32;
     gh::splitk_plan(d.ka, d.nb, (int)M, GH_EPI_STORE, d.slices, d.rows);
     d.off = z.n_elems;
     z.n_elems += (int64_t)d.ka * d.nb;
@@ -350,11 +339,10 @@ Sizes train_sizes(int64_t M, int L, int k_in, int H, int np, DwLayer *layer = nu
     z.slices = std::max<int64_t>(z.slices, d.slices);
     if (layer) layer[l] = d;
   }
-  const int tile = 16 * row_tiles(M);
-  z.wgs = (M + tile - 1) / tile;
+  z.wgs = row_grid(M, row_tiles(M));
   z.db_pitch = (int64_t)(L - 1) * H + NOUT;
-  z.g_bytes = (size_t)(L - 1) * M * H * 2;
-  z.gout_bytes = (size_t)M * NOUT * 2;
+  z.g_bytes = (size_t)(L - 1) * padded_rows(M) * H * 2;
+  z.gout_bytes = (size_t)padded_rows(M) * K0 * 2;
   z.part_bytes = (size_t)z.part_elems * 4;
   z.db_bytes = (size_t)z.wgs * z.db_pitch * 4;
   return z;
@@ -368,7 +356,7 @@ bool sizes_ok(int64_t M, int L, int k_in, int H, int n_out, int np) {
 
 template <int H, int RT>
 int launch_backward(const float *G, int64_t ldg, int64_t M, const BackArgs &a, hipStream_t st) {
-  const dim3 grid((unsigned)((M + 16 * RT - 1) / (16 * RT)));
+  const dim3 grid((unsigned)row_grid(M, RT));
   constexpr size_t lds = rows_lds_bytes<H, RT>();
   const void *fn = (const void *)&mlp_rows_backward<H, RT>;
   if (lds + 1024 > 64 * 1024 &&
@@ -383,9 +371,9 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace
 
 extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
-                                         int32_t n_out, const void *const *wt, const float *const *bias,
+                                         int32_t n_out, const void *const *wt, const float *const *bias, void *Xt,
                                          void *const *Y, float *Z, int64_t ldz, void *stream) {
-  if (!X || !wt || !bias || !Y || !Z || ldz < n_out || !sizes_ok(M, n_layers, k_in, hidden, n_out, NOUT))
+  if (!X || !wt || !bias || !Xt || !aligned16(Xt) || !Y || !Z || ldz < n_out || !sizes_ok(M, n_layers, k_in, hidden, n_out, NOUT))
     return GH_EINVAL;
   MlpArgs a{};
   MlpKeep keep{};
@@ -393,6 +381,7 @@ extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_lay
   a.k_in = k_in;
   a.n_out = n_out;
   a.x_vec = 1;
+  keep.x = (__bf16 *)Xt;
   if (!aligned16(X)) return GH_EINVAL;
   for (int l = 0; l < n_layers; ++l) {
     if (!wt[l] || !bias[l] || !aligned16(wt[l]) || (l < n_layers - 1 && (!Y[l] || !aligned16(Y[l]) || !aligned16(bias[l]))))
@@ -405,9 +394,9 @@ extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_lay
   hipStream_t st = (hipStream_t)stream;
   const int rt = row_tiles(M);
 #define GH_ROWS(H)                                                                  \
-  (rt == 1 ? launch_rows_forward<H, 1, true>(x, k_in, M, a, keep, Z, ldz, st)       \
-           : (rt == 2 ? launch_rows_forward<H, 2, true>(x, k_in, M, a, keep, Z, ldz, st) \
-                      : launch_rows_forward<H, 4, true>(x, k_in, M, a, keep, Z, ldz, st)))
+  (rt == 1 ? launch_rows_forward<H, 1, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)       \
+           : (rt == 2 ? launch_rows_forward<H, 2, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st) \
+                      : launch_rows_forward<H, 4, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)))
   return hidden == 256 ? GH_ROWS(256) : GH_ROWS(128);
 #undef GH_ROWS
 }
@@ -419,16 +408,16 @@ extern "C" int gh_mlp_train_workspace(int64_t M, int32_t n_layers, int32_t k_in,
   return GH_OK;
 }
 
-extern "C" int gh_mlp_train_backward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
+extern "C" int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
                                           int32_t n_out, int32_t np, const void *const *w, const void *const *Y,
                                           const float *G, int64_t ldg, float *dW, float *db, float *const *G32, void *ws,
                                           int64_t ws_bytes, void *stream) {
-  if (!X || !w || !Y || !G || !dW || !db || !ws || ldg < n_out || !sizes_ok(M, n_layers, k_in, hidden, n_out, np))
+  if (!Xt || !w || !Y || !G || !dW || !db || !ws || ldg < n_out || !sizes_ok(M, n_layers, k_in, hidden, n_out, np))
     return GH_EINVAL;
   const int L = n_layers;
   DwArgs d{};
   const Sizes z = train_sizes(M, L, k_in, hidden, np, d.layer);
-  if (ws_bytes < (int64_t)z.total() || !aligned16(ws) || !aligned16(X) || !aligned16(dW)) return GH_EINVAL;
+  if (ws_bytes < (int64_t)z.total() || !aligned16(ws) || !aligned16(Xt) || !aligned16(dW)) return GH_EINVAL;
   for (int l = 0; l < L; ++l)
     if ((l > 0 && (!w[l] || !aligned16(w[l]))) ||
         (l < L - 1 && (!Y[l] || !aligned16(Y[l]) || (G32 && (!G32[l] || !aligned16(G32[l]))))))
@@ -437,9 +426,8 @@ extern "C" int gh_mlp_train_backward_bf16(const void *X, int64_t M, int32_t n_la
   BackArgs a{};
   a.n_layers = L;
   a.n_out = n_out;
-  a.np = np;
   for (int l = 0; l < L - 1; ++l) {
-    a.g[l] = (__bf16 *)(p + (size_t)l * M * hidden * 2);
+    a.g[l] = (__bf16 *)(p + (size_t)l * padded_rows(M) * hidden * 2);
     a.y[l] = (const __bf16 *)Y[l];
     if (G32) a.g32[l] = G32[l];
   }
@@ -462,14 +450,21 @@ extern "C" int gh_mlp_train_backward_bf16(const void *X, int64_t M, int32_t n_la
   d.M = M;
   d.n_elems = z.n_elems;
   for (int l = 0; l < L; ++l) {
-    d.layer[l].A = l == 0 ? (const __bf16 *)X : a.y[l - 1];
+    d.layer[l].A = l == 0 ? (const __bf16 *)Xt : a.y[l - 1];
     d.layer[l].B = l == L - 1 ? a.g_out : a.g[l];
     d.layer[l].part = part;
     part += (int64_t)d.layer[l].ka * d.layer[l].nb * d.layer[l].slices;
   }
   const dim3 grid((unsigned)((L - 2) * (hidden / 128) + 2), (unsigned)z.slices);
-  if (hidden == 256) hipLaunchKernelGGL(mlp_weight_grad<256>, grid, dim3(DW_THREADS), 0, st, d);
-  else hipLaunchKernelGGL(mlp_weight_grad<128>, grid, dim3(DW_THREADS), 0, st, d);
+  const size_t lds = (size_t)DW_STAGES * 32 * (128 + hidden) * sizeof(__bf16);
+  if (hidden == 256) {
+    if (hipFuncSetAttribute((const void *)&mlp_weight_grad<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
+      return GH_EHIP;
+    hipLaunchKernelGGL(mlp_weight_grad<256>, grid, dim3(DW_THREADS), lds, st, d);
+  } else {
+    hipLaunchKernelGGL(mlp_weight_grad<128>, grid, dim3(DW_THREADS), lds, st, d);
+  }
   if (hipGetLastError() != hipSuccess) return GH_EHIP;
   const int n_db = (L - 1) * hidden + np;
   const int dw_blocks = (int)((z.n_elems / 4 + 255) / 256);

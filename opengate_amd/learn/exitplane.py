@@ -34,7 +34,7 @@ import time
 import numpy as np
 
 from .. import _abi as A
-from .mlp import MLP
+from .mlp import MLP, _pointers
 
 SIZES = [8, 256, 256, 256, 256, 256, 6]
 N_FEATURES = 6
@@ -218,6 +218,8 @@ class ExitPlaneGenerator:
         if out is None:
             out = [torch.empty(n, device=self.dev, dtype=torch.float32) for _ in range(8)]
         m = min(int(chunk), max(n, 1))
+        if events is None and n > 0 and self._one_call():
+            return self._generate(n, seed, first, out, m, weight)
         X = torch.empty(m, self.mlp.psizes[0], device=self.dev, dtype=torch.bfloat16)
         bufs = None
         if not self.mlp.fused_ok():
@@ -246,6 +248,25 @@ class ExitPlaneGenerator:
                                               _stream())
             if rc != 0:
                 raise RuntimeError(f"gh_exitplane_decode failed ({rc})")
+        return out
+
+    def _one_call(self):
+        """gh_exitplane_generate takes this network: hidden width 256, and the 6 features as its
+        outputs."""
+        return self.mlp.Wf is not None and self.mlp.psizes[1] == 256 and self.sizes[-1] == 6
+
+    def _generate(self, n, seed, first, out, m, weight):
+        """Noise, network and decoder in one call; m: photons per launch of the network."""
+        rows = 0 if n <= 32768 else max(m, 65536)
+        Z = _torch().empty(rows, 8, device=self.dev, dtype=_torch().float32) if rows else None
+        wp, bp, hold = self.mlp._fused_args()
+        rc = self.lib.gh_exitplane_generate(int(seed) & (2**64 - 1), int(first), n, self.sizes[0], len(self.sizes) - 1,
+                                            256, wp, bp, self.qmap.qtab.data_ptr(), self.qmap.n_knots, self.qmap.g_max,
+                                            (C.c_float * 3)(*self.focal), self.plane_z, (C.c_float * 3)(), float(weight),
+                                            _pointers(out), None if Z is None else Z.data_ptr(), rows, _stream())
+        del hold
+        if rc != 0:
+            raise RuntimeError(f"gh_exitplane_generate failed ({rc})")
         return out
 
     def flops_per_photon(self):

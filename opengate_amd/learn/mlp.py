@@ -28,16 +28,33 @@ def _torch():
 
 # the C layouts of gh_adam_tensor and gh_adam_pack
 _ADAM = struct.Struct("=5Q4ifi")
-_PACK = struct.Struct("=Q2i")
+_PACK = struct.Struct("=2Q2i")
 
 
 def _pointers(tensors):
     """Device addresses of tensors as a C array of pointers."""
-    return struct.pack(f"={len(tensors)}Q", *[t.data_ptr() for t in tensors])
+    return struct.pack(f"={len(tensors)}Q", *[0 if t is None else t.data_ptr() for t in tensors])
+
+
+def pad(n, q):
+    return (n + q - 1) // q * q
 
 
 def pad8(n):
-    return (n + 7) // 8 * 8
+    return pad(n, 8)
+
+
+def fragment_order(w, out):
+    """Matrix w [N][K] into out, a flat bf16 buffer in fragment order (include/gatehip.h): N
+    padded to 16, K to 32 with zeros. Returns out."""
+    torch = _torch()
+    n, k = w.shape
+    t = torch.zeros(pad(n, 16), pad(k, 32), device=w.device, dtype=torch.bfloat16)
+    t[:n, :k] = w
+    # (n tile, n, k step, k group, k) -> (n tile, k step, k group, n, k)
+    out.view(t.shape[0] // 16, t.shape[1] // 32, 4, 16, 8).copy_(
+        t.view(t.shape[0] // 16, 16, t.shape[1] // 32, 4, 8).permute(0, 2, 3, 1, 4))
+    return out
 
 
 class MLP:
@@ -64,22 +81,40 @@ class MLP:
 
     # ------------------------------------------------------------------ helpers
     def _refresh(self):
-        """bf16 copies of the weights (kept in place: the optimiser kernel writes them) and, for
-        the fused kernels, their transposes [N][K] (first layer K -> 32, last layer N -> 16)."""
+        """bf16 copies of the weights (kept in place: the optimiser kernel writes them): row-major
+        and, for the fused kernels, the forward (W^T) and backward (W) copies in fragment order."""
         torch = _torch()
         if getattr(self, "W16", None) is None or [t.shape for t in self.W16] != [w.shape for w in self.W]:
             self.W16 = [torch.empty(w.shape, device=self.dev, dtype=torch.bfloat16) for w in self.W]
-            self.Wt = None
+            self.Wf = self.Wb = None
             if self.fused_ok():
+                sizes = [pad(w.shape[1], 16) * pad(w.shape[0], 32) for w in self.W16]
+                sizes += [pad(w.shape[0], 16) * pad(w.shape[1], 32) for w in self.W16[1:]]
+                copies = torch.zeros(sum(sizes), device=self.dev, dtype=torch.bfloat16).split(sizes)
                 L = len(self.W16)
-                self.Wt = [torch.zeros(self.FUSED_N_OUT if l == L - 1 else w.shape[1],
-                                       self.FUSED_K_IN if l == 0 else w.shape[0], device=self.dev, dtype=torch.bfloat16)
-                           for l, w in enumerate(self.W16)]
+                self.Wf, self.Wb = list(copies[:L]), [None, *copies[L:]]
+        if self.dev.type == "cuda" and all(w.is_contiguous() for w in self.W):
+            tab = [_ADAM.pack(w.data_ptr(), 0, 0, 0, t.data_ptr(), *w.shape, 0, 0, 0.0, 0)
+                   for w, t in zip(self.W, self.W16)]
+            rc = self.lib.gh_pack_weights(b"".join(tab), b"".join(map(self._pack, range(len(tab)))), len(tab),
+                                          self._stream())
+            if rc != 0:
+                raise RuntimeError(f"gh_pack_weights failed ({rc})")
+            return
         for t, w in zip(self.W16, self.W):
             t.copy_(w)
-        if self.Wt is not None:
-            for t, w in zip(self.Wt, self.W16):
-                t[:w.shape[1], :w.shape[0]] = w.t()
+        if self.Wf is not None:
+            for l, w in enumerate(self.W16):
+                fragment_order(w.t(), self.Wf[l])
+                if l:
+                    fragment_order(w, self.Wb[l])
+
+    def _pack(self, l):
+        """gh_adam_pack of weight l."""
+        if self.Wf is None:
+            return _PACK.pack(0, 0, 0, 0)
+        return _PACK.pack(self.Wf[l].data_ptr(), self.Wb[l].data_ptr() if l else 0, pad(self.W[l].shape[0], 32),
+                          pad(self.W[l].shape[1], 32))
 
     def _stream(self):
         return C.c_void_p(_torch().cuda.current_stream().cuda_stream)
@@ -151,22 +186,22 @@ class MLP:
     TRAIN_MAX_ROWS = 4194240  # GH_MLP_TRAIN_MAX_ROWS
 
     def fused_ok(self):
-        """gh_mlp_forward_bf16 handles 2..8 layers with equal hidden widths of 128 or 256,
+        """gh_mlp_forward_packed_bf16 handles 2..8 layers with equal hidden widths of 128 or 256,
         at most 32 inputs and 16 outputs."""
         hidden = set(self.psizes[1:-1])
         return (2 <= len(self.W) <= self.FUSED_MAX_LAYERS and len(hidden) == 1 and hidden <= {128, 256}
                 and self.psizes[0] <= self.FUSED_K_IN and self.psizes[-1] <= self.FUSED_N_OUT)
 
     def _fused_args(self):
-        """Pointer arrays (bytes) of the transposed weights and the biases; the tensors they
+        """Pointer arrays (bytes) of the forward weight copies and the biases; the tensors they
         point to stay referenced by the returned list."""
         bs = [b if b.is_contiguous() and b.data_ptr() % 16 == 0 else b.clone(memory_format=_torch().contiguous_format)
               for b in self.b]
-        return _pointers(self.Wt), _pointers(bs), bs
+        return _pointers(self.Wf), _pointers(bs), bs
 
     def _train_fused(self, X):
         """gh_mlp_train_* take the network and this batch."""
-        return self.Wt is not None and 1 <= X.shape[0] <= self.TRAIN_MAX_ROWS and X.data_ptr() % 16 == 0
+        return self.Wf is not None and 1 <= X.shape[0] <= self.TRAIN_MAX_ROWS and X.data_ptr() % 16 == 0
 
     def _forward_fused(self, X, keep):
         torch = _torch()
@@ -174,26 +209,28 @@ class MLP:
         Z = torch.empty(M, self.psizes[-1], device=self.dev, dtype=torch.float32)
         if not keep:
             return self.infer_fused(X, Z)[:, : self.sizes[-1]]
-        Y = torch.empty(L - 1, M, self.psizes[1], device=self.dev, dtype=torch.bfloat16)
+        Xt = torch.empty(pad(M, 32), self.FUSED_K_IN, device=self.dev, dtype=torch.bfloat16)
+        Y = torch.empty(L - 1, pad(M, 32), self.psizes[1], device=self.dev, dtype=torch.bfloat16)
         wp, bp, hold = self._fused_args()
         rc = self.lib.gh_mlp_train_forward_bf16(X.data_ptr(), M, L, self.psizes[0], self.psizes[1], self.sizes[-1],
-                                                wp, bp, _pointers(Y), Z.data_ptr(), Z.stride(0), self._stream())
+                                                wp, bp, Xt.data_ptr(), _pointers(Y), Z.data_ptr(), Z.stride(0),
+                                                self._stream())
         del hold
         if rc != 0:
             raise RuntimeError(f"gh_mlp_train_forward_bf16 failed ({rc})")
-        self._xs, self._zs = [X, *Y], None
+        self._xs, self._zs = (M, Xt, Y), None
         return Z[:, : self.sizes[-1]]
 
     def _backward_fused(self, grad_out, tensor_sums):
         torch = _torch()
-        X, Y, L = self._xs[0], self._xs[1:], len(self.W)
-        M, k_in, hidden, n_out, n_pad = X.shape[0], self.psizes[0], self.psizes[1], self.sizes[-1], self.psizes[-1]
+        (M, Xt, Y), L = self._xs, len(self.W)
+        k_in, hidden, n_out, n_pad = self.psizes[0], self.psizes[1], self.sizes[-1], self.psizes[-1]
         G, G32 = grad_out, None
         if tensor_sums:
             G = torch.zeros(M, n_pad, device=self.dev, dtype=torch.float32)
             G[:, :n_out] = grad_out
             G32 = torch.empty(L - 1, M, hidden, device=self.dev, dtype=torch.float32)
-        elif G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != X.device or G.stride(1) != 1:
+        elif G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != Xt.device or G.stride(1) != 1:
             G = torch.empty(M, n_out, device=self.dev, dtype=torch.float32)
             G[:] = grad_out
         shapes = [tuple(w.shape) for w in self.W]
@@ -204,7 +241,7 @@ class MLP:
         if rc != 0:
             raise RuntimeError(f"gh_mlp_train_workspace failed ({rc})")
         ws = torch.empty(size.value, device=self.dev, dtype=torch.uint8)
-        rc = self.lib.gh_mlp_train_backward_bf16(X.data_ptr(), M, L, k_in, hidden, n_out, n_pad, _pointers(self.W16),
+        rc = self.lib.gh_mlp_train_backward_bf16(Xt.data_ptr(), M, L, k_in, hidden, n_out, n_pad, _pointers(self.Wb),
                                                  _pointers(Y), G.data_ptr(), G.stride(0), flat.data_ptr(),
                                                  dbf.data_ptr(), None if G32 is None else _pointers(G32),
                                                  ws.data_ptr(), size.value, self._stream())
@@ -219,16 +256,16 @@ class MLP:
         return dW, list(dbf.split([n for _, n in shapes]))
 
     def infer_fused(self, X, out):
-        """All layers in one kernel (gh_mlp_forward_bf16): X (M, in padded) bf16 with row
+        """All layers in one kernel (gh_mlp_forward_packed_bf16): X (M, in padded) bf16 with row
         pitch X.stride(0), out (M, >= out) FP32 with row pitch out.stride(0); only the
         first sizes[-1] columns of out are written. Same values as infer()."""
         wp, bp, hold = self._fused_args()
-        rc = self.lib.gh_mlp_forward_bf16(X.data_ptr(), X.stride(0), X.shape[0], len(self.W), self.psizes[0],
+        rc = self.lib.gh_mlp_forward_packed_bf16(X.data_ptr(), X.stride(0), X.shape[0], len(self.W), self.psizes[0],
                                           self.psizes[1], self.sizes[-1], wp, bp, out.data_ptr(), out.stride(0),
                                           self._stream())
         del hold
         if rc != 0:
-            raise RuntimeError(f"gh_mlp_forward_bf16 failed ({rc})")
+            raise RuntimeError(f"gh_mlp_forward_packed_bf16 failed ({rc})")
         return out
 
     def backward(self, grad_out, tensor_sums=False):
@@ -277,8 +314,7 @@ class MLP:
             tab.append(_ADAM.pack(p.data_ptr(), g.data_ptr(), self.m[i].data_ptr(), self.v[i].data_ptr(),
                                   self.W16[i].data_ptr() if is_w else 0, rows, cols, vr, vc,
                                   float(self.wd) if is_w else 0.0, 0))
-            t = self.Wt[i] if is_w and self.Wt is not None else None
-            packs.append(_PACK.pack(0, 0, 0) if t is None else _PACK.pack(t.data_ptr(), t.shape[1], 0))
+            packs.append(self._pack(i) if is_w else _PACK.pack(0, 0, 0, 0))
         b1, b2 = self.betas
         rc = self.lib.gh_adam_step_packed(b"".join(tab), b"".join(packs), len(params), float(self.lr), float(b1),
                                           float(b2), float(self.eps), self.t, self._stream())
