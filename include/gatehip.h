@@ -366,6 +366,22 @@ int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_layers, int3
                                int32_t np, const void *const *w, const void *const *Y, const float *G, int64_t ldg,
                                float *dW, float *db, float *const *G32, void *ws, int64_t ws_bytes, void *stream);
 
+/* Losses of the training loops with their gradients (no counterpart in the reference's source, as
+ * for gh_adam_step).
+ * gh_sliced_w2: A (pitch lda) and B (pitch ldb): M points of K <= 8 values, M at most
+ * GH_SLICED_W2_MAX_ROWS; dir: K x P directions. With a = A dir and b = B dir (FP32 multiply-adds
+ * in the order of K): loss[c] = sum of the squared differences of the sorted columns c of a and
+ * b; grad (M x P) = d(sum of loss / (M P)) / da (equal values of a column sort by row). work: 2 M P floats of
+ * device memory.
+ * gh_softmax_ce: logits Z (M rows, pitch ldz, n_classes <= 16 columns), class of row i =
+ * cls[rows[i]] (cls[i] with rows NULL), in 0..n_classes-1; loss[b] = sum over rows 256 b ..
+ * 256 b + 255 of the cross-entropy; grad (M x n_classes) = d(sum of loss / M) / dZ. */
+#define GH_SLICED_W2_MAX_ROWS 16384
+int gh_sliced_w2(const float *A, int64_t lda, const float *B, int64_t ldb, const float *dir, int32_t M, int32_t K,
+                 int32_t P, float *work, float *grad, float *loss, void *stream);
+int gh_softmax_ce(const float *Z, int64_t ldz, int32_t M, int32_t n_classes, const int64_t *cls, const int64_t *rows,
+                  float *grad, float *loss, void *stream);
+
 /* Learned exit-plane source (replaces the generator call of GANSourceDefaultGenerator.generator,
  * sources/gansources.py:644-684, and its copy/move of the keys, :686-757).
  * gh_gaussian_bf16: out[r*ld + c] = N(0,1) noise in bf16 for rows first_row .. first_row+n_rows-1

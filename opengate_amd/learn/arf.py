@@ -7,9 +7,9 @@ each energy window (class 0 = not detected), as ARFActor does with a garf networ
 GateARFTrainingDatasetActor.cpp:85-140). Everything on the GPU runs in the library's
 kernels: the detector model transport that labels the training set (gh_run with a
 device phase-space source and per-event crystal energy), the energy blur and windows
-(gh_energy_windows), the network (gh_gemm_bf16, cross-entropy gradient from PyTorch
-tensors), the photon-to-head pairing (gh_spect_pairs) and the image accumulation
-(gh_arf_accumulate / gh_counts_accumulate).
+(gh_energy_windows), the network and its training (learn/mlp.py, gh_softmax_ce), the
+photon-to-head pairing (gh_spect_pairs) and the image accumulation (gh_arf_accumulate /
+gh_counts_accumulate).
 
 The plain counterpart of the learned response transports every (photon, head) pair
 through the voxelised detector model (hexagonal-hole lead collimator over a NaI layer)
@@ -288,27 +288,45 @@ class ArfModel:
             if cw.numel() != self.n_win + 1 or bool((cw < 0).any()):
                 raise ValueError("class_weight needs one non-negative weight per class")
         losses = torch.empty(steps, device=self.dev)
+        # unweighted loss: one kernel (gh_softmax_ce), its sums per 256 rows and step
+        parts = None
+        if cw is None and 0 < batch < 2**31 and self.n_win + 1 <= 16:
+            cls = cls.contiguous()
+            lo, hi = torch.aminmax(cls)
+            if int(lo) < 0 or int(hi) > self.n_win:
+                raise ValueError("classes outside 0..number of windows")
+            parts = torch.empty(steps, (batch + 255) // 256, device=self.dev)
         for it in range(steps):
             self.mlp.lr = lr_min + 0.5 * (lr - lr_min) * (1.0 + math.cos(math.pi * it / max(1, steps)))
             idx = torch.randint(0, N, (batch,), device=self.dev, generator=g)
             xb = X[idx].contiguous()
             z = self.mlp.forward(xb)
-            logp = torch.log_softmax(z, 1)
-            yb = cls[idx]
-            grad = logp.exp()
-            grad[torch.arange(batch, device=self.dev), yb] -= 1.0
-            if cw is None:
-                losses[it] = -logp.gather(1, yb[:, None]).mean()
-                grad /= batch
+            if parts is not None:
+                grad = torch.empty(batch, self.n_win + 1, device=self.dev)
+                rc = self.lib.gh_softmax_ce(_ptr(z), z.stride(0), batch, self.n_win + 1, _ptr(cls), _ptr(idx),
+                                            _ptr(grad), _ptr(parts[it]), _stream())
+                if rc != 0:
+                    raise RuntimeError(f"gh_softmax_ce failed ({rc})")
             else:
-                w = cw[yb]
-                ws = w.sum().clamp_min(1e-30)
-                losses[it] = -(w * logp.gather(1, yb[:, None])[:, 0]).sum() / ws
-                grad *= (w / ws)[:, None]
+                logp = torch.log_softmax(z, 1)
+                yb = cls[idx]
+                grad = logp.exp()
+                grad[torch.arange(batch, device=self.dev), yb] -= 1.0
+                if cw is None:
+                    losses[it] = -logp.gather(1, yb[:, None]).mean()
+                    grad /= batch
+                else:
+                    w = cw[yb]
+                    ws = w.sum().clamp_min(1e-30)
+                    losses[it] = -(w * logp.gather(1, yb[:, None])[:, 0]).sum() / ws
+                    grad *= (w / ws)[:, None]
             dW, db = self.mlp.backward(grad)
             self.mlp.step(dW, db)
             if log_every and (it % log_every == 0 or it == steps - 1):
-                print(f"[arf fit] step {it} loss {float(losses[it]):.5f}", flush=True)
+                now = losses[it] if parts is None else parts[it].sum() / batch
+                print(f"[arf fit] step {it} loss {float(now):.5f}", flush=True)
+        if parts is not None:
+            losses = (parts.sum(1, dtype=torch.float64) / batch).float()
         self.history = losses.cpu().numpy()
         return self.history
 

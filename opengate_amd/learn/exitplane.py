@@ -23,9 +23,9 @@ Representation (what the network is trained on):
 
 Training loss: sliced 2-Wasserstein distance between a generated batch and a data
 batch in the Gaussianised space (random unit projections plus the coordinate axes,
-1-D optimal transport by sorting). The loss and its gradient w.r.t. the generator
-output are computed with PyTorch tensor operations; the gradient is then pushed
-through the network by the hand-written backward GEMMs.
+1-D optimal transport by sorting). The projections, the sorts, the loss and its
+gradient on the projections are one kernel (gh_sliced_w2; PyTorch tensor operations
+beyond 16384 points per batch); the gradient w.r.t. the generator output is then pushed through the network by the hand-written backward passes.
 """
 import ctypes as C
 import math
@@ -176,25 +176,28 @@ class ExitPlaneGenerator:
         gen = torch.Generator(device=self.dev).manual_seed(int(seed))
         eye = torch.eye(N_FEATURES, device=self.dev)
         losses = torch.empty(steps, device=self.dev)
+        # per step and projection: sums of the loss kernel
+        parts = (torch.empty(steps, projections + N_FEATURES, device=self.dev)
+                 if 0 < batch <= self.W2_MAX_ROWS else None)
         X = torch.empty(batch, self.mlp.psizes[0], device=self.dev, dtype=torch.bfloat16)
         for it in range(steps):
             self.mlp.lr = lr_min + 0.5 * (lr - lr_min) * (1.0 + math.cos(math.pi * it / max(1, steps)))
             self.noise(batch, seed * 1_000_003 + 17, first=it * batch, out=X)
-            out = self.mlp.forward(X)
-            o = out.detach().requires_grad_(True)
+            o = self.mlp.forward(X)
             d = G[torch.randint(0, N, (batch,), device=self.dev, generator=gen)]
             th = torch.randn(N_FEATURES, projections, device=self.dev, generator=gen)
             th = torch.cat([th / th.norm(dim=0, keepdim=True), eye], 1)
-            loss = ((torch.sort(o @ th, 0).values - torch.sort(d @ th, 0).values) ** 2).mean()
-            loss.backward()
+            grad = self._sliced_w2(o, d, th, parts, losses, it)
             # Adam divides a gradient by its own size, so over a few steps a difference of one
             # rounding in a bias gradient moves single weights by a tenth of a step: the sums
             # keep their bits, and with them the weights of a seeded fit
-            dW, db = self.mlp.backward(o.grad, tensor_sums=True)
+            dW, db = self.mlp.backward(grad, tensor_sums=True)
             self.mlp.step(dW, db)
-            losses[it] = loss.detach()
             if log_every and (it % log_every == 0 or it == steps - 1):
-                print(f"[exitplane fit] step {it} loss {float(loss):.5f}", flush=True)
+                now = losses[it] if parts is None else parts[it].sum() / (batch * parts.shape[1])
+                print(f"[exitplane fit] step {it} loss {float(now):.5f}", flush=True)
+        if parts is not None:
+            losses = (parts.sum(1, dtype=torch.float64) / (batch * parts.shape[1])).float()
         self.history = losses.cpu().numpy()
         t2 = time.perf_counter()
         # GEMM work of one step: forward, weight gradients, and input gradients below layer 0
@@ -204,6 +207,27 @@ class ExitPlaneGenerator:
                           "step_ms": 1e3 * (t2 - t1) / max(1, steps), "gemm_flop_per_step": flops,
                           "gemm_tflops_over_loop": flops * steps / max(t2 - t1, 1e-9) / 1e12}
         return self.history
+
+    W2_MAX_ROWS = 16384  # GH_SLICED_W2_MAX_ROWS
+
+    def _sliced_w2(self, o, d, th, parts, losses, it):
+        """Gradient w.r.t. the generator outputs o of the sliced distance to the data d on the
+        directions th; the loss goes to parts[it] (sums per direction) or losses[it]."""
+        torch = _torch()
+        if parts is None:
+            o = o.detach().requires_grad_(True)
+            loss = ((torch.sort(o @ th, 0).values - torch.sort(d @ th, 0).values) ** 2).mean()
+            loss.backward()
+            losses[it] = loss.detach()
+            return o.grad
+        th = th.contiguous()
+        g = torch.empty(o.shape[0], th.shape[1], device=self.dev)
+        work = torch.empty(2 * g.numel(), device=self.dev)
+        rc = self.lib.gh_sliced_w2(o.data_ptr(), o.stride(0), d.data_ptr(), d.stride(0), th.data_ptr(), o.shape[0],
+                                   N_FEATURES, th.shape[1], work.data_ptr(), g.data_ptr(), parts[it].data_ptr(), _stream())
+        if rc != 0:
+            raise RuntimeError(f"gh_sliced_w2 failed ({rc})")
+        return g @ th.t()
 
     # ------------------------------------------------------------------ generation
     def generate(self, n, seed, first=0, out=None, chunk=1 << 22, weight=1.0, events=None):
