@@ -109,29 +109,34 @@ class QuantileMap:
 
     @classmethod
     def fit(cls, F, n_knots=4096, g_max=5.5):
-        torch = _torch()
-        N, D = F.shape
-        g = torch.linspace(-g_max, g_max, n_knots, device=F.device, dtype=torch.float64)
-        lev = torch.special.ndtr(g)
-        idx = torch.clamp(torch.round(lev * (N - 1)), 0, N - 1).long()
-        qtab = torch.empty(D, n_knots, device=F.device, dtype=torch.float32)
-        for j in range(D):
-            qtab[j] = torch.sort(F[:, j]).values[idx]
-        return cls(qtab, g_max)
+        return cls.fit_scores(F, n_knots, g_max, scores=False)[0]
 
-    @staticmethod
-    def gaussianize(F):
+    @classmethod
+    def gaussianize(cls, F):
         """Rank-based Gaussian scores of every column: Phi^-1((rank + 1/2)/N)."""
+        return cls.fit_scores(F, tables=False)[1]
+
+    @classmethod
+    def fit_scores(cls, F, n_knots=4096, g_max=5.5, tables=True, scores=True):
+        """(fit(F), gaussianize(F)) with one stable sort per column; None for the one
+        not asked for."""
         torch = _torch()
         N, D = F.shape
-        G = torch.empty_like(F, dtype=torch.float32)
-        ranks = torch.empty(N, device=F.device, dtype=torch.float64)
-        ar = (torch.arange(N, device=F.device, dtype=torch.float64) + 0.5) / N
+        if tables:
+            g = torch.linspace(-g_max, g_max, n_knots, device=F.device, dtype=torch.float64)
+            lev = torch.special.ndtr(g)
+            idx = torch.clamp(torch.round(lev * (N - 1)), 0, N - 1).long()
+            qtab = torch.empty(D, n_knots, device=F.device, dtype=torch.float32)
+        if scores:
+            G = torch.empty_like(F, dtype=torch.float32)
+            by_rank = torch.special.ndtri((torch.arange(N, device=F.device, dtype=torch.float64) + 0.5) / N).float()
         for j in range(D):
-            order = torch.argsort(F[:, j], stable=True)
-            ranks[order] = ar
-            G[:, j] = torch.special.ndtri(ranks).float()
-        return G
+            s = torch.sort(F[:, j], stable=True)
+            if tables:
+                qtab[j] = s.values[idx]
+            if scores:
+                G[s.indices, j] = by_rank
+        return cls(qtab, g_max) if tables else None, G if scores else None
 
 
 class ExitPlaneGenerator:
@@ -167,8 +172,7 @@ class ExitPlaneGenerator:
         torch = _torch()
         t0 = time.perf_counter()
         F = exit_features(phsp, self.focal, self.plane_z, self.dev)
-        self.qmap = QuantileMap.fit(F, n_knots=n_knots)
-        G = QuantileMap.gaussianize(F)
+        self.qmap, G = QuantileMap.fit_scores(F, n_knots=n_knots)
         del F
         N = G.shape[0]
         torch.cuda.synchronize()
