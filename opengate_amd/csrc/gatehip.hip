@@ -84,22 +84,35 @@ struct SimDev {
   uint64_t n_hist, first_hist;
 };
 
+// Work queue: chunk c belongs to queue c mod QUEUES, each queue with a counter of its own.
+// Atomics on one address run one after the other (12 ns each, measured: the first chunks of
+// 4096 waves took 50 us, and 64-history chunks capped a run at 5e9 histories/s), on 8 addresses
+// in different lines 8 at a time. A wave's first chunk follows from its place in the launch
+// without an atomic; the counters start behind those. (With a contiguous eighth of the chunks
+// per queue a batched launch worked on 8 simulations at once and was 8-30 % slower.)
+constexpr int QUEUES = 8, QUEUE_STRIDE = 32;  // 256 bytes from counter to counter
+
 struct Launch {
   const SimDev *sims;
   int n_sims;
   const uint64_t *chunk_offsets;  // [n_sims+1] prefix sum of chunks per sim
   uint64_t total_chunks;
   uint32_t chunk;
-  unsigned long long *next_chunk;
+  unsigned long long *queue;      // [QUEUES * QUEUE_STRIDE] chunks taken from each queue
+  uint32_t queues_empty;          // bit q: the first chunks of its waves are all that queue q has
   uint64_t seed;
   int max_iter;   // step-phase iterations (2 tentative steps each) between slow phases
   int slow_min;   // lanes waiting for slow work that end a step phase
   int refill_min; // dead lanes that trigger a refill (<= slow_min)
   int scatter_tries; // Compton / Rayleigh sampler tries per slow phase before a photon waits
   Phys P;
-  unsigned long long *counters;   // [12]
-  double *energies;               // [4]
+  unsigned long long *partial;    // [workgroup][RESULTS] counters and (as bits) energy sums
 };
+
+// chunks of queue q
+__host__ __device__ inline uint64_t queue_chunks(uint64_t total_chunks, int q) {
+  return (total_chunks + (uint64_t)(QUEUES - 1 - q)) / QUEUES;
+}
 
 // --------------------------------------------------------------------- wave helpers
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
@@ -229,6 +242,7 @@ struct SqCache {
 enum { C_HIST = 0, C_STEPS, C_DEPOSITS, C_COMPTON, C_RAYLEIGH, C_PHOTO, C_ESCAPED, C_WORLD, C_CUT,
        C_EVICT, C_RECORDED, C_REJ, N_COUNTERS };
 enum { E_DEP = 0, E_OUT, E_ESC, E_WORLD, N_ENERGIES };
+constexpr int RESULTS = N_COUNTERS + N_ENERGIES;  // 16 words per workgroup
 
 struct LaneStats {
   uint32_t steps, rej;
@@ -681,6 +695,7 @@ transport_kernel(Launch L) {
   const float *mu_tab = T.mu;
   const float *maj_tab = T.maj;
   __shared__ unsigned long long s_cnt[N_COUNTERS];
+  __shared__ uint32_t s_empty;  // work queues seen empty by a wave of this workgroup
   // energy tallies of the statistics: one FP64 slot per lane and category, so that the
   // lanes of a wave never add to one LDS address at once (64 same-address FP64 atomics
   // serialise in the LDS unit and hold up the table reads of every wave of the CU)
@@ -708,6 +723,7 @@ transport_kernel(Launch L) {
     }
   }
   if (threadIdx.x < N_COUNTERS) s_cnt[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0) s_empty = L.queues_empty;
   for (int k = 0; k < N_ENERGIES; ++k) s_en[k * BLOCK + threadIdx.x] = 0.0;
   __syncthreads();
   LaneStats st;
@@ -740,8 +756,11 @@ transport_kernel(Launch L) {
 
   // wave-uniform work state
   int cur_sim = 0;
-  uint64_t cur_next = 0, cur_end = 0;
+  uint32_t cur_next = 0, cur_end = 0;  // histories of cur_sim (below 2^32)
   bool have_work = true;
+  // the queue this wave takes chunks from (-1: not started). Its first chunks go to the waves
+  // of its workgroups in turn, one wave of every workgroup first (few chunks: over all CUs)
+  int queue = -1;
   uint32_t qn = 0;               // photons in this wave's birth queue
   const uint32_t slow_min = (uint32_t)L.slow_min;
   const uint32_t refill_min = (uint32_t)L.refill_min;
@@ -796,22 +815,37 @@ transport_kernel(Launch L) {
   // still need transport go into the wave's queue (empty when the pass starts).
   auto birth_pass = [&]() {
     while (have_work && cur_next >= cur_end) {
-      unsigned long long c = 0;
-      if (lane_id() == 0) c = atomicAdd(L.next_chunk, 1ull);
-      c = __shfl(c, 0, 64);
-      if (c >= L.total_chunks) { have_work = false; break; }
+      uint64_t c;
+      if (queue < 0) {
+        queue = (int)(blockIdx.x % QUEUES);
+        const uint32_t blocks = (gridDim.x - (uint32_t)queue + QUEUES - 1) / QUEUES;
+        c = (threadIdx.x >> 6) * blocks + blockIdx.x / QUEUES;
+      } else {
+        // this wave's queue, or the next that no wave of the workgroup has seen empty
+        const uint32_t left = ~*(volatile uint32_t *)&s_empty & ((1u << QUEUES) - 1u);
+        if (left == 0u) { have_work = false; break; }
+        queue = (queue + __ffs((int)((left | left << QUEUES) >> queue)) - 1) % QUEUES;
+        unsigned long long got = 0;
+        if (lane_id() == 0) {
+          got = atomicAdd(L.queue + queue * QUEUE_STRIDE, 1ull);
+          if (got >= queue_chunks(L.total_chunks, queue)) atomicOr(&s_empty, 1u << queue);
+        }
+        c = got;
+      }
+      c = __shfl(c, 0, 64) * QUEUES + (uint64_t)queue;
+      if (c >= L.total_chunks) continue;
       int s = 0;
       while (s + 1 < L.n_sims && L.chunk_offsets[s + 1] <= c) ++s;
       cur_sim = s;
       const uint64_t local = (c - L.chunk_offsets[s]) * (uint64_t)L.chunk;
-      cur_next = local;
+      cur_next = (uint32_t)local;
       const uint64_t e = local + L.chunk;
       const uint64_t nh = sim(s).n_hist;
-      cur_end = e < nh ? e : nh;
+      cur_end = (uint32_t)(e < nh ? e : nh);
     }
     if (!have_work) return;
-    const uint64_t left = cur_end - cur_next;
-    const uint32_t avail = (uint32_t)(left < 64u ? left : 64u);
+    const uint32_t left = cur_end - cur_next;
+    const uint32_t avail = left < 64u ? left : 64u;
     const uint32_t lane = lane_id();
     const SimDev &s = sim(cur_sim);
     int bm = M_DEAD;
@@ -819,7 +853,7 @@ transport_kernel(Launch L) {
     b.x = b.y = b.z = b.u = b.v = b.w = b.E = b.wt = 0.0f;
     uint32_t bh = 0, bc3 = 0;
     if (lane < avail) {
-      bh = (uint32_t)(cur_next + lane);
+      bh = cur_next + lane;
       Rng g;
       rng_init(g, L.seed, s.first_hist + bh, (uint32_t)(BATCHED ? cur_sim : 0));
       sample_source(s, BATCHED ? SpecTab{s.e_val, s.e_width, s.e_cdf, s.e_guide} : spec0, g, bh, b);
@@ -1138,6 +1172,8 @@ transport_kernel(Launch L) {
   }
 
   // ------------------------------------------------------------- counters
+  // per workgroup to memory, summed by finish_kernel (16 same-line FP64 atomics per wave took up
+  // to 200 us at the end of a launch)
   {
     const uint64_t steps = wave_sum<uint64_t>((uint64_t)st.steps);
     const uint64_t rej = wave_sum<uint64_t>((uint64_t)st.rej);
@@ -1145,14 +1181,47 @@ transport_kernel(Launch L) {
       atomicAdd(s_cnt + C_STEPS, (unsigned long long)steps);
       atomicAdd(s_cnt + C_REJ, (unsigned long long)rej);
     }
+    double *own = s_en + (threadIdx.x & ~63u);
+    for (int k = 0; k < N_ENERGIES; ++k) {
+      const double v = wave_sum<double>(own[k * BLOCK + lane_id()]);
+      if (lane_id() == 0) own[k * BLOCK] = v;
+    }
   }
   __syncthreads();
-  if (threadIdx.x < N_COUNTERS && s_cnt[threadIdx.x])
-    atomicAdd(L.counters + threadIdx.x, s_cnt[threadIdx.x]);
-  for (int k = 0; k < N_ENERGIES; ++k) {
-    const double v = wave_sum<double>(s_en[k * BLOCK + threadIdx.x]);
-    if (lane_id() == 0 && v != 0.0) unsafeAtomicAdd(L.energies + k, v);
+  unsigned long long *out = L.partial + (size_t)blockIdx.x * RESULTS;
+  if (threadIdx.x < N_COUNTERS) out[threadIdx.x] = s_cnt[threadIdx.x];
+  if (threadIdx.x < N_ENERGIES) {
+    double v = 0.0;
+    for (uint32_t w = 0; w < blockDim.x; w += 64) v += s_en[threadIdx.x * BLOCK + w];
+    out[N_COUNTERS + threadIdx.x] = (unsigned long long)__double_as_longlong(v);
   }
+}
+
+// sums of the workgroups' results, in a fixed order; out: host memory
+__global__ void __launch_bounds__(1024) finish_kernel(const unsigned long long *__restrict__ partial, int n,
+                                                      unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long s_u[1024];
+  __shared__ double s_d[1024];
+  const int k = threadIdx.x % RESULTS, g = threadIdx.x / RESULTS;  // 64 rows at a time
+  unsigned long long u = 0;
+  double d = 0.0;
+  for (int r = g; r < n; r += 1024 / RESULTS) {
+    const unsigned long long v = partial[(size_t)r * RESULTS + k];
+    if (k < N_COUNTERS) u += v;
+    else d += __longlong_as_double((long long)v);
+  }
+  s_u[threadIdx.x] = u;
+  s_d[threadIdx.x] = d;
+  __syncthreads();
+  for (int o = 512; o >= RESULTS; o >>= 1) {
+    if ((int)threadIdx.x < o) {
+      s_u[threadIdx.x] += s_u[threadIdx.x + o];
+      s_d[threadIdx.x] += s_d[threadIdx.x + o];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < RESULTS)
+    out[k] = k < N_COUNTERS ? s_u[k] : (unsigned long long)__double_as_longlong(s_d[k]);
 }
 
 // ---------------------------------------------------------------------- phsp check
@@ -1248,12 +1317,12 @@ struct gh_ctx {
   // simulations
   std::vector<SimHost> sims;
   // run scratch
-  SimDev *d_sims = nullptr;
-  uint64_t *d_chunk_off = nullptr;
-  unsigned long long *d_next = nullptr;
-  unsigned long long *d_counters = nullptr;
-  double *d_energies = nullptr;
-  size_t d_sims_cap = 0;
+  // one upload per run, from pinned memory: queue counters, simulation descriptors, chunk offsets
+  unsigned char *h_up = nullptr, *d_up = nullptr;
+  size_t up_cap = 0;
+  unsigned long long *d_partial = nullptr;  // per workgroup results
+  size_t partial_cap = 0;
+  unsigned long long *h_result = nullptr;   // their sums, pinned, written by finish_kernel
   gh_launch last_launch{};
   int last_stage = 0;
 };
@@ -1540,11 +1609,10 @@ void gh_destroy(gh_ctx *ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto &s : ctx->sims) { free_all(s.owned); free_all(s.source_owned); }
   free_all(ctx->phys_owned);
-  if (ctx->d_sims) (void)hipFree(ctx->d_sims);
-  if (ctx->d_chunk_off) (void)hipFree(ctx->d_chunk_off);
-  if (ctx->d_next) (void)hipFree(ctx->d_next);
-  if (ctx->d_counters) (void)hipFree(ctx->d_counters);
-  if (ctx->d_energies) (void)hipFree(ctx->d_energies);
+  if (ctx->d_up) (void)hipFree(ctx->d_up);
+  if (ctx->h_up) (void)hipHostFree(ctx->h_up);
+  if (ctx->d_partial) (void)hipFree(ctx->d_partial);
+  if (ctx->h_result) (void)hipHostFree(ctx->h_result);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -1909,32 +1977,14 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     }
     devs[s] = h.dev;
   }
-  if (!ctx->d_sims || ctx->d_sims_cap < (size_t)ns) {
-    if (ctx->d_sims) { (void)hipFree(ctx->d_sims); ctx->d_sims = nullptr; }
-    if (ctx->d_chunk_off) { (void)hipFree(ctx->d_chunk_off); ctx->d_chunk_off = nullptr; }
-    HIPCHK(hipMalloc(&ctx->d_sims, ns * sizeof(SimDev)));
-    HIPCHK(hipMalloc(&ctx->d_chunk_off, (ns + 1) * sizeof(uint64_t)));
-    ctx->d_sims_cap = ns;
-  }
-  if (!ctx->d_next) {
-    HIPCHK(hipMalloc(&ctx->d_next, sizeof(unsigned long long)));
-    HIPCHK(hipMalloc(&ctx->d_counters, 12 * sizeof(unsigned long long)));
-    HIPCHK(hipMalloc(&ctx->d_energies, 4 * sizeof(double)));
-  }
-
   Launch L;
-  L.sims = ctx->d_sims;
   L.n_sims = ns;
-  L.chunk_offsets = ctx->d_chunk_off;
-  L.next_chunk = ctx->d_next;
   L.seed = seed;
   L.max_iter = lp.refill_interval;
   L.slow_min = std::max(1, std::min(64, lp.slow_min));
   L.refill_min = std::max(1, std::min(L.slow_min, lp.refill_min));
   L.scatter_tries = lp.scatter_tries;
   L.P = ctx->P;
-  L.counters = ctx->d_counters;
-  L.energies = ctx->d_energies;
   // staging level and block: all tables in LDS shared by one 1024-thread workgroup per CU
   // when they fit, else mu + majorant in LDS with 256-thread workgroups, else none. The
   // budgets leave room for the kernel's static LDS (per-lane energy slots, birth queues and
@@ -2000,25 +2050,58 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, lp.block, shmem));
     lp.grid = std::max(1, ctx->n_cu) * std::max(1, per_cu);
   }
-  // work-queue chunk: automatic = about four chunks per wave of the launch (64 to 4096
-  // histories, a multiple of 64), so that a short run still spreads over every wave; which
-  // wave runs a history does not change its result
+  // work-queue chunk: automatic. Up to 128 histories per wave, one chunk per wave, which it gets
+  // without an atomic, and all waves have work (1000 histories in chunks of 64: 122 us, of 4: 79;
+  // 20000: 141 and 115). Beyond, chunks of 128, and of 256 from 4096 histories per wave on: the
+  // smaller the chunk the shorter the last waves' tail, the more atomics (ct256, 1e7 histories:
+  // 64 2089 us, 128 2063, 256 2112, 1024 2297; 1e8: 64 18711, 128 18524, 256 18437, 4096 19251).
+  // Which wave runs a history does not change its result
   if (lp.chunk <= 0) {
     uint64_t total = 0;
     for (int s = 0; s < ns; ++s) total += n_histories[s];
     const uint64_t waves = (uint64_t)lp.grid * (uint64_t)(lp.block / 64);
-    uint64_t c = total / std::max<uint64_t>(1, 4 * waves);
-    c = std::min<uint64_t>(4096, std::max<uint64_t>(64, c & ~(uint64_t)63));
-    lp.chunk = (int32_t)c;
+    const uint64_t share = (total + waves - 1) / waves;
+    lp.chunk = share <= 128 ? (int32_t)std::max<uint64_t>(4, (share + 3) & ~(uint64_t)3) : (share < 4096 ? 128 : 256);
   }
   for (int s = 0; s < ns; ++s) offs[s + 1] = offs[s] + (n_histories[s] + lp.chunk - 1) / lp.chunk;
   L.total_chunks = offs[ns];
   L.chunk = (uint32_t)lp.chunk;
-  HIPCHK(hipMemcpyAsync(ctx->d_sims, devs.data(), ns * sizeof(SimDev), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemcpyAsync(ctx->d_chunk_off, offs.data(), (ns + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemsetAsync(ctx->d_next, 0, sizeof(unsigned long long), ctx->stream));
-  HIPCHK(hipMemsetAsync(ctx->d_counters, 0, 12 * sizeof(unsigned long long), ctx->stream));
-  HIPCHK(hipMemsetAsync(ctx->d_energies, 0, 4 * sizeof(double), ctx->stream));
+  const size_t queue_bytes = QUEUES * QUEUE_STRIDE * sizeof(unsigned long long);
+  const size_t sims_bytes = (ns * sizeof(SimDev) + 15) & ~(size_t)15;
+  const size_t up_bytes = queue_bytes + sims_bytes + (ns + 1) * sizeof(uint64_t);
+  if (ctx->up_cap < up_bytes) {
+    if (ctx->d_up) { (void)hipFree(ctx->d_up); ctx->d_up = nullptr; }
+    if (ctx->h_up) { (void)hipHostFree(ctx->h_up); ctx->h_up = nullptr; }
+    ctx->up_cap = 0;
+    HIPCHK(hipMalloc(&ctx->d_up, up_bytes));
+    HIPCHK(hipHostMalloc(&ctx->h_up, up_bytes, hipHostMallocDefault));
+    ctx->up_cap = up_bytes;
+  }
+  if (ctx->partial_cap < (size_t)lp.grid) {
+    if (ctx->d_partial) { (void)hipFree(ctx->d_partial); ctx->d_partial = nullptr; }
+    ctx->partial_cap = 0;
+    HIPCHK(hipMalloc(&ctx->d_partial, (size_t)lp.grid * RESULTS * sizeof(unsigned long long)));
+    ctx->partial_cap = (size_t)lp.grid;
+  }
+  if (!ctx->h_result) HIPCHK(hipHostMalloc(&ctx->h_result, RESULTS * sizeof(unsigned long long), hipHostMallocDefault));
+  {
+    // a queue's counter starts behind the first chunks of its waves
+    unsigned long long *q = (unsigned long long *)ctx->h_up;
+    std::memset(q, 0, queue_bytes);
+    L.queues_empty = 0;
+    for (int k = 0; k < QUEUES; ++k) {
+      const uint64_t blocks = lp.grid > k ? ((uint64_t)lp.grid - k + QUEUES - 1) / QUEUES : 0;
+      q[k * QUEUE_STRIDE] = blocks * (uint64_t)(lp.block / 64);
+      if (q[k * QUEUE_STRIDE] >= queue_chunks(L.total_chunks, k)) L.queues_empty |= 1u << k;
+    }
+    std::memcpy(ctx->h_up + queue_bytes, devs.data(), ns * sizeof(SimDev));
+    std::memcpy(ctx->h_up + queue_bytes + sims_bytes, offs.data(), (ns + 1) * sizeof(uint64_t));
+  }
+  L.queue = (unsigned long long *)ctx->d_up;
+  L.sims = (const SimDev *)(ctx->d_up + queue_bytes);
+  L.chunk_offsets = (const uint64_t *)(ctx->d_up + queue_bytes + sims_bytes);
+  L.partial = ctx->d_partial;
+  HIPCHK(hipMemcpyAsync(ctx->d_up, ctx->h_up, up_bytes, hipMemcpyHostToDevice, ctx->stream));
   ctx->last_launch = lp;
   ctx->last_stage = stage;
   HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
@@ -2028,11 +2111,16 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     HIPCHK(hipGetLastError());
   }
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
-  unsigned long long c[12];
-  double e[4];
-  HIPCHK(hipMemcpyAsync(c, ctx->d_counters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(e, ctx->d_energies, sizeof(e), hipMemcpyDeviceToHost, ctx->stream));
+  std::memset(ctx->h_result, 0, RESULTS * sizeof(unsigned long long));
+  if (L.total_chunks > 0) {
+    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->d_partial, (int)lp.grid, ctx->h_result);
+    HIPCHK(hipGetLastError());
+  }
   HIPCHK(hipStreamSynchronize(ctx->stream));
+  unsigned long long c[N_COUNTERS];
+  double e[N_ENERGIES];
+  std::memcpy(c, ctx->h_result, sizeof(c));
+  std::memcpy(e, ctx->h_result + N_COUNTERS, sizeof(e));
   float ms = 0.0f;
   HIPCHK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   if (out) {
