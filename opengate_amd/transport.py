@@ -451,15 +451,15 @@ class GpuEngine:
     def get_tally(self, sim_id=0):
         _, _, tal = self.sims[sim_id]
         nz_ny_nx = tuple(reversed([int(x) for x in tal.size]))
-        res = {"edep": np.zeros(nz_ny_nx)}
+        res = {"edep": np.empty(nz_ny_nx)}
         if tal.edep2:
-            res["edep2"] = np.zeros(nz_ny_nx)
+            res["edep2"] = np.empty(nz_ny_nx)
         if tal.dose:
-            res["dose"] = np.zeros(nz_ny_nx)
+            res["dose"] = np.empty(nz_ny_nx)
         if tal.dose2:
-            res["dose2"] = np.zeros(nz_ny_nx)
+            res["dose2"] = np.empty(nz_ny_nx)
         if tal.counts:
-            res["counts"] = np.zeros(nz_ny_nx)
+            res["counts"] = np.empty(nz_ny_nx)
         self._check(self.lib.gh_get_tally(self.ctx, int(sim_id), A.dptr(res["edep"]), A.dptr(res.get("edep2")),
                                           A.dptr(res.get("dose")), A.dptr(res.get("dose2")),
                                           A.dptr(res.get("counts"))), "gh_get_tally")
