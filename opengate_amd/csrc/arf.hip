@@ -12,7 +12,7 @@
 // x' = axial (z), y' = tangential, z' = -n_k (towards the source) the direction is
 // d' = (d_z, d.e_k, -c); theta = acos(c), phi = atan2(d'_y, d'_x)
 // (GateARFTrainingDatasetActor.cpp:99-107 with the plane normal as third axis).
-// Every (photon, head) pair is written with a wave-aggregated atomic slot: the NN input
+// Every (photon, head) pair is written to a slot that its workgroup reserved: the NN input
 // row (bf16: E, theta, phi scaled by norm[]), the pixel index (head*ny + iy)*nx + ix,
 // the weight, and optionally the photon in the frame of a detector model whose hexagonal
 // hole lattice (pitch, first lattice vector along x') has a lattice point at
@@ -38,6 +38,8 @@
 #include "../../include/gatehip.h"
 #include "gh_device.h"
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
 namespace {
 
 using namespace gh;
@@ -60,13 +62,29 @@ __device__ __forceinline__ uint32_t mbcnt(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// Pairs found by a workgroup wait in LDS until PAIR_CAP could overflow, and then take their slots
+// with one atomic: all slots come from one counter, which serves an atomic every 12 ns wherever it
+// comes from. (One atomic for each wave and 64 tested heads was that bound: 10^6 photons on 128 heads,
+// 500 us; so 46.) The waiting pairs hold what the geometry needs anyway; angles and
+// rows are computed when they are written, by full waves.
+constexpr int PAIR_CAP = 768;
+
+template <bool DET>
 __global__ void __launch_bounds__(256) spect_pairs_kernel(const float *__restrict__ x, const float *__restrict__ y,
                                                           const float *__restrict__ z, const float *__restrict__ u,
                                                           const float *__restrict__ v, const float *__restrict__ w,
                                                           const float *__restrict__ E, const float *__restrict__ wt,
                                                           int64_t n, gh_spect_desc D, const float *__restrict__ cs,
                                                           PairOut o) {
-  __shared__ int owner_lane[4][64];
+  enum { PX, PY, PZ, DU, DV, DW, EN, WT, CAND_FIELDS };
+  enum { C, DY, QW, QE, QWT, HU, HZ, PAIR_FIELDS };
+  __shared__ float s_cand[CAND_FIELDS][256];
+  __shared__ int s_k0[256];
+  __shared__ float s_pair[DET ? PAIR_FIELDS : HU][PAIR_CAP];
+  __shared__ int s_pix[PAIR_CAP];
+  __shared__ int s_n[2][2][4];  // of candidates and of pairs, by wave; two in turn: one barrier a round
+  __shared__ unsigned long long s_slot;
+  const int wave = (int)(threadIdx.x >> 6);
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const float two_pi = 6.28318530717958647692f;
   const float dalpha = two_pi / (float)D.n_proj;
@@ -78,52 +96,110 @@ __global__ void __launch_bounds__(256) spect_pairs_kernel(const float *__restric
   const int jlo = all_heads ? 0 : -margin, jhi = all_heads ? D.n_proj - 1 : margin;
   const float half_w = 0.5f * (float)D.nx * D.spacing[0], half_h = 0.5f * (float)D.ny * D.spacing[1];
   const float a2x = 0.5f * D.pitch, a2y = 0.86602540378443865f * D.pitch;
-  // every lane of a wave runs the same rounds so that slots are assigned with wave-wide
-  // ballots
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride) {
+  int waiting = 0;  // the same in every thread, as every bound of the loops below
+
+  // position of this lane's item among those of the workgroup; every thread gets their number
+  auto place = [&](int (&counts)[4], bool mine, int &total) {
+    const uint64_t m = __ballot(mine);
+    if (lane_id() == 0) counts[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0;
+    total = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q < wave) before += counts[q];
+      total += counts[q];
+    }
+    return before + (int)mbcnt(m);
+  };
+
+  auto write_out = [&]() {
+    __syncthreads();
+    if (threadIdx.x == 0) s_slot = atomicAdd(o.count, (unsigned long long)waiting);
+    __syncthreads();
+    for (int p = (int)threadIdx.x; p < waiting; p += 256) {
+      const uint64_t slot = s_slot + (uint64_t)p;
+      if ((int64_t)slot >= o.capacity) break;
+      const float c = s_pair[C][p], dy = s_pair[DY][p], qw = s_pair[QW][p], qe = s_pair[QE][p];
+      const float theta = acosf(fminf(c, 1.0f));
+      const float phi = atan2f(dy, qw);
+      if (o.x16) {
+        bf16x8 row = {};
+        row[0] = (__bf16)fmaf(qe, D.norm[0], D.norm[1]);
+        row[1] = (__bf16)fmaf(theta, D.norm[2], D.norm[3]);
+        row[2] = (__bf16)fmaf(phi, D.norm[4], D.norm[5]);
+        __builtin_memcpy(o.x16 + slot * 8, &row, sizeof(row));
+      }
+      if (o.tp) { o.tp[2 * slot] = theta; o.tp[2 * slot + 1] = phi; }
+      o.pix[slot] = s_pix[p];
+      o.wgt[slot] = s_pair[QWT][p];
+      if constexpr (DET) {
+        // head frame: x' axial (hz), y' tangential (hu); reduce to the lattice cell
+        float rx = s_pair[HZ][p], ry = s_pair[HU][p];
+        if (D.pitch > 0.0f) {
+          const float jj = floorf(ry / a2y);
+          ry = fmaf(-jj, a2y, ry);
+          rx = fmaf(-jj, a2x, rx);
+          const float ii = floorf(rx / D.pitch);
+          rx = fmaf(-ii, D.pitch, rx);
+        }
+        o.det[0][slot] = D.patch_origin[0] + rx;
+        o.det[1][slot] = D.patch_origin[1] + ry;
+        o.det[2][slot] = D.patch_origin[2];
+        o.det[3][slot] = qw;
+        o.det[4][slot] = dy;
+        o.det[5][slot] = -c;
+        o.det[6][slot] = qe;
+        o.det[7][slot] = s_pair[QWT][p];
+      }
+    }
+    __syncthreads();
+    waiting = 0;
+  };
+
+  int turn = 0, round = 0;
+  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride, turn ^= 1) {
     const int64_t i = base + threadIdx.x;
-    const bool valid = i < n;
-    float px = 0.f, py = 0.f, pz = 0.f, du = 0.f, dv = 0.f, dw = 1.f, e = 0.f, ww = 0.f;
+    float du = 0.f, dv = 0.f, dw = 1.f, ww = 0.f;
     bool cand = false;
-    int k0 = 0;
-    if (valid) {
-      px = x[i] - D.center[0]; py = y[i] - D.center[1]; pz = z[i] - D.center[2];
-      du = u[i]; dv = v[i]; dw = w[i]; e = E[i]; ww = wt[i];
+    if (i < n) {
+      du = u[i]; dv = v[i]; dw = w[i]; ww = wt[i];
       // only directions within theta_max of the transverse plane can reach a head
       cand = fabsf(dw) < sin_max && ww > 0.0f;
-      if (cand && !all_heads) {
+    }
+    int n_cand;
+    const int at = place(s_n[0][turn], cand, n_cand);
+    if (cand) {
+      int k0 = 0;
+      if (!all_heads) {
         const float beta = atan2f(dv, du) - D.angle0;
         k0 = (int)floorf(beta / dalpha + 0.5f);
       }
+      s_k0[at] = k0;
+      s_cand[PX][at] = x[i] - D.center[0];
+      s_cand[PY][at] = y[i] - D.center[1];
+      s_cand[PZ][at] = z[i] - D.center[2];
+      s_cand[DU][at] = du; s_cand[DV][at] = dv; s_cand[DW][at] = dw;
+      s_cand[EN][at] = E[i];
+      s_cand[WT][at] = ww;
     }
-    // expand the (candidate photon, head) work items of the wave over its 64 lanes: lane
-    // l of round r takes item 64 r + l = (candidate ci, head offset j); the candidate's
-    // data comes from its owner lane by a cross-lane read
-    const uint64_t cmask = __ballot(cand);
-    const int n_cand = __popcll(cmask);
-    if (n_cand == 0) continue;
-    if (cand) owner_lane[threadIdx.x >> 6][mbcnt(cmask)] = (int)lane_id();
-    __builtin_amdgcn_wave_barrier();
+    __syncthreads();
+    // the (candidate photon, head) items of the workgroup over its 256 threads
     const int width = jhi - jlo + 1;
-    const int n_items = n_cand * width;
-    for (int it0 = 0; it0 < n_items; it0 += 64) {
-      const int item = it0 + (int)lane_id();
-      const bool act = item < n_items;
-      const int ci = act ? item / width : 0;
-      const int j = jlo + (act ? item - ci * width : 0);
-      const int src = owner_lane[threadIdx.x >> 6][ci];
-      const float qx = __shfl(px, src, 64), qy = __shfl(py, src, 64), qz = __shfl(pz, src, 64);
-      const float qu = __shfl(du, src, 64), qv = __shfl(dv, src, 64), qw = __shfl(dw, src, 64);
-      const float qe = __shfl(e, src, 64), qwt = __shfl(ww, src, 64);
-      const int qk0 = __shfl(k0, src, 64);
+    const int64_t n_items = (int64_t)n_cand * width;
+    for (int64_t it0 = 0; it0 < n_items; it0 += 256, round ^= 1) {
+      if (waiting > PAIR_CAP - 256) write_out();
+      const int64_t item = it0 + (int64_t)threadIdx.x;
       bool hit = false;
       int32_t pixel = 0;
+      int ci = 0;
       float c = 0.f, dy = 0.f, hu = 0.f, hz = 0.f;
-      int k = 0;
-      if (act) {
-        const float px = qx, py = qy, pz = qz, du = qu, dv = qv, dw = qw;
-        const int k0 = qk0;
-        k = ((k0 + j) % D.n_proj + D.n_proj) % D.n_proj;
+      if (item < n_items) {
+        ci = n_items <= INT32_MAX ? (int)((uint32_t)item / (uint32_t)width) : (int)(item / width);
+        const int j = jlo + (int)(item - (int64_t)ci * width);
+        const float px = s_cand[PX][ci], py = s_cand[PY][ci], pz = s_cand[PZ][ci];
+        const float du = s_cand[DU][ci], dv = s_cand[DV][ci], dw = s_cand[DW][ci];
+        const int k = ((s_k0[ci] + j) % D.n_proj + D.n_proj) % D.n_proj;
         const float ca = cs[2 * k], sa = cs[2 * k + 1];
         c = fmaf(du, ca, dv * sa);
         if (c > D.cos_theta_max) {
@@ -145,49 +221,24 @@ __global__ void __launch_bounds__(256) spect_pairs_kernel(const float *__restric
           }
         }
       }
-      const uint64_t m = __ballot(hit);
-      if (m == 0) continue;
-      const uint32_t leader = __ffsll((unsigned long long)m) - 1;
-      unsigned long long slot0 = 0;
-      if (lane_id() == leader) slot0 = atomicAdd(o.count, (unsigned long long)__popcll(m));
-      slot0 = __shfl(slot0, leader, 64);
-      if (!hit) continue;
-      const uint64_t slot = slot0 + mbcnt(m);
-      if ((int64_t)slot >= o.capacity) continue;
-      const float theta = acosf(fminf(c, 1.0f));
-      const float phi = atan2f(dy, qw);
-      if (o.x16) {
-        __bf16 *row = o.x16 + slot * 8;
-        row[0] = (__bf16)fmaf(qe, D.norm[0], D.norm[1]);
-        row[1] = (__bf16)fmaf(theta, D.norm[2], D.norm[3]);
-        row[2] = (__bf16)fmaf(phi, D.norm[4], D.norm[5]);
-#pragma unroll
-        for (int q = 3; q < 8; ++q) row[q] = (__bf16)0.0f;
-      }
-      if (o.tp) { o.tp[2 * slot] = theta; o.tp[2 * slot + 1] = phi; }
-      o.pix[slot] = pixel;
-      o.wgt[slot] = qwt;
-      if (o.det[0]) {
-        // head frame: x' axial (hz), y' tangential (hu); reduce to the lattice cell
-        float rx = hz, ry = hu;
-        if (D.pitch > 0.0f) {
-          const float jj = floorf(ry / a2y);
-          ry = fmaf(-jj, a2y, ry);
-          rx = fmaf(-jj, a2x, rx);
-          const float ii = floorf(rx / D.pitch);
-          rx = fmaf(-ii, D.pitch, rx);
+      int found;
+      const int p = waiting + place(s_n[1][round], hit, found);
+      if (hit) {
+        s_pix[p] = pixel;
+        s_pair[C][p] = c;
+        s_pair[DY][p] = dy;
+        s_pair[QW][p] = s_cand[DW][ci];
+        s_pair[QE][p] = s_cand[EN][ci];
+        s_pair[QWT][p] = s_cand[WT][ci];
+        if constexpr (DET) {
+          s_pair[HU][p] = hu;
+          s_pair[HZ][p] = hz;
         }
-        o.det[0][slot] = D.patch_origin[0] + rx;
-        o.det[1][slot] = D.patch_origin[1] + ry;
-        o.det[2][slot] = D.patch_origin[2];
-        o.det[3][slot] = qw;
-        o.det[4][slot] = dy;
-        o.det[5][slot] = -c;
-        o.det[6][slot] = qe;
-        o.det[7][slot] = qwt;
       }
+      waiting += found;
     }
   }
+  if (waiting) write_out();
 }
 
 struct Windows {
@@ -274,11 +325,11 @@ __global__ void __launch_bounds__(256) counts_accumulate_kernel(const int32_t *_
   }
 }
 
-int grid_for(int64_t n) {
+int grid_for(int64_t n, int per_cu = 16) {
   int dev = 0, n_cu = 256;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
   const int64_t want = (n + 255) / 256;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)n_cu * 16));
+  return (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)n_cu * per_cu));
 }
 
 }  // namespace
@@ -302,8 +353,14 @@ extern "C" int gh_spect_pairs(const float *const rec[8], int64_t n, const gh_spe
     }
   }
   if (n == 0) return GH_OK;
-  hipLaunchKernelGGL(spect_pairs_kernel, dim3(grid_for(n)), dim3(256), 0, (hipStream_t)stream, rec[0], rec[1], rec[2],
-                     rec[3], rec[4], rec[5], rec[6], rec[7], n, *det, angle_cs, o);
+  // as many workgroups as the chip holds at once: each then writes its pairs out few times
+  const dim3 grid(grid_for(n, 5));
+  if (det_rec)
+    hipLaunchKernelGGL(spect_pairs_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, rec[0], rec[1], rec[2],
+                       rec[3], rec[4], rec[5], rec[6], rec[7], n, *det, angle_cs, o);
+  else
+    hipLaunchKernelGGL(spect_pairs_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, rec[0], rec[1], rec[2],
+                       rec[3], rec[4], rec[5], rec[6], rec[7], n, *det, angle_cs, o);
   return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
 }
 
