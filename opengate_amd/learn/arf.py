@@ -344,15 +344,24 @@ class ArfModel:
         if bufs is None and not fused:
             bufs = [torch.empty(c, max(self.mlp.psizes[1:-1]), device=self.dev, dtype=torch.bfloat16)
                     for _ in range(2)]
+        n_pix = img.numel() // self.n_win
+        need = C.c_int64(0)
+        if self.lib.gh_arf_accumulate_workspace(c, self.n_win, n_pix, int(img2 is not None), C.byref(need)) != 0:
+            raise RuntimeError("gh_arf_accumulate_workspace failed")
+        work = torch.empty(need.value, device=self.dev, dtype=torch.uint8) if need.value else None
         for s in range(0, m, c):
             k = min(c, m - s)
             if fused:
                 self.mlp.infer_fused(buf.x16[s:s + k], Z[:k])
             else:
                 self.mlp.infer(buf.x16[s:s + k], Z[:k], bufs)
-            rc = self.lib.gh_arf_accumulate(_ptr(Z), Z.shape[1], k, C.c_void_p(buf.pix.data_ptr() + 4 * s),
-                                            C.c_void_p(buf.wgt.data_ptr() + 4 * s), self.n_win, plane, _ptr(img),
-                                            _ptr(img2), _stream())
+            pairs = (_ptr(Z), Z.shape[1], k, C.c_void_p(buf.pix.data_ptr() + 4 * s),
+                     C.c_void_p(buf.wgt.data_ptr() + 4 * s), self.n_win, plane)
+            if work is not None:
+                rc = self.lib.gh_arf_accumulate_binned(*pairs, n_pix, _ptr(img), _ptr(img2), _ptr(work), work.numel(),
+                                                       _stream())
+            else:
+                rc = self.lib.gh_arf_accumulate(*pairs, _ptr(img), _ptr(img2), _stream())
             if rc != 0:
                 raise RuntimeError(f"gh_arf_accumulate failed ({rc})")
 

@@ -78,10 +78,56 @@ def test_pairs_beyond_capacity_are_counted():
     cs = torch.from_numpy(h.angle_table()).cuda()
     p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
     dev = [torch.from_numpy(a).cuda() for a in rec]
-    rc = A.load_library().gh_spect_pairs((A.FP * 8)(*[C.cast(p(a), A.FP) for a in dev]), 20000, C.byref(h.desc()), p(cs),
-                                         cap, p(buf.x16), p(buf.pix), p(buf.wgt), None, C.c_void_p(), p(buf.count), None)
+    photons = (A.FP * 8)(*[C.cast(p(a), A.FP) for a in dev])
+    rc = A.load_library().gh_spect_pairs(photons, 20000, C.byref(h.desc()), p(cs), cap, p(buf.x16), p(buf.pix),
+                                         p(buf.wgt), None, C.c_void_p(), p(buf.count), None)
     assert rc == 0
     torch.cuda.synchronize()
     assert int(buf.count) == cnt
     pix = buf.pix.cpu().numpy()
     assert np.all(pix[:cap] >= 0) and np.all(pix[cap:] == -1)
+
+
+# one pair; sorting workgroups of 4096 pairs; bins of 4096 pixels; every record size; one hot pixel
+@pytest.mark.parametrize("m,heads,plane,n_win,squared,hot", [(1, 1, 1, 1, True, False), (4096, 1, 4096, 3, True, False),
+                                                             (4097, 3, 4097, 4, False, False),
+                                                             (70001, 16, 768, 3, True, True),
+                                                             (100003, 128, 16384, 3, True, False),
+                                                             (100000, 7, 65536, 8, True, False),
+                                                             (90000, 5, 999, 7, False, True)])
+def test_binned_accumulation(m, heads, plane, n_win, squared, hot):
+    import ctypes as C
+
+    import torch
+
+    from opengate_amd import _abi as A
+
+    print(f"[gpu case] binned accumulation m={m} heads={heads} plane={plane} windows={n_win}", flush=True)
+    lib, g = A.load_library(), np.random.default_rng(m)
+    n_pix = heads * plane
+    logits = g.normal(size=(m, n_win + 2)).astype(np.float32)
+    pix = g.integers(0, n_pix, m).astype(np.int32)
+    if hot:
+        pix[: m // 2] = n_pix - 1
+    wgt = g.uniform(0.5, 1.5, m).astype(np.float32)
+    L, P, W = (torch.from_numpy(a).cuda() for a in (logits, pix, wgt))
+    p = lambda t: C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p()  # noqa: E731
+    bins = (n_pix + 4095) // 4096
+    work = torch.full((4 * ((3 * bins + 4) // 4 * 4) + 16 * ((n_win + 4) // 4) * m,), 255, dtype=torch.uint8,
+                      device="cuda")
+    need = C.c_int64(-1)
+    assert lib.gh_arf_accumulate_workspace(m, n_win, n_pix, int(squared), C.byref(need)) == 0
+    assert need.value in (0, work.numel())
+    got, want = [], []
+    for out in (got, want):
+        out += [torch.full((heads * n_win * plane,), 0.25, dtype=torch.float64, device="cuda") for _ in range(2)]
+    i2 = lambda out: out[1] if squared else None  # noqa: E731
+    args = (p(L), n_win + 2, m, p(P), p(W), n_win, plane)
+    assert lib.gh_arf_accumulate_binned(*args, n_pix, p(got[0]), p(i2(got)), p(work), work.numel() - 1, None) != 0
+    for _ in range(2):  # the workspace needs no clearing
+        assert lib.gh_arf_accumulate_binned(*args, n_pix, p(got[0]), p(i2(got)), p(work), work.numel(), None) == 0
+        assert lib.gh_arf_accumulate(*args, p(want[0]), p(i2(want)), None) == 0
+    for a, b in zip(got, want):  # the same terms, FP64 sums in another order
+        np.testing.assert_allclose(a.cpu().numpy(), b.cpu().numpy(), rtol=1e-11, atol=0)
+    ref = 0.25 + 2 * R.accumulate_arf(logits, pix, wgt, n_win, plane, heads)
+    np.testing.assert_allclose(got[0].cpu().numpy(), ref.reshape(-1), rtol=1e-5)
