@@ -276,20 +276,24 @@ __global__ void __launch_bounds__(256) softmax_ce_kernel(const float *__restrict
   if (i < M) {
     const float *z = Z + i * ldz;
     const int y = (int)cls[rows ? rows[i] : i];
-    float v[CE_MAX_CLASSES], mx = -INFINITY, s = 0.0f;
+    float v[CE_MAX_CLASSES], e[CE_MAX_CLASSES], mx = -INFINITY;
 #pragma unroll
     for (int k = 0; k < CE_MAX_CLASSES; ++k)
       if (k < C) { v[k] = z[k]; mx = fmaxf(mx, v[k]); }
 #pragma unroll
-    for (int k = 0; k < CE_MAX_CLASSES; ++k)
-      if (k < C) s += expf(v[k] - mx);
-    const float lse = logf(s);
+    for (int k = 0; k < CE_MAX_CLASSES; ++k) e[k] = k < C ? expf(v[k] - mx) : 0.0f;
+    // halves added onto halves, as a reduction over lanes adds them
+#pragma unroll
+    for (int o = CE_MAX_CLASSES / 2; o > 0; o >>= 1)
+#pragma unroll
+      for (int k = 0; k < o; ++k) e[k] += e[k + o];
+    const float lse = logf(e[0]), scale = 1.0f / (float)M;
 #pragma unroll
     for (int k = 0; k < CE_MAX_CLASSES; ++k)
       if (k < C) {
         const float lp = (v[k] - mx) - lse;
         if (k == y) l = -lp;
-        grad[(int64_t)i * C + k] = (expf(lp) - (k == y ? 1.0f : 0.0f)) / (float)M;
+        grad[(int64_t)i * C + k] = (expf(lp) - (k == y ? 1.0f : 0.0f)) * scale;
       }
   }
 #pragma unroll

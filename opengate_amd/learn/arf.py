@@ -320,7 +320,7 @@ class ArfModel:
                     ws = w.sum().clamp_min(1e-30)
                     losses[it] = -(w * logp.gather(1, yb[:, None])[:, 0]).sum() / ws
                     grad *= (w / ws)[:, None]
-            dW, db = self.mlp.backward(grad)
+            dW, db = self.mlp.backward(grad, tensor_sums=True)
             self.mlp.step(dW, db)
             if log_every and (it % log_every == 0 or it == steps - 1):
                 now = losses[it] if parts is None else parts[it].sum() / batch
