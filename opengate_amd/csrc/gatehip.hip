@@ -74,6 +74,8 @@ struct SimDev {
   int vox_nx, vox_ny;
   float vox_s[3];
   // tally
+  // with a TLE tally (edep, edep2) and (dose, dose2) lie side by side for each voxel where both
+  // are kept: then edep2 = edep + 1 and the step from voxel to voxel is two; otherwise one
   double *edep, *edep2, *dose, *dose2, *counts;
   int aligned, tnx, tny, tnz;
   float tcorner[3], tinv[3], ts[3];  // tally grid (aligned: the phantom grid, corner 0)
@@ -114,7 +116,10 @@ struct Launch {
   int scatter_tries; // Compton / Rayleigh sampler tries per slow phase before a photon waits
   Phys P;
   unsigned long long *partial;    // [workgroup][RESULTS] counters and (as bits) energy sums
+  int pair_ofs;                   // word of the dynamic LDS where the waves' pair buffers start, -1: none
 };
+
+constexpr int PAIR_WORDS = 2 * 64;  // of a wave's buffer of (value, voxel) entries
 
 // chunks of queue q
 __host__ __device__ inline uint64_t queue_chunks(uint64_t total_chunks, int q) {
@@ -256,6 +261,8 @@ struct LaneStats {
   unsigned long long *cnt;  // LDS [N_COUNTERS]
   double *en;               // LDS [N_ENERGIES][BLOCK]: this lane's column
   int stride;               // BLOCK
+  uint32_t *pair;           // LDS: this wave's PAIR_WORDS, used if paired
+  bool paired;              // uniform over the launch
   __device__ __forceinline__ void inc(int k) {
     const uint64_t m = __ballot(1);
     if (__lane_id() == (uint32_t)(__ffsll((unsigned long long)m) - 1))
@@ -273,29 +280,71 @@ __device__ __forceinline__ TallyOut tally_out(const SimDev &s) {
   return TallyOut{s.edep, s.edep2, s.counts, s.dose, s.dose2};
 }
 
+// Adds v and v^2 of every active lane to the two adjacent values of its voxel. The memory side
+// takes 23.6 atomic requests per ns over the chip, from 4096 voxels to 16 million alike, and
+// neighbouring lanes on one 64-byte piece make one request: so the lanes hand their (voxel, v)
+// round through LDS and each pair of lanes adds the two values of one voxel (two planes, or one
+// lane adding both: 11.8 voxels per ns; so 23.3, and 19 with 4 active lanes of 64). The kerma
+// estimator deposits at almost every step and is bound by these requests (2e7 histories on
+// Schneider's materials 8.56 -> 6.34 ms). The analog tallies are not (a third of the requests a
+// step), and there the exchange costs more than it saves (ct256 of 5e8 histories 91 -> 100 ms,
+// a batch of 8 5.5 -> 6.0): they keep planes and two atomics a lane.
+__device__ __forceinline__ void pair_add(double *base, int vox, float v, const LaneStats &st) {
+  if (st.paired) {
+    const uint64_t m = __ballot(1);
+    const uint32_t k = (uint32_t)__popcll(m), r = mbcnt(m);
+    volatile uint32_t *w = st.pair;
+    w[r] = __float_as_uint(v);
+    w[64 + r] = (uint32_t)vox;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      const uint32_t item = q * k + r, e = item >> 1;
+      double d = (double)__uint_as_float(w[e]);
+      d = (item & 1u) ? d * d : d;
+      gatomic_add(base + 2 * (int64_t)w[64 + e] + (item & 1u), d);
+    }
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    gatomic_add(base + 2 * (int64_t)vox, (double)v);
+    gatomic_add(base + 2 * (int64_t)vox + 1, (double)v * (double)v);
+  }
+}
+
+template <bool TLE>
 __device__ __forceinline__ void flush_slot(const TallyOut &o, int vox, float sum, float dsum, uint32_t cnt,
                                            LaneStats &st) {
-  gatomic_add(o.edep + vox, (double)sum);
-  if (o.edep2) gatomic_add(o.edep2 + vox, (double)sum * (double)sum);
+  if (TLE && o.edep2) {
+    pair_add(o.edep, vox, sum, st);
+  } else {
+    gatomic_add(o.edep + vox, (double)sum);
+    if (o.edep2) gatomic_add(o.edep2 + vox, (double)sum * (double)sum);
+  }
   if (o.counts) gatomic_add(o.counts + vox, (double)cnt);
-  if (o.dose) gatomic_add(o.dose + vox, (double)dsum);
-  if (o.dose2) gatomic_add(o.dose2 + vox, (double)dsum * (double)dsum);
+  if (TLE && o.dose && o.dose2) {
+    pair_add(o.dose, vox, dsum, st);
+  } else {
+    if (o.dose) gatomic_add(o.dose + vox, (double)dsum);
+    if (o.dose2) gatomic_add(o.dose2 + vox, (double)dsum * (double)dsum);
+  }
   st.inc(C_DEPOSITS);
   st.add_e(E_DEP, (double)sum);
 }
 
+template <bool TLE>
 __device__ __forceinline__ void sq_flush_all(const SimDev &s, SqCache &c, LaneStats &st) {
   const TallyOut o = tally_out(s);
-  if (c.n > 0) flush_slot(o, c.v0, c.s0, c.d0, c.c0, st);
-  if (c.n > 1) flush_slot(o, c.v1, c.s1, c.d1, c.c1, st);
-  if (c.n > 2) flush_slot(o, c.v2, c.s2, c.d2, c.c2, st);
-  if (c.n > 3) flush_slot(o, c.v3, c.s3, c.d3, c.c3, st);
+  if (c.n > 0) flush_slot<TLE>(o, c.v0, c.s0, c.d0, c.c0, st);
+  if (c.n > 1) flush_slot<TLE>(o, c.v1, c.s1, c.d1, c.c1, st);
+  if (c.n > 2) flush_slot<TLE>(o, c.v2, c.s2, c.d2, c.c2, st);
+  if (c.n > 3) flush_slot<TLE>(o, c.v3, c.s3, c.d3, c.c3, st);
   c.n = 0;
 }
 
 // Adds deposit x (dose dx) of the current history to tally voxel tv. A history's
 // deposits in the same voxel are summed in FP32 before the squared value is formed;
 // with more than 4 distinct voxels the oldest slot is flushed (counted as an eviction).
+template <bool TLE>
 __device__ __forceinline__ void deposit(const SimDev &s, SqCache &c, int tv, float x, float dx,
                                         LaneStats &st) {
   if (tv < 0) { st.add_e(E_OUT, (double)x); return; }
@@ -313,7 +362,7 @@ __device__ __forceinline__ void deposit(const SimDev &s, SqCache &c, int tv, flo
     return;
   }
   if (c.n == 4) {
-    flush_slot(tally_out(s), c.v0, c.s0, c.d0, c.c0, st);
+    flush_slot<TLE>(tally_out(s), c.v0, c.s0, c.d0, c.c0, st);
     c.v0 = c.v1; c.s0 = c.s1; c.d0 = c.d1; c.c0 = c.c1;
     c.v1 = c.v2; c.s1 = c.s2; c.d1 = c.d2; c.c1 = c.c2;
     c.v2 = c.v3; c.s2 = c.s3; c.d2 = c.d3; c.c2 = c.c3;
@@ -735,6 +784,8 @@ transport_kernel(Launch L) {
   __syncthreads();
   LaneStats st;
   st.steps = 0u; st.rej = 0u; st.cnt = s_cnt; st.en = s_en + threadIdx.x; st.stride = BLOCK;
+  st.paired = TLE && L.pair_ofs >= 0;
+  st.pair = (uint32_t *)lds + (st.paired ? L.pair_ofs : 0) + (threadIdx.x >> 6) * PAIR_WORDS;
   const uint32_t qbase = threadIdx.x & ~63u;
 
   Hot hot;
@@ -876,7 +927,7 @@ transport_kernel(Launch L) {
           const int tv = tally_voxel(s, b.x, b.y, b.z);
           if (lab >= s.det_label_min && s.det_label_min >= 0) ev = x;
           if (s.event_edep) s.event_edep[bh] = ev;
-          if (tv >= 0) flush_slot(tally_out(s), tv, x, x * P.inv_rho[lab], 1u, st);
+          if (tv >= 0) flush_slot<TLE>(tally_out(s), tv, x, x * P.inv_rho[lab], 1u, st);
           else st.add_e(E_OUT, (double)x);
         } else {
           if (s.event_edep) s.event_edep[bh] = ev;
@@ -994,7 +1045,7 @@ transport_kernel(Launch L) {
                 const SimDev &s0 = sim(0);
                 const MatRow mr = shared_rows ? mat_tab[lab] : MatRow{1.0f, lab};
                 const float x = (ph.E * ph.wt) * (lerp_node_scaled(P.muen + mr.row * NB1, mr.rho, ec) * ec.inv_maj);
-                deposit(s0, sq, tally_voxel(s0, ph.x, ph.y, ph.z), x, x * P.inv_rho[lab], st);
+                deposit<TLE>(s0, sq, tally_voxel(s0, ph.x, ph.y, ph.z), x, x * P.inv_rho[lab], st);
               }
               // u01 x majorant < mu, with u01 = odd22(ba) 2^-22 and the 2^-22 folded into
               // maj22: the same single rounding of the same exact product
@@ -1158,11 +1209,11 @@ transport_kernel(Launch L) {
           const float irho = P.inv_rho[clab];
           const bool det = s.det_label_min >= 0 && clab >= s.det_label_min;
           if (x_dep != 0.0f) {
-            deposit(s, sq, tv, x_dep, x_dep * irho, st);
+            deposit<TLE>(s, sq, tv, x_dep, x_dep * irho, st);
             if (det) ev_edep += x_dep;
           }
           if (x_cut != 0.0f) {
-            deposit(s, sq, tv, x_cut, x_cut * irho, st);
+            deposit<TLE>(s, sq, tv, x_cut, x_cut * irho, st);
             if (det) ev_edep += x_cut;
           }
         }
@@ -1172,7 +1223,7 @@ transport_kernel(Launch L) {
         // the event record goes first: a read of the descriptor placed after the flush's
         // atomics would wait for them
         if (s.event_edep) s.event_edep[history_of(rng) - s.first_hist] = ev_edep;
-        sq_flush_all(s, sq, st);
+        sq_flush_all<TLE>(s, sq, st);
         mode = M_DEAD;
       }
     }
@@ -1302,6 +1353,26 @@ struct SimHost {
   int det = -1;
   uint64_t event_cap = 0;
   uint64_t event_n = 0;  // histories of the last run (valid per-history detector energies)
+
+  // first value, values per voxel and place of image k (edep, edep2, dose, dose2, counts)
+  struct Image {
+    double *p;
+    int step;
+  };
+  Image image(int k) const {
+    double *p[5] = {dev.edep, dev.edep2, dev.dose, dev.dose2, dev.counts};
+    const int e = dev.tle && dev.edep2 ? 2 : 1, d = dev.tle && dev.dose && dev.dose2 ? 2 : 1;
+    return {p[k], k < 2 ? e : (k < 4 ? d : 1)};
+  }
+  // the allocations behind the images: first value and number of values
+  std::vector<std::pair<double *, size_t>> tallies() const {
+    std::vector<std::pair<double *, size_t>> v;
+    for (int k = 0; k < 5; ++k) {
+      const Image im = image(k);
+      if (im.p && (im.step == 1 || k == 0 || k == 2)) v.push_back({im.p, n_tally * im.step});
+    }
+    return v;
+  }
 };
 
 }  // namespace
@@ -1358,11 +1429,27 @@ void free_all(std::vector<void *> &v) {
 #define MADV_POPULATE_WRITE 23  // Linux 5.14
 #endif
 
+// n doubles, `step` apart on the device
 struct HostCopy {
-  void *dst;
-  const void *src;
-  size_t bytes;
+  double *dst;
+  const double *src;
+  size_t n;
+  int step;
 };
+
+// one of two interleaved images, into memory that the device can write (pinned: over the link)
+__global__ void __launch_bounds__(256) take_image_kernel(const double *__restrict__ src, int64_t n, int step,
+                                                         double *__restrict__ dst) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[step * i];
+}
+
+hipError_t device_copy(void *dst, const HostCopy &c, hipMemcpyKind kind, hipStream_t stream) {
+  if (c.step == 1) return hipMemcpyAsync(dst, c.src, c.n * sizeof(double), kind, stream);
+  const unsigned grid = (unsigned)std::min<size_t>((c.n + 255) / 256, 1024);
+  hipLaunchKernelGGL(take_image_kernel, dim3(grid), dim3(256), 0, stream, c.src, (int64_t)c.n, c.step, (double *)dst);
+  return hipGetLastError();
+}
 
 // Device to pageable host memory. The runtime's own copy stages through pinned memory with one
 // host thread, which the first touch of a fresh destination's pages holds at 9.5 GB/s (128 MB in
@@ -1442,7 +1529,7 @@ std::vector<StagingBlock> staging_take(int device, size_t n) {
   }
   while (v.size() < n) {
     StagingBlock b;
-    if (hipEventCreateWithFlags(&b.done, hipEventDisableTiming) != hipSuccess ||
+    if (hipEventCreateWithFlags(&b.done, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess ||
         hipHostMalloc(&b.host, RING_BLOCK, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       staging_free(b);
@@ -1467,27 +1554,27 @@ void staging_give(int device, std::vector<StagingBlock> &v) {
 }
 
 int copy_to_host(gh_ctx *ctx, const std::vector<HostCopy> &parts) {
-  std::vector<HostCopy> blocks, direct;
+  std::vector<HostCopy> blocks, direct, via_device;
   size_t total = 0;
   for (const HostCopy &c : parts) {
     hipPointerAttribute_t at{};
     const bool known = hipPointerGetAttributes(&at, c.dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
     if (!known) (void)hipGetLastError();
     if (known) {  // pinned, managed or device memory needs no staging
-      direct.push_back(c);
+      (c.step == 1 || at.type == hipMemoryTypeHost ? direct : via_device).push_back(c);
       continue;
     }
-    total += c.bytes;
-    for (size_t o = 0; o < c.bytes; o += RING_BLOCK)
-      blocks.push_back({(char *)c.dst + o, (const char *)c.src + o, std::min(RING_BLOCK, c.bytes - o)});
+    total += c.n * sizeof(double);
+    constexpr size_t N = RING_BLOCK / sizeof(double);
+    for (size_t o = 0; o < c.n; o += N) blocks.push_back({c.dst + o, c.src + o * c.step, std::min(N, c.n - o), c.step});
   }
   const size_t cpus = std::max(1u, std::thread::hardware_concurrency());
   size_t threads = std::min({total / RING_BYTES_PER_THREAD, (size_t)RING_THREADS, cpus});
   threads = blocks.empty() ? 0 : std::max<size_t>(threads, 1);
   std::vector<StagingBlock> ring = staging_take(ctx->device, 2 * threads);
   threads = std::min(threads, ring.size() / 2);
-  if (threads == 0) {  // no pinned memory to be had: the runtime's own staging
-    direct = parts;
+  if (threads == 0) {  // nothing to stage, or no pinned memory to be had: the runtime's own staging
+    for (const HostCopy &c : blocks) (c.step == 1 ? direct : via_device).push_back(c);
   } else {
     // thread k takes blocks k, k + threads, ...; its slot s is ring block 2 k + s
     std::atomic<int> failed{0};
@@ -1495,16 +1582,16 @@ int copy_to_host(gh_ctx *ctx, const std::vector<HostCopy> &parts) {
       hipError_t e = hipSetDevice(ctx->device);
       auto fetch = [&](size_t b, int s) {
         if (e == hipSuccess)
-          e = hipMemcpyAsync(ring[2 * k + s].host, blocks[b].src, blocks[b].bytes, hipMemcpyDeviceToHost, ctx->stream);
+          e = device_copy(ring[2 * k + s].host, blocks[b], hipMemcpyDeviceToHost, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ring[2 * k + s].done, ctx->stream);
       };
       int s = 0;
       if (k < blocks.size()) fetch(k, 0);
       for (size_t b = k; b < blocks.size() && e == hipSuccess; b += threads, s ^= 1) {
         if (b + threads < blocks.size()) fetch(b + threads, s ^ 1);
-        map_pages(blocks[b].dst, blocks[b].bytes);
+        map_pages(blocks[b].dst, blocks[b].n * sizeof(double));
         if (e == hipSuccess) e = hipEventSynchronize(ring[2 * k + s].done);
-        if (e == hipSuccess) std::memcpy(blocks[b].dst, ring[2 * k + s].host, blocks[b].bytes);
+        if (e == hipSuccess) std::memcpy(blocks[b].dst, ring[2 * k + s].host, blocks[b].n * sizeof(double));
       }
       if (e != hipSuccess) failed.store((int)e);
     };
@@ -1525,7 +1612,16 @@ int copy_to_host(gh_ctx *ctx, const std::vector<HostCopy> &parts) {
     }
   }
   staging_give(ctx->device, ring);
-  for (const HostCopy &c : direct) HIPCHK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDefault, ctx->stream));
+  for (const HostCopy &c : direct) HIPCHK(device_copy(c.dst, c, hipMemcpyDefault, ctx->stream));
+  for (const HostCopy &c : via_device) {
+    void *image = nullptr;
+    HIPCHK(hipMalloc(&image, c.n * sizeof(double)));
+    hipError_t e = device_copy(image, c, hipMemcpyDefault, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(c.dst, image, c.n * sizeof(double), hipMemcpyDefault, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    (void)hipFree(image);
+    HIPCHK(e);
+  }
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return GH_OK;
 }
@@ -2042,20 +2138,22 @@ int gh_add_simulation(gh_ctx *ctx, const gh_phantom_desc *ph, const gh_source_de
     d.tinv[i] = 1.0f / d.ts[i];
   }
   double *dd;
-  if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
-  d.edep = dd;
-  if (tal->flags & GH_TALLY_EDEP2) {
-    if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
-    d.edep2 = dd;
-  }
-  if (tal->flags & GH_TALLY_DOSE) {
-    if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
-    d.dose = dd;
-  }
-  if (tal->flags & GH_TALLY_DOSE2) {
-    if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
-    d.dose2 = dd;
-  }
+  // an image and its image of squares; side by side for the kerma estimator
+  auto images = [&](bool one, bool two, double **a, double **a2) -> int {
+    const bool pair = one && two && (tal->flags & GH_TALLY_TLE);
+    if (one || pair) {
+      if ((rc = dev_upload<double>(ctx, nullptr, (pair ? 2 : 1) * ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
+      *a = dd;
+      if (pair) *a2 = dd + 1;
+    }
+    if (two && !pair) {
+      if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
+      *a2 = dd;
+    }
+    return GH_OK;
+  };
+  if ((rc = images(true, (tal->flags & GH_TALLY_EDEP2) != 0, &d.edep, &d.edep2))) return rc;
+  if ((rc = images((tal->flags & GH_TALLY_DOSE) != 0, (tal->flags & GH_TALLY_DOSE2) != 0, &d.dose, &d.dose2))) return rc;
   if (tal->flags & GH_TALLY_COUNTS) {
     if ((rc = dev_upload<double>(ctx, nullptr, ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
     d.counts = dd;
@@ -2102,10 +2200,7 @@ int gh_reset_tally(gh_ctx *ctx, int32_t sim_id) {
   if (sim_id < 0 || sim_id >= (int32_t)ctx->sims.size()) FAIL(GH_EINVAL, "gh_reset_tally: bad sim id");
   HIPCHK(hipSetDevice(ctx->device));
   SimHost &h = ctx->sims[sim_id];
-  const size_t bytes = h.n_tally * sizeof(double);
-  double *arrs[5] = {h.dev.edep, h.dev.edep2, h.dev.dose, h.dev.dose2, h.dev.counts};
-  for (double *a : arrs)
-    if (a) HIPCHK(hipMemsetAsync(a, 0, bytes, ctx->stream));
+  for (const auto &t : h.tallies()) HIPCHK(hipMemsetAsync(t.first, 0, t.second * sizeof(double), ctx->stream));
   if (h.dev.rec_count) HIPCHK(hipMemsetAsync(h.dev.rec_count, 0, sizeof(unsigned long long), ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return GH_OK;
@@ -2230,6 +2325,15 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
              : (stage == 1 ? GH_PICK(true, 1, 256, false) : GH_PICK(true, 0, 256, false));
   }
 #undef GH_PICK
+  // buffers of the paired tally adds behind the tables, where the budget leaves room for them
+  L.pair_ofs = -1;
+  if (tle) {
+    const size_t at = (shmem + 15) & ~(size_t)15, end = at + (lp.block / 64) * PAIR_WORDS * sizeof(uint32_t);
+    if (end <= (big ? budget_big : budget_small)) {
+      L.pair_ofs = (int)(at / sizeof(uint32_t));
+      shmem = end;
+    }
+  }
   if (shmem > 64 * 1024) HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
   if (lp.grid <= 0) {
     int per_cu = 0;
@@ -2325,18 +2429,22 @@ int gh_autotune(gh_ctx *ctx, const uint64_t *n_trial, uint64_t seed, gh_launch *
   if (!n_trial || !best) FAIL(GH_EINVAL, "gh_autotune: null argument");
   HIPCHK(hipSetDevice(ctx->device));
   // snapshot every tally so that trial histories leave no trace
-  std::vector<std::pair<double *, double *>> saved;
+  struct Saved {
+    double *tally;
+    void *copy;
+    size_t bytes;
+  };
+  std::vector<Saved> saved;
   std::vector<unsigned long long> rec_counts;
   std::vector<void *> tmp;
   for (auto &h : ctx->sims) {
-    double *arrs[5] = {h.dev.edep, h.dev.edep2, h.dev.dose, h.dev.dose2, h.dev.counts};
-    for (double *a : arrs) {
-      if (!a) continue;
+    for (const auto &t : h.tallies()) {
+      const size_t bytes = t.second * sizeof(double);
       void *b = nullptr;
-      HIPCHK(hipMalloc(&b, h.n_tally * sizeof(double)));
+      HIPCHK(hipMalloc(&b, bytes));
       tmp.push_back(b);
-      HIPCHK(hipMemcpyAsync(b, a, h.n_tally * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-      saved.push_back({a, (double *)b});
+      HIPCHK(hipMemcpyAsync(b, t.first, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+      saved.push_back({t.first, b, bytes});
     }
     unsigned long long rc = 0;
     if (h.dev.rec_count) HIPCHK(hipMemcpy(&rc, h.dev.rec_count, sizeof(rc), hipMemcpyDeviceToHost));
@@ -2367,13 +2475,8 @@ int gh_autotune(gh_ctx *ctx, const uint64_t *n_trial, uint64_t seed, gh_launch *
       best_lp.chunk = 0;  // automatic: sized by the production run's own history count
     }
   }
-  for (auto &pr : saved) {
-    size_t n = 0;
-    for (auto &h : ctx->sims)
-      for (double *a : {h.dev.edep, h.dev.edep2, h.dev.dose, h.dev.dose2, h.dev.counts})
-        if (a == pr.first) n = h.n_tally;
-    (void)hipMemcpyAsync(pr.first, pr.second, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream);
-  }
+  for (const Saved &t : saved)
+    (void)hipMemcpyAsync(t.tally, t.copy, t.bytes, hipMemcpyDeviceToDevice, ctx->stream);
   for (size_t s = 0; s < ctx->sims.size(); ++s)
     if (ctx->sims[s].dev.rec_count)
       (void)hipMemcpyAsync(ctx->sims[s].dev.rec_count, &rec_counts[s], sizeof(unsigned long long),
@@ -2394,15 +2497,14 @@ int gh_get_tally(gh_ctx *ctx, int32_t sim_id, double *edep, double *edep2, doubl
   if (sim_id < 0 || sim_id >= (int32_t)ctx->sims.size()) FAIL(GH_EINVAL, "gh_get_tally: bad sim id");
   HIPCHK(hipSetDevice(ctx->device));
   SimHost &h = ctx->sims[sim_id];
-  const size_t bytes = h.n_tally * sizeof(double);
   double *dst[5] = {edep, edep2, dose, dose2, counts};
-  double *src[5] = {h.dev.edep, h.dev.edep2, h.dev.dose, h.dev.dose2, h.dev.counts};
   const char *names[5] = {"edep", "edep2", "dose", "dose2", "counts"};
   std::vector<HostCopy> parts;
   for (int k = 0; k < 5; ++k) {
     if (!dst[k]) continue;
-    if (!src[k]) FAIL(GH_ESTATE, std::string("gh_get_tally: ") + names[k] + " not enabled");
-    parts.push_back({dst[k], src[k], bytes});
+    const SimHost::Image im = h.image(k);
+    if (!im.p) FAIL(GH_ESTATE, std::string("gh_get_tally: ") + names[k] + " not enabled");
+    parts.push_back({dst[k], im.p, h.n_tally, im.step});
   }
   return copy_to_host(ctx, parts);
 }
