@@ -366,6 +366,14 @@ int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_layers, int3
                                int32_t np, const void *const *w, const void *const *Y, const float *G, int64_t ldg,
                                float *dW, float *db, float *const *G32, void *ws, int64_t ws_bytes, void *stream);
 
+/* Column sums of `count` (at most 8) FP32 matrices of M rows in one fixed order of additions, that
+ * of PyTorch's sum over the rows: G[k] M x n[k] with row pitch ld[k]; out[k]: n_pad[k] sums (a
+ * power of two from 8 to 256, at least n[k]; those behind n[k] are zero). work: 256 sum(n_pad)
+ * floats. M at most GH_COLUMN_SUMS_MAX_ROWS. */
+#define GH_COLUMN_SUMS_MAX_ROWS 65536
+int gh_column_sums(const float *const *G, const int64_t *ld, const int32_t *n, const int32_t *n_pad, int32_t count,
+                   int64_t M, float *const *out, float *work, int64_t work_floats, void *stream);
+
 /* Losses of the training loops with their gradients (no counterpart in the reference's source, as
  * for gh_adam_step).
  * gh_sliced_w2: A (pitch lda) and B (pitch ldb): M points of K <= 8 values, M at most

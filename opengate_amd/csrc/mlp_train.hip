@@ -368,6 +368,104 @@ int launch_backward(const float *G, int64_t ldg, int64_t M, const BackArgs &a, h
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
+// ------------------------------------------------------------------ column sums
+// Sums over the rows of several FP32 matrices, in one fixed order of additions: workgroup c of
+// `ctas` and its thread row y of `by` add the rows s + S i, s = c by + y and S = by ctas, in
+// four running sums (i mod 4), then those, then the thread rows by halves, then the workgroups
+// (y, y + by, ... and the thread rows by halves again). This is the order in which PyTorch sums
+// the columns of a matrix of these widths, found by comparing bits over 1..70000 rows
+// (tests/test_gpu_column_sums.py holds it): fits divide by the size of nearly cancelled sums in
+// their first steps, so another order gives other weights. Its calls, one a layer, took 125 us for
+// 5 x 16384 x 256 and 32 for 3 x 5003 x 128; these two launches 23 and 15, the first bound by
+// reading 84 MB from behind the L2 (5.2 TB/s), the second by the one workgroup of its last layer.
+struct ColSum {
+  const float *g;
+  int64_t ld;
+  int n, n_pad;    // columns, and with the zero columns behind them
+  int by, ctas;
+  float *part;     // [ctas][n_pad]
+  float *out;      // n_pad
+};
+struct ColSums {
+  ColSum m[MAXL];
+  int64_t M;
+};
+constexpr int COLSUM_THREADS = 128;
+
+// thread rows and workgroups of a matrix of M x n rows
+void column_plan(int64_t M, int n_pad, int &by, int &ctas) {
+  by = COLSUM_THREADS / (n_pad / 4);
+  if (M < 16 * by && M < 256) by = 1;
+  const int64_t rows = (M + by - 1) / by, want = (rows + 15) / 16;
+  ctas = rows < 256 ? 1 : (want <= 128 ? (int)want : (want <= 256 ? 128 : 256));
+}
+
+__device__ __forceinline__ float4 add4(float4 a, float4 b) {
+  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
+__global__ void __launch_bounds__(COLSUM_THREADS) column_part_kernel(ColSums C) {
+  const ColSum m = C.m[blockIdx.y];
+  if ((int)blockIdx.x >= m.ctas) return;
+  __shared__ float4 s_v[COLSUM_THREADS];
+  const int groups = m.n_pad / 4, t = threadIdx.x, col = (t % groups) * 4, y = t / groups;
+  float4 a[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  auto rows = [&](auto load) {
+    const int64_t S = (int64_t)m.by * m.ctas;
+    int64_t r = (int64_t)blockIdx.x * m.by + y;
+#pragma unroll 4
+    for (; r + 3 * S < C.M; r += 4 * S) {
+      float4 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = load(m.g + (r + k * S) * m.ld + col);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[k] = add4(a[k], v[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (r + k * S < C.M) a[k] = add4(a[k], load(m.g + (r + k * S) * m.ld + col));
+  };
+  if (y < m.by && col < m.n) {
+    if ((m.ld & 3) == 0 && col + 4 <= m.n && ((uintptr_t)m.g & 15) == 0) {
+      rows([](const float *p) { return *(const float4 *)p; });
+    } else {
+      const int left = m.n - col;
+      rows([left](const float *p) {
+        return make_float4(p[0], left > 1 ? p[1] : 0.0f, left > 2 ? p[2] : 0.0f, left > 3 ? p[3] : 0.0f);
+      });
+    }
+  }
+  float4 v = add4(add4(add4(a[0], a[1]), a[2]), a[3]);
+  for (int o = m.by / 2; o > 0; o >>= 1) {
+    s_v[t] = v;
+    __syncthreads();
+    if (y < o) v = add4(v, s_v[t + o * groups]);
+    __syncthreads();
+  }
+  if (y == 0) *(float4 *)((m.ctas > 1 ? m.part + (int64_t)blockIdx.x * m.n_pad : m.out) + col) = v;
+}
+
+__global__ void __launch_bounds__(COLSUM_THREADS) column_total_kernel(ColSums C) {
+  const ColSum m = C.m[blockIdx.y];
+  const int cols = COLSUM_THREADS / m.by, t = threadIdx.x, col = (int)blockIdx.x * cols + t % cols, y = t / cols;
+  if (m.ctas == 1 || (int)blockIdx.x * cols >= m.n_pad) return;
+  __shared__ float s_v[COLSUM_THREADS];
+  float v = 0.0f;
+  if (col < m.n_pad) {
+#pragma unroll 8
+    for (int c = y; c < m.ctas; c += m.by) v += m.part[(int64_t)c * m.n_pad + col];
+  }
+  for (int o = m.by / 2; o > 0; o >>= 1) {
+    s_v[t] = v;
+    __syncthreads();
+    if (y < o) v += s_v[t + o * cols];
+    __syncthreads();
+  }
+  if (y == 0 && col < m.n_pad) m.out[col] = v;
+}
+
 }  // namespace
 
 extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
@@ -470,5 +568,37 @@ extern "C" int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_l
   const int dw_blocks = (int)((z.n_elems / 4 + 255) / 256);
   hipLaunchKernelGGL(mlp_grad_sums, dim3(dw_blocks + (n_db + 15) / 16), dim3(256), 0, st, d, dW, dw_blocks, a.db,
                      (int)z.wgs, (int)z.db_pitch, n_db, db);
+  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+}
+
+extern "C" int gh_column_sums(const float *const *G, const int64_t *ld, const int32_t *n, const int32_t *n_pad,
+                              int32_t count, int64_t M, float *const *out, float *work, int64_t work_floats,
+                              void *stream) {
+  if (!G || !ld || !n || !n_pad || !out || !work || count <= 0 || count > MAXL || M <= 0 ||
+      M > GH_COLUMN_SUMS_MAX_ROWS || !aligned16(work))
+    return GH_EINVAL;
+  ColSums c{};
+  c.M = M;
+  int ctas = 1, blocks = 1;
+  int64_t used = 0;
+  for (int k = 0; k < count; ++k) {
+    const int w = n_pad[k];
+    if (!G[k] || !out[k] || !aligned16(out[k]) || n[k] <= 0 || n[k] > w || ld[k] < n[k] || w < 8 || w > 256 ||
+        (w & (w - 1)) != 0)
+      return GH_EINVAL;
+    ColSum &m = c.m[k];
+    m.g = G[k]; m.ld = ld[k]; m.n = n[k]; m.n_pad = w; m.out = out[k];
+    column_plan(M, w, m.by, m.ctas);
+    m.part = work + used;
+    if (m.ctas > 1) {
+      used += (int64_t)m.ctas * w;
+      blocks = std::max(blocks, (w * m.by + COLSUM_THREADS - 1) / COLSUM_THREADS);
+    }
+    ctas = std::max(ctas, m.ctas);
+  }
+  if (work_floats < used) return GH_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(column_part_kernel, dim3(ctas, count), dim3(COLSUM_THREADS), 0, st, c);
+  if (ctas > 1) hipLaunchKernelGGL(column_total_kernel, dim3(blocks, count), dim3(COLSUM_THREADS), 0, st, c);
   return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
 }

@@ -184,6 +184,7 @@ class MLP:
     # ------------------------------------------------------------------ fused inference
     FUSED_K_IN, FUSED_N_OUT, FUSED_MAX_LAYERS = 32, 16, 8
     TRAIN_MAX_ROWS = 4194240  # GH_MLP_TRAIN_MAX_ROWS
+    COLUMN_SUMS_MAX_ROWS = 65536  # GH_COLUMN_SUMS_MAX_ROWS
 
     def fused_ok(self):
         """gh_mlp_forward_packed_bf16 handles 2..8 layers with equal hidden widths of 128 or 256,
@@ -226,13 +227,11 @@ class MLP:
         (M, Xt, Y), L = self._xs, len(self.W)
         k_in, hidden, n_out, n_pad = self.psizes[0], self.psizes[1], self.sizes[-1], self.psizes[-1]
         G, G32 = grad_out, None
-        if tensor_sums:
-            G = torch.zeros(M, n_pad, device=self.dev, dtype=torch.float32)
-            G[:, :n_out] = grad_out
-            G32 = torch.empty(L - 1, M, hidden, device=self.dev, dtype=torch.float32)
-        elif G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != Xt.device or G.stride(1) != 1:
+        if G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != Xt.device or G.stride(1) != 1:
             G = torch.empty(M, n_out, device=self.dev, dtype=torch.float32)
             G[:] = grad_out
+        if tensor_sums:
+            G32 = torch.empty(L - 1, M, hidden, device=self.dev, dtype=torch.float32)
         shapes = [tuple(w.shape) for w in self.W]
         flat = torch.empty(sum(k * n for k, n in shapes), device=self.dev, dtype=torch.float32)
         dbf = torch.empty((L - 1) * hidden + n_pad, device=self.dev, dtype=torch.float32)
@@ -251,9 +250,20 @@ class MLP:
         for k, n in shapes:
             dW.append(flat[o:o + k * n].view(k, n))
             o += k * n
-        if tensor_sums:
-            return dW, [g.sum(0) for g in (*G32, G)]
-        return dW, list(dbf.split([n for _, n in shapes]))
+        db = list(dbf.split([n for _, n in shapes]))
+        if tensor_sums and M <= self.COLUMN_SUMS_MAX_ROWS and n_pad <= 256 and n_pad & (n_pad - 1) == 0:
+            grads, widths, pads = [*G32, G], [hidden] * (L - 1) + [n_out], [hidden] * (L - 1) + [n_pad]
+            work = torch.empty(256 * sum(pads), device=self.dev, dtype=torch.float32)
+            rc = self.lib.gh_column_sums(_pointers(grads), struct.pack(f"={L}q", *[g.stride(0) for g in grads]),
+                                         struct.pack(f"={L}i", *widths), struct.pack(f"={L}i", *pads), L, M,
+                                         _pointers(db), work.data_ptr(), work.numel(), self._stream())
+            if rc != 0:
+                raise RuntimeError(f"gh_column_sums failed ({rc})")
+        elif tensor_sums:
+            Gp = torch.zeros(M, n_pad, device=self.dev, dtype=torch.float32)
+            Gp[:, :n_out] = G
+            db = [g.sum(0) for g in (*G32, Gp)]
+        return dW, db
 
     def infer_fused(self, X, out):
         """All layers in one kernel (gh_mlp_forward_packed_bf16): X (M, in padded) bf16 with row
@@ -270,8 +280,8 @@ class MLP:
 
     def backward(self, grad_out, tensor_sums=False):
         """grad_out: dLoss/dOutput (M, out) FP32. Returns [dW...], [db...] (FP32, padded).
-        tensor_sums: take the bias gradients as PyTorch's column sums of the FP32 gradients,
-        the bits of the layer-by-layer path, instead of the kernels' own sums (2e-7 apart)."""
+        tensor_sums: take the bias gradients as column sums of the FP32 gradients in PyTorch's
+        order, the bits of the layer-by-layer path, instead of the kernels' own sums (2e-7 apart)."""
         torch = _torch()
         if self._zs is None:
             return self._backward_fused(grad_out, tensor_sums)
