@@ -145,11 +145,15 @@ __device__ __forceinline__ T wave_sum(T v) {
 // label of voxel vox from 2^lb-bit labels packed in 32-bit words (voxel v in word
 // v >> (5 - lb), bits (v mod 2^(5-lb)) << lb): one global load and one bit-field extract
 // for every layout, no branch on it
-__device__ __forceinline__ int packed_label(const uint32_t *labels, uint32_t lb, int vox) {
+__device__ __forceinline__ uint32_t packed_label_word(const uint32_t *labels, uint32_t lb, int vox) {
   const auto *g = (const __attribute__((address_space(1))) uint32_t *)labels;
-  const uint32_t v = (uint32_t)vox;
-  const uint32_t w = g[v >> (5u - lb)];
-  return (int)__builtin_amdgcn_ubfe(w, (v & ((1u << (5u - lb)) - 1u)) << lb, 1u << lb);
+  return g[(uint32_t)vox >> (5u - lb)];
+}
+__device__ __forceinline__ int packed_label_of(uint32_t w, uint32_t lb, int vox) {
+  return (int)__builtin_amdgcn_ubfe(w, ((uint32_t)vox & ((1u << (5u - lb)) - 1u)) << lb, 1u << lb);
+}
+__device__ __forceinline__ int packed_label(const uint32_t *labels, uint32_t lb, int vox) {
+  return packed_label_of(packed_label_word(labels, lb, vox), lb, vox);
 }
 
 struct Hot {
@@ -162,7 +166,8 @@ struct Hot {
     isx = s.inv_s[0]; isy = s.inv_s[1]; isz = s.inv_s[2];
     lb = (uint32_t)s.lb;
   }
-  __device__ __forceinline__ int label(int vox) const { return packed_label(labels, lb, vox); }
+  __device__ __forceinline__ uint32_t label_word(int vox) const { return packed_label_word(labels, lb, vox); }
+  __device__ __forceinline__ int label_of(uint32_t word, int vox) const { return packed_label_of(word, lb, vox); }
 };
 
 // (int)floorf(x) in one instruction (floor and conversion; out-of-range values clamp to the
@@ -1019,19 +1024,41 @@ transport_kernel(Launch L) {
         uint32_t w0 = rng.c0, w1 = rng.c1, w2 = rng.c2, w3 = 0x80000000u | sblock;
         philox10(w0, w1, w2, w3, rng.k0, rng.k1);
         sblock++;
-        auto woodcock = [&](auto k_c) {
-          if (mode == M_STEP) {
+        // The three steps' flights first, as if none of them collided: a step's position does not
+        // depend on the labels before it, so their reads are under way together instead of one
+        // after the other. (The flights behind a collision or an exit are not used; the lane
+        // would idle through them anyway.)
+        float d[3];
+        int vox[3];
+        uint32_t word[3];
+        {
+          float qx = ph.x, qy = ph.y, qz = ph.z;
+          auto flight = [&](auto k_c) {
+            constexpr int K = decltype(k_c)::value;
             uint32_t bd, ba;
-            step_fields<decltype(k_c)::value>(w0, w1, w2, w3, bd, ba);
-            const float d = -glog(odd22(bd) * 0x1p-22f, s_logtab) * ec.inv_maj;
-            const float nx = fmaf(d, ph.u, ph.x), ny = fmaf(d, ph.v, ph.y), nz = fmaf(d, ph.w, ph.z);
-            const int ix = floor_int(nx * hot.isx), iy = floor_int(ny * hot.isy), iz = floor_int(nz * hot.isz);
-            if ((unsigned)ix < (unsigned)hot.nx && (unsigned)iy < (unsigned)hot.ny &&
-                (unsigned)iz < (unsigned)hot.nz) {
-              ph.x = nx; ph.y = ny; ph.z = nz;
+            step_fields<K>(w0, w1, w2, w3, bd, ba);
+            d[K] = -glog(odd22(bd) * 0x1p-22f, s_logtab) * ec.inv_maj;
+            qx = fmaf(d[K], ph.u, qx); qy = fmaf(d[K], ph.v, qy); qz = fmaf(d[K], ph.w, qz);
+            const int ix = floor_int(qx * hot.isx), iy = floor_int(qy * hot.isy), iz = floor_int(qz * hot.isz);
+            const bool in = (unsigned)ix < (unsigned)hot.nx && (unsigned)iy < (unsigned)hot.ny &&
+                            (unsigned)iz < (unsigned)hot.nz;
+            vox[K] = in ? ix + hot.nx * (iy + hot.ny * iz) : -1;
+            word[K] = hot.label_word(in ? vox[K] : 0);
+          };
+          flight(std::integral_constant<int, 0>{});
+          flight(std::integral_constant<int, 1>{});
+          flight(std::integral_constant<int, 2>{});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        auto woodcock = [&](auto k_c) {
+          constexpr int K = decltype(k_c)::value;
+          if (mode == M_STEP) {
+            if (vox[K] >= 0) {
+              ph.x = fmaf(d[K], ph.u, ph.x); ph.y = fmaf(d[K], ph.v, ph.y); ph.z = fmaf(d[K], ph.w, ph.z);
               st.steps++;
-              const int vox = ix + hot.nx * (iy + hot.ny * iz);
-              const int lab = hot.label(vox);
+              uint32_t bd, ba;
+              step_fields<K>(w0, w1, w2, w3, bd, ba);
+              const int lab = hot.label_of(word[K], vox[K]);
               // table rows per material (or expanded in LDS): one read; shared composition
               // rows: the material's (density, row) pair first
               float mu;
@@ -1051,7 +1078,7 @@ transport_kernel(Launch L) {
               // maj22: the same single rounding of the same exact product
               if (odd22(ba) * ec.maj22 < mu) {
                 mode = M_COLLIDE;
-                cvox = vox;
+                cvox = vox[K];
                 clab = lab;
               }
             } else {
