@@ -116,6 +116,7 @@ struct Launch {
   int scatter_tries; // Compton / Rayleigh sampler tries per slow phase before a photon waits
   Phys P;
   unsigned long long *partial;    // [workgroup][RESULTS] counters and (as bits) energy sums
+  uint32_t copy_mask;             // tally copies - 1 (single-simulation launches: sims[] holds one entry each)
   int pair_ofs;                   // word of the dynamic LDS where the waves' pair buffers start, -1: none
 };
 
@@ -794,8 +795,9 @@ transport_kernel(Launch L) {
   const uint32_t qbase = threadIdx.x & ~63u;
 
   Hot hot;
-  // descriptor of simulation i (always 0 in the single-simulation forms)
-  auto sim = [&](int i) -> const SimDev & { return L.sims[BATCHED ? i : 0]; };
+  // descriptor of simulation i (in the single-simulation forms the one with this workgroup's
+  // copy of the tallies)
+  auto sim = [&](int i) -> const SimDev & { return L.sims[BATCHED ? (uint32_t)i : blockIdx.x & L.copy_mask]; };
   if (!BATCHED) hot.load(sim(0));
   const float tle_emax = TLE ? sim(0).tle_emax : 0.0f;
   const float tle_emin = TLE ? sim(0).tle_emin : 0.0f;
@@ -1282,6 +1284,32 @@ transport_kernel(Launch L) {
   }
 }
 
+// Tally copies. Atomics on one 64-byte piece of memory are served one every 12 ns, so a run is no
+// faster than its most-hit piece of eight voxels: around a point source inside the phantom that
+// piece takes near 2 % of the histories. Such a run adds into one of COPIES sets of tallies by
+// workgroup, and this kernel folds them into the first and clears the others for the next run. For
+// water64 (2 x 64^3 values; its fold 12 us) 3e5 histories 205 -> 219 us, 1e6 365 -> 365, 3e6
+// 805 -> 727, 1e7 2335 -> 1996, 1e8 21950 -> 18220: from COPY_MIN_SHARE histories a value on.
+constexpr int COPIES = 8;
+constexpr size_t COPY_MAX_VALUES = (size_t)4 << 20;
+constexpr size_t COPY_MIN_SHARE = 4;  // histories per value
+__global__ void __launch_bounds__(256) fold_copies_kernel(double *__restrict__ tally, double *__restrict__ copies,
+                                                          int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    double v[COPIES - 1];
+#pragma unroll
+    for (int c = 0; c < COPIES - 1; ++c) v[c] = copies[c * n + i];
+    double sum = 0.0;
+#pragma unroll
+    for (int c = 0; c < COPIES - 1; ++c) {
+      sum += v[c];
+      if (v[c] != 0.0) copies[c * n + i] = 0.0;
+    }
+    if (sum != 0.0) tally[i] += sum;
+  }
+}
+
 // sums of the workgroups' results, in a fixed order; out: host memory
 __global__ void __launch_bounds__(1024) finish_kernel(const unsigned long long *__restrict__ partial, int n,
                                                       unsigned long long *__restrict__ out) {
@@ -1377,6 +1405,7 @@ struct SimHost {
   std::vector<void *> source_owned;  // device allocations of its current source
   size_t n_tally = 0;
   int flags = 0;
+  std::vector<double *> copies;  // of the tallies() (COPIES - 1 each), zero between runs
   int det = -1;
   uint64_t event_cap = 0;
   uint64_t event_n = 0;  // histories of the last run (valid per-history detector energies)
@@ -2245,6 +2274,34 @@ int gh_reset_phsp(gh_ctx *ctx, int32_t sim_id) {
   return GH_OK;
 }
 
+// Whether this run uses the copies of the tallies, which are there when it returns true.
+static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories) {
+  const SimDev &d = h.dev;
+  if (d.pos_type != GH_POS_POINT) return false;
+  for (int i = 0; i < 3; ++i)
+    if (!(d.pos_mat[9 + i] >= 0.0f && d.pos_mat[9 + i] <= d.L[i])) return false;
+  size_t values = 0;
+  for (const auto &t : h.tallies()) values += t.second;
+  if (values > COPY_MAX_VALUES || n_histories < values * COPY_MIN_SHARE) return false;
+  if (!h.copies.empty()) return true;
+  std::vector<double *> fresh;
+  for (const auto &t : h.tallies()) {
+    const size_t bytes = (COPIES - 1) * t.second * sizeof(double);
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess || hipMemsetAsync(p, 0, bytes, ctx->stream) != hipSuccess) {
+      (void)hipGetLastError();  // no memory for them: the run does without
+      (void)hipStreamSynchronize(ctx->stream);
+      if (p) (void)hipFree(p);
+      for (double *q : fresh) (void)hipFree(q);
+      return false;
+    }
+    fresh.push_back((double *)p);
+  }
+  for (double *q : fresh) h.owned.push_back(q);
+  h.copies = std::move(fresh);
+  return true;
+}
+
 int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_history, uint64_t seed,
            const gh_launch *launch, gh_counters *out) {
   if (!ctx) return GH_EINVAL;
@@ -2287,6 +2344,18 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
   }
   Launch L;
   L.n_sims = ns;
+  L.copy_mask = 0;
+  if (ns == 1 && tally_copies(ctx, ctx->sims[0], n_histories[0])) {
+    const SimHost &h = ctx->sims[0];
+    const auto t = h.tallies();
+    devs.resize(COPIES, h.dev);
+    for (int c = 1; c < COPIES; ++c)
+      for (size_t k = 0; k < t.size(); ++k)
+        for (double **p : {&devs[c].edep, &devs[c].edep2, &devs[c].dose, &devs[c].dose2, &devs[c].counts})
+          if (*p && *p >= t[k].first && *p < t[k].first + t[k].second)
+            *p = h.copies[k] + (size_t)(c - 1) * t[k].second + (*p - t[k].first);
+    L.copy_mask = COPIES - 1;
+  }
   L.seed = seed;
   L.max_iter = lp.refill_interval;
   L.slow_min = std::max(1, std::min(64, lp.slow_min));
@@ -2384,7 +2453,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
   L.total_chunks = offs[ns];
   L.chunk = (uint32_t)lp.chunk;
   const size_t queue_bytes = QUEUES * QUEUE_STRIDE * sizeof(unsigned long long);
-  const size_t sims_bytes = (ns * sizeof(SimDev) + 15) & ~(size_t)15;
+  const size_t sims_bytes = (devs.size() * sizeof(SimDev) + 15) & ~(size_t)15;
   const size_t up_bytes = queue_bytes + sims_bytes + (ns + 1) * sizeof(uint64_t);
   if (ctx->up_cap < up_bytes) {
     if (ctx->d_up) { (void)hipFree(ctx->d_up); ctx->d_up = nullptr; }
@@ -2411,7 +2480,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
       q[k * QUEUE_STRIDE] = blocks * (uint64_t)(lp.block / 64);
       if (q[k * QUEUE_STRIDE] >= queue_chunks(L.total_chunks, k)) L.queues_empty |= 1u << k;
     }
-    std::memcpy(ctx->h_up + queue_bytes, devs.data(), ns * sizeof(SimDev));
+    std::memcpy(ctx->h_up + queue_bytes, devs.data(), devs.size() * sizeof(SimDev));
     std::memcpy(ctx->h_up + queue_bytes + sims_bytes, offs.data(), (ns + 1) * sizeof(uint64_t));
   }
   L.queue = (unsigned long long *)ctx->d_up;
@@ -2426,6 +2495,16 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     void *args[] = {&L};
     HIPCHK(hipLaunchKernel(fn, dim3(lp.grid), dim3(lp.block), args, shmem, ctx->stream));
     HIPCHK(hipGetLastError());
+    if (L.copy_mask) {
+      const SimHost &h = ctx->sims[0];
+      const auto t = h.tallies();
+      for (size_t k = 0; k < t.size(); ++k) {
+        const unsigned grid = (unsigned)std::min<size_t>((t[k].second + 255) / 256, 4096);
+        hipLaunchKernelGGL(fold_copies_kernel, dim3(grid), dim3(256), 0, ctx->stream, t[k].first, h.copies[k],
+                           (int64_t)t[k].second);
+      }
+      HIPCHK(hipGetLastError());
+    }
   }
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
   std::memset(ctx->h_result, 0, RESULTS * sizeof(unsigned long long));
