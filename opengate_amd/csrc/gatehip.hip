@@ -1289,22 +1289,26 @@ transport_kernel(Launch L) {
 // piece takes near 2 % of the histories. Such a run adds into one of COPIES sets of tallies by
 // workgroup, and this kernel folds them into the first and clears the others for the next run. For
 // water64 (2 x 64^3 values; its fold 12 us) 3e5 histories 205 -> 219 us, 1e6 365 -> 365, 3e6
-// 805 -> 727, 1e7 2335 -> 1996, 1e8 21950 -> 18220: from COPY_MIN_SHARE histories a value on.
+// 805 -> 705, 1e7 2335 -> 1935, 1e8 21950 -> 17610 (14800 are the requests themselves): from
+// COPY_MIN_SHARE histories a value on. (With copies a power of two apart 780, 2240, 20800.)
 constexpr int COPIES = 8;
 constexpr size_t COPY_MAX_VALUES = (size_t)4 << 20;
 constexpr size_t COPY_MIN_SHARE = 4;  // histories per value
+// values from a copy to the next: a voxel's copies lie on different memory channels
+__host__ __device__ constexpr size_t copy_pitch(size_t n) { return (n + 511) / 512 * 512 + 512 + 32; }
 __global__ void __launch_bounds__(256) fold_copies_kernel(double *__restrict__ tally, double *__restrict__ copies,
                                                           int64_t n) {
+  const int64_t pitch = (int64_t)copy_pitch((size_t)n);
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     double v[COPIES - 1];
 #pragma unroll
-    for (int c = 0; c < COPIES - 1; ++c) v[c] = copies[c * n + i];
+    for (int c = 0; c < COPIES - 1; ++c) v[c] = copies[c * pitch + i];
     double sum = 0.0;
 #pragma unroll
     for (int c = 0; c < COPIES - 1; ++c) {
       sum += v[c];
-      if (v[c] != 0.0) copies[c * n + i] = 0.0;
+      if (v[c] != 0.0) copies[c * pitch + i] = 0.0;
     }
     if (sum != 0.0) tally[i] += sum;
   }
@@ -2286,7 +2290,7 @@ static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories) {
   if (!h.copies.empty()) return true;
   std::vector<double *> fresh;
   for (const auto &t : h.tallies()) {
-    const size_t bytes = (COPIES - 1) * t.second * sizeof(double);
+    const size_t bytes = (COPIES - 1) * copy_pitch(t.second) * sizeof(double);
     void *p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess || hipMemsetAsync(p, 0, bytes, ctx->stream) != hipSuccess) {
       (void)hipGetLastError();  // no memory for them: the run does without
@@ -2353,7 +2357,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
       for (size_t k = 0; k < t.size(); ++k)
         for (double **p : {&devs[c].edep, &devs[c].edep2, &devs[c].dose, &devs[c].dose2, &devs[c].counts})
           if (*p && *p >= t[k].first && *p < t[k].first + t[k].second)
-            *p = h.copies[k] + (size_t)(c - 1) * t[k].second + (*p - t[k].first);
+            *p = h.copies[k] + (size_t)(c - 1) * copy_pitch(t[k].second) + (*p - t[k].first);
     L.copy_mask = COPIES - 1;
   }
   L.seed = seed;
