@@ -74,8 +74,8 @@ struct SimDev {
   int vox_nx, vox_ny;
   float vox_s[3];
   // tally
-  // with a TLE tally (edep, edep2) and (dose, dose2) lie side by side for each voxel where both
-  // are kept: then edep2 = edep + 1 and the step from voxel to voxel is two; otherwise one
+  // (edep, edep2) and (dose, dose2) lie side by side for each voxel where both are kept: then
+  // edep2 = edep + 1 and the step from voxel to voxel is two; otherwise one
   double *edep, *edep2, *dose, *dose2, *counts;
   int aligned, tnx, tny, tnz;
   float tcorner[3], tinv[3], ts[3];  // tally grid (aligned: the phantom grid, corner 0)
@@ -294,11 +294,12 @@ __device__ __forceinline__ TallyOut tally_out(const SimDev &s) {
 // round through LDS and each pair of lanes adds the two values of one voxel (two planes, or one
 // lane adding both: 11.8 voxels per ns; so 23.3, and 19 with 4 active lanes of 64). The kerma
 // estimator deposits at almost every step and is bound by these requests (2e7 histories on
-// Schneider's materials 8.56 -> 6.34 ms). The analog tallies are not (a third of the requests a
-// step), and there the exchange costs more than it saves (ct256 of 5e8 histories 91 -> 100 ms,
-// a batch of 8 5.5 -> 6.0): they keep planes and two atomics a lane.
+// Schneider's materials 8.56 -> 6.34 ms). The analog estimator is not; where a deposit of its
+// leaves the slots early, the exchange would cost more than it saves (ct256 of 5e8 histories with
+// all its deposits exchanged one by one 91 -> 100 ms), and a lane adds both.
+template <bool TLE>
 __device__ __forceinline__ void pair_add(double *base, int vox, float v, const LaneStats &st) {
-  if (st.paired) {
+  if (TLE && st.paired) {
     const uint64_t m = __ballot(1);
     const uint32_t k = (uint32_t)__popcll(m), r = mbcnt(m);
     volatile uint32_t *w = st.pair;
@@ -321,7 +322,10 @@ __device__ __forceinline__ void pair_add(double *base, int vox, float v, const L
 
 // With only that pair of images the entries of up to three deposits a lane wait in the buffer, the
 // deposits' k-th from entry 64 k on, until the whole wave adds them: one exchange for three, and
-// atomics by full waves (2e7 histories on Schneider's materials 6.31 -> 5.03 ms, 1e5 510 -> 385 us).
+// atomics by full waves (TLE, 2e7 histories on Schneider's materials 6.31 -> 5.03 ms, 1e5 510 ->
+// 385 us; the deposits of ending analog histories: water64 of 1e8 17.6 -> 17.06 ms, ct256 of 5e8
+// 85.4 -> 84.8; a batch of 8, whose lanes add both values themselves, gained from the layout: 5.22 ->
+// 5.05).
 __device__ __forceinline__ void list_entry(int region, int vox, float sum, LaneStats &st) {
   const uint32_t r = mbcnt(__ballot(1));
   volatile uint32_t *w = st.pair + region * 64;
@@ -349,15 +353,14 @@ __device__ __forceinline__ void add_list(double *base, bool e0, bool e1, bool e2
 template <bool TLE>
 __device__ __forceinline__ void flush_slot(const TallyOut &o, int vox, float sum, float dsum, uint32_t cnt,
                                            LaneStats &st) {
-  if (TLE && o.edep2) {
-    pair_add(o.edep, vox, sum, st);
+  if (o.edep2) {
+    pair_add<TLE>(o.edep, vox, sum, st);
   } else {
     gatomic_add(o.edep + vox, (double)sum);
-    if (o.edep2) gatomic_add(o.edep2 + vox, (double)sum * (double)sum);
   }
   if (o.counts) gatomic_add(o.counts + vox, (double)cnt);
-  if (TLE && o.dose && o.dose2) {
-    pair_add(o.dose, vox, dsum, st);
+  if (o.dose && o.dose2) {
+    pair_add<TLE>(o.dose, vox, dsum, st);
   } else {
     if (o.dose) gatomic_add(o.dose + vox, (double)dsum);
     if (o.dose2) gatomic_add(o.dose2 + vox, (double)dsum * (double)dsum);
@@ -827,7 +830,7 @@ transport_kernel(Launch L) {
   __syncthreads();
   LaneStats st;
   st.steps = 0u; st.rej = 0u; st.cnt = s_cnt; st.en = s_en + threadIdx.x; st.stride = BLOCK;
-  st.paired = TLE && L.pair_ofs >= 0;
+  st.paired = !BATCHED && L.pair_ofs >= 0;
   st.listed = false;
   st.pair = (uint32_t *)lds + (st.paired ? L.pair_ofs : 0) + (threadIdx.x >> 6) * PAIR_WORDS;
   const uint32_t qbase = threadIdx.x & ~63u;
@@ -837,7 +840,7 @@ transport_kernel(Launch L) {
   // copy of the tallies)
   auto sim = [&](int i) -> const SimDev & { return L.sims[BATCHED ? (uint32_t)i : blockIdx.x & L.copy_mask]; };
   if (!BATCHED) hot.load(sim(0));
-  if (TLE) {
+  if (!BATCHED) {
     const SimDev &s0 = sim(0);
     st.listed = st.paired && s0.edep2 && !s0.counts && !s0.dose && !s0.dose2;
   }
@@ -1297,7 +1300,7 @@ transport_kernel(Launch L) {
         // the event record goes first: a read of the descriptor placed after the flush's
         // atomics would wait for them
         if (s.event_edep) s.event_edep[history_of(rng) - s.first_hist] = ev_edep;
-        if (TLE && st.listed) {
+        if (!BATCHED && st.listed) {
           if ((listed[0] = sq.n > 0)) list_entry(0, sq.v0, sq.s0, st);
           if ((listed[1] = sq.n > 1)) list_entry(1, sq.v1, sq.s1, st);
           if ((listed[2] = sq.n > 2)) list_entry(2, sq.v2, sq.s2, st);
@@ -1308,7 +1311,7 @@ transport_kernel(Launch L) {
         mode = M_DEAD;
       }
     }
-    if (TLE && st.listed) {
+    if (!BATCHED && st.listed) {
       add_list(sim(0).edep, listed[0], listed[1], listed[2], st);
       if (__ballot(listed[3])) {
         if (listed[3]) list_entry(0, sq.v3, sq.s3, st);
@@ -1480,7 +1483,7 @@ struct SimHost {
   };
   Image image(int k) const {
     double *p[5] = {dev.edep, dev.edep2, dev.dose, dev.dose2, dev.counts};
-    const int e = dev.tle && dev.edep2 ? 2 : 1, d = dev.tle && dev.dose && dev.dose2 ? 2 : 1;
+    const int e = dev.edep2 ? 2 : 1, d = dev.dose && dev.dose2 ? 2 : 1;
     return {p[k], k < 2 ? e : (k < 4 ? d : 1)};
   }
   // the allocations behind the images: first value and number of values
@@ -2257,9 +2260,9 @@ int gh_add_simulation(gh_ctx *ctx, const gh_phantom_desc *ph, const gh_source_de
     d.tinv[i] = 1.0f / d.ts[i];
   }
   double *dd;
-  // an image and its image of squares; side by side for the kerma estimator
+  // an image and its image of squares, side by side
   auto images = [&](bool one, bool two, double **a, double **a2) -> int {
-    const bool pair = one && two && (tal->flags & GH_TALLY_TLE);
+    const bool pair = one && two;
     if (one || pair) {
       if ((rc = dev_upload<double>(ctx, nullptr, (pair ? 2 : 1) * ntal, &dd, h.owned))) { free_all(h.owned); return rc; }
       *a = dd;
@@ -2486,7 +2489,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
 #undef GH_PICK
   // buffers of the paired tally adds behind the tables, where the budget leaves room for them
   L.pair_ofs = -1;
-  if (tle) {
+  if (!batched) {
     const size_t at = (shmem + 15) & ~(size_t)15, end = at + (lp.block / 64) * PAIR_WORDS * sizeof(uint32_t);
     if (end <= (big ? budget_big : budget_small)) {
       L.pair_ofs = (int)(at / sizeof(uint32_t));
