@@ -1242,7 +1242,7 @@ transport_kernel(Launch L) {
           }
         }
         if (done) {
-          const float e1 = ph.E / q;
+          const float e1 = quotient(ph.E, q);
           // electrons of photons scored by the kerma estimator give nothing locally
           x_dep = (TLE && !in_world && ph.E <= tle_emax) ? 0.0f : (ph.E - e1) * ph.wt;
           ph.E = e1;

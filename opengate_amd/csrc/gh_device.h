@@ -79,6 +79,19 @@ GH_DEV uint32_t rng_next(Rng &g) {
 // uniform in (0, 1): odd multiples of 2^-24
 GH_DEV float u01(Rng &g) { return (float)((rng_next(g) >> 8) | 1u) * 0x1p-24f; }
 
+// a / b, correctly rounded, for normal operands whose quotient and remainder are normal too (a may
+// be zero): reciprocal, one Newton step, quotient and one remainder step (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990; no difference from the general
+// division over all 2^23 divisors with 8192 dividends each). 6 instructions; the general one, which
+// also scales its operands, takes 10: in the scatter samplers ct256 of 5e8 histories 84.6 -> 83.9 ms,
+// water64 of 1e6 346 -> 336 us.
+GH_DEV float quotient(float a, float b) {
+  const float y0 = __builtin_amdgcn_rcpf(b);
+  const float y = fmaf(fmaf(-b, y0, 1.0f), y0, y0);
+  const float q = a * y;
+  return fmaf(fmaf(-b, q, a), y, q);
+}
+
 // ---------------------------------------------------------------- math
 // Table of glog (written by gen_log_table.py). x = 2^e m with m in [0.5, 1) (frexp), i =
 // the top six mantissa bits of x: entry i covers m in [1/2 + i/128, 1/2 + (i+1)/128) and
@@ -163,7 +176,7 @@ GH_DEV void rotate(float &u, float &v, float &w, float c, float cp, float sp) {
   float nu, nv, nw;
   if (fabsf(w) < 0.99999f) {
     const float tmp = sqrtf(fmaf(-w, w, 1.0f));
-    const float f = st / tmp;
+    const float f = quotient(st, tmp);
     nu = fmaf(c, u, f * fmaf(u * w, cp, -(v * sp)));
     nv = fmaf(c, v, f * fmaf(v * w, cp, u * sp));
     nw = fmaf(c, w, -((st * cp) * tmp));
@@ -172,8 +185,9 @@ GH_DEV void rotate(float &u, float &v, float &w, float c, float cp, float sp) {
     nv = st * sp;
     nw = (w > 0.0f) ? c : -c;
   }
-  normalize3(nu, nv, nw);
-  u = nu; v = nv; w = nw;
+  // (unit length but for rounding, so normalize3 with the short division)
+  const float inv = quotient(1.0f, sqrtf(fmaf(nw, nw, fmaf(nv, nv, nu * nu))));
+  u = nu * inv; v = nv * inv; w = nw * inv;
 }
 
 // largest i in [0, n-2] with a[i] <= x (a ascending)
@@ -349,16 +363,16 @@ GH_DEV void branching(const Tabs &T, int nb1, int lab, const ECache &c, float &p
 // tries were all rejected in a later pass, so that a wave does not wait for its slowest
 // lane. The draws of a photon are the same either way. Returns true if accepted.
 GH_DEV bool compton_try(Rng &g, const Tabs &T, int nx, int lab, float E, float &q, float &c) {
-  const float alpha = E / MEC2;
+  const float alpha = quotient(E, MEC2);
   const float a2 = alpha + alpha;
   const float onep = 1.0f + a2;
-  const float thr = onep / (9.0f + a2);
+  const float thr = quotient(onep, 9.0f + a2);
   const float r1 = u01(g), r2 = u01(g), r3 = u01(g);
   const float t = fmaf(a2, r2, 1.0f);
   const bool low = r1 <= thr;
-  q = low ? t : onep / t;
-  const float iq = 1.0f / q;
-  c = 1.0f - (q - 1.0f) / alpha;
+  q = low ? t : quotient(onep, t);
+  const float iq = quotient(1.0f, q);
+  c = 1.0f - quotient(q - 1.0f, alpha);
   const bool acc = low ? (r3 <= 4.0f * (iq - iq * iq)) : (r3 <= 0.5f * fmaf(c, c, iq));
   if (!acc) return false;
   const float kk = E * KPM;
