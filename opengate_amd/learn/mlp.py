@@ -93,7 +93,9 @@ class MLP:
                 copies = torch.zeros(sum(sizes), device=self.dev, dtype=torch.bfloat16).split(sizes)
                 L = len(self.W16)
                 self.Wf, self.Wb = list(copies[:L]), [None, *copies[L:]]
-        if self.dev.type == "cuda" and all(w.is_contiguous() for w in self.W):
+        # one launch for tensors that it can read as they are: FP32 rows of full width where it is launched
+        if self.dev.type == "cuda" and all(w.is_contiguous() and w.dtype == torch.float32 and w.shape[0] % 8 == 0 and
+                                           w.device.index == torch.cuda.current_device() for w in self.W):
             tab = [_ADAM.pack(w.data_ptr(), 0, 0, 0, t.data_ptr(), *w.shape, 0, 0, 0.0, 0)
                    for w, t in zip(self.W, self.W16)]
             rc = self.lib.gh_pack_weights(b"".join(tab), b"".join(map(self._pack, range(len(tab)))), len(tab),
@@ -196,8 +198,9 @@ class MLP:
     def _fused_args(self):
         """Pointer arrays (bytes) of the forward weight copies and the biases; the tensors they
         point to stay referenced by the returned list."""
-        bs = [b if b.is_contiguous() and b.data_ptr() % 16 == 0 else b.clone(memory_format=_torch().contiguous_format)
-              for b in self.b]
+        torch = _torch()
+        bs = [self.b[l].to(torch.float32).contiguous() for l in range(len(self.W))]
+        bs = [b if b.data_ptr() % 16 == 0 else b.clone() for b in bs]
         return _pointers(self.Wf), _pointers(bs), bs
 
     def _train_fused(self, X):
@@ -335,6 +338,19 @@ class MLP:
         return {"sizes": self.sizes, "W": [w.cpu() for w in self.W], "b": [b.cpu() for b in self.b]}
 
     def load_state_dict(self, d):
-        self.W = [w.to(self.dev) for w in d["W"]]
-        self.b = [b.to(self.dev) for b in d["b"]]
+        """Weights and biases of any floating type, with or without the padding."""
+        self.W = [self._filled(w, self.sizes[l:l + 2], self.psizes[l:l + 2]) for l, w in enumerate(d["W"])]
+        self.b = []
+        for l, b in enumerate(d["b"]):
+            b = self._filled(b.reshape(-1), self.sizes[l + 1:l + 2], self.psizes[l + 1:l + 2])
+            self.b.append(b.expand(self.W[l].shape[1]).contiguous() if b.numel() == 1 and l < len(self.W) else b)
         self._refresh()
+
+    def _filled(self, t, sizes, full):
+        """t in FP32 on the device, padded with zeros if it has the network's own sizes."""
+        t = t.to(self.dev, _torch().float32)
+        if list(t.shape) != sizes or sizes == full:
+            return t
+        out = _torch().zeros(full, device=self.dev)
+        out[tuple(slice(n) for n in sizes)] = t
+        return out
