@@ -196,12 +196,18 @@ class MLP:
                 and self.psizes[0] <= self.FUSED_K_IN and self.psizes[-1] <= self.FUSED_N_OUT)
 
     def _fused_args(self):
-        """Pointer arrays (bytes) of the forward weight copies and the biases; the tensors they
-        point to stay referenced by the returned list."""
-        torch = _torch()
-        bs = [self.b[l].to(torch.float32).contiguous() for l in range(len(self.W))]
-        bs = [b if b.data_ptr() % 16 == 0 else b.clone() for b in bs]
-        return _pointers(self.Wf), _pointers(bs), bs
+        """Pointer arrays (bytes) of the forward weight copies and the biases; what was made for
+        them stays referenced by the returned list."""
+        f32, hold, at = _torch().float32, [], []
+        for l in range(len(self.W)):
+            b = self.b[l]
+            p = b.data_ptr()
+            if p & 15 or b.dtype is not f32 or not b.is_contiguous():
+                b = b.to(f32, copy=True).contiguous()
+                hold.append(b)
+                p = b.data_ptr()
+            at.append(p)
+        return _pointers(self.Wf), struct.pack(f"={len(at)}Q", *at), hold
 
     def _train_fused(self, X):
         """gh_mlp_train_* take the network and this batch."""
