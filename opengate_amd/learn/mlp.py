@@ -80,6 +80,8 @@ class MLP:
         self._refresh()
 
     # ------------------------------------------------------------------ helpers
+    PACK_MAX_TENSORS = 32  # of one gh_pack_weights or gh_adam_step_packed call
+
     def _refresh(self):
         """bf16 copies of the weights (kept in place: the optimiser kernel writes them): row-major
         and, for the fused kernels, the forward (W^T) and backward (W) copies in fragment order."""
@@ -94,8 +96,9 @@ class MLP:
                 L = len(self.W16)
                 self.Wf, self.Wb = list(copies[:L]), [None, *copies[L:]]
         # one launch for tensors that it can read as they are: FP32 rows of full width where it is launched
-        if self.dev.type == "cuda" and all(w.is_contiguous() and w.dtype == torch.float32 and w.shape[0] % 8 == 0 and
-                                           w.device.index == torch.cuda.current_device() for w in self.W):
+        if self.dev.type == "cuda" and 0 < len(self.W) <= self.PACK_MAX_TENSORS and all(
+                w.is_contiguous() and w.dtype == torch.float32 and w.shape[0] % 8 == 0 and
+                w.device.index == torch.cuda.current_device() for w in self.W):
             tab = [_ADAM.pack(w.data_ptr(), 0, 0, 0, t.data_ptr(), *w.shape, 0, 0, 0.0, 0)
                    for w, t in zip(self.W, self.W16)]
             rc = self.lib.gh_pack_weights(b"".join(tab), b"".join(map(self._pack, range(len(tab)))), len(tab),

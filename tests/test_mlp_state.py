@@ -83,3 +83,16 @@ def test_results_of_any_stored_type(sizes, dtype, padded):
         net.infer_fused(X, Z[0])
         want.infer_fused(X, Z[1])
         assert torch.equal(Z[0][:, : sizes[-1]], Z[1][:, : sizes[-1]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers", [32, 33])
+def test_networks_of_many_layers(layers):
+    # beyond the tensors of one packing launch the copies are made one by one
+    print(f"[gpu case] network of {layers} layers", flush=True)
+    sizes = [8] * (layers + 1)
+    net = _loaded(sizes, _state(sizes, torch.float32, True), "cuda")
+    for w, w16 in zip(net.W, net.W16):
+        assert torch.equal(w.to(torch.bfloat16), w16)
+    out = net.forward(torch.randn(20, 8, device="cuda").to(torch.bfloat16))
+    assert out.shape == (20, 8) and bool(out.isfinite().all())
