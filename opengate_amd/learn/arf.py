@@ -282,6 +282,8 @@ class ArfModel:
         N = X.shape[0]
         g = torch.Generator(device=self.dev).manual_seed(int(seed))
         cls = cls.long()
+        if cls.dim() != 1 or cls.shape[0] < N or cls.device != X.device:
+            raise ValueError("classes: one per row of X, on its device")
         cw = None
         if class_weight is not None:
             cw = torch.as_tensor(class_weight, dtype=torch.float32, device=self.dev)
