@@ -322,9 +322,11 @@ class MLP:
     def step(self, dW, db):
         """Adam update of the FP32 master weights and biases in one kernel (gh_adam_step),
         which also keeps the padding at zero and writes the bf16 weight copies (both layouts)."""
-        self.t += 1
         params = self.W + self.b
         grads = list(dW) + list(db)
+        if len(grads) < len(params):
+            raise RuntimeError("a gradient for every weight and bias is needed")
+        self.t += 1
         valid = [(k, n) for k, n in zip(self.sizes[:-1], self.sizes[1:])] + [(1, n) for n in self.sizes[1:]]
         tab, packs = [], []
         L = len(self.W)
