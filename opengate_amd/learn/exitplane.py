@@ -246,7 +246,7 @@ class ExitPlaneGenerator:
         if out is None:
             out = [torch.empty(n, device=self.dev, dtype=torch.float32) for _ in range(8)]
         m = min(int(chunk), max(n, 1))
-        if events is None and n > 0 and self._one_call():
+        if events is None and n > 0 and m > 0 and len(out) == 8 and self._one_call():
             return self._generate(n, seed, first, out, m, weight)
         X = torch.empty(m, self.mlp.psizes[0], device=self.dev, dtype=torch.bfloat16)
         bufs = None
