@@ -239,7 +239,9 @@ class MLP:
         (M, Xt, Y), L = self._xs, len(self.W)
         k_in, hidden, n_out, n_pad = self.psizes[0], self.psizes[1], self.sizes[-1], self.psizes[-1]
         G, G32 = grad_out, None
-        if G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != Xt.device or G.stride(1) != 1:
+        # (rows that overlap, as those of an expanded gradient, are laid out: the kernels take a row pitch)
+        if (G.dtype != torch.float32 or G.shape != (M, n_out) or G.device != Xt.device or G.stride(1) != 1 or
+                G.stride(0) < n_out):
             G = torch.empty(M, n_out, device=self.dev, dtype=torch.float32)
             G[:] = grad_out
         if tensor_sums:
