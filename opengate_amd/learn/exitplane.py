@@ -25,7 +25,8 @@ Training loss: sliced 2-Wasserstein distance between a generated batch and a dat
 batch in the Gaussianised space (random unit projections plus the coordinate axes,
 1-D optimal transport by sorting). The projections, the sorts, the loss and its
 gradient on the projections are one kernel (gh_sliced_w2; PyTorch tensor operations
-beyond 16384 points per batch); the gradient w.r.t. the generator output is then pushed through the network by the hand-written backward passes.
+for batches that it does not take); the gradient w.r.t. the generator output is then pushed
+through the network by the hand-written backward passes.
 """
 import ctypes as C
 import math
@@ -182,7 +183,7 @@ class ExitPlaneGenerator:
         losses = torch.empty(steps, device=self.dev)
         # per step and projection: sums of the loss kernel
         parts = (torch.empty(steps, projections + N_FEATURES, device=self.dev)
-                 if 0 < batch <= self.W2_MAX_ROWS else None)
+                 if self._w2_kernel(batch, projections + N_FEATURES) else None)
         X = torch.empty(batch, self.mlp.psizes[0], device=self.dev, dtype=torch.bfloat16)
         for it in range(steps):
             self.mlp.lr = lr_min + 0.5 * (lr - lr_min) * (1.0 + math.cos(math.pi * it / max(1, steps)))
@@ -213,6 +214,12 @@ class ExitPlaneGenerator:
         return self.history
 
     W2_MAX_ROWS = 16384  # GH_SLICED_W2_MAX_ROWS
+
+    @classmethod
+    def _w2_kernel(cls, batch, directions):
+        """gh_sliced_w2 takes a batch on this many directions: its sort holds a column in LDS, it
+        indexes the projections in 32 bits and has a grid row for 32 directions."""
+        return 0 < batch <= cls.W2_MAX_ROWS and batch * directions < 2**31 and directions <= 2**20
 
     def _sliced_w2(self, o, d, th, parts, losses, it):
         """Gradient w.r.t. the generator outputs o of the sliced distance to the data d on the
