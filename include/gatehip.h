@@ -474,11 +474,16 @@ int gh_arf_accumulate(const float *logits, int64_t ldl, int64_t m, const int32_t
                       int32_t n_win, int32_t plane, double *img, double *img2, void *stream);
 /* gh_arf_accumulate for many pairs on n_pix = heads x plane pixels, sorted by pixel first: needs
  * `bytes` of 16-byte aligned device memory as `work` for the call's time (0: too few pairs or too
- * many pixels, use gh_arf_accumulate). Pairs on pixels outside [0, n_pix) are left out. */
+ * many pixels, use gh_arf_accumulate). Pairs on pixels outside [0, n_pix) are left out. As with
+ * gh_arf_accumulate, other streams may add to the same images meanwhile; `_own` updates the images
+ * without atomics, for a caller who knows that nobody else touches them during the call. */
 int gh_arf_accumulate_workspace(int64_t m, int32_t n_win, int64_t n_pix, int32_t squared, int64_t *bytes);
 int gh_arf_accumulate_binned(const float *logits, int64_t ldl, int64_t m, const int32_t *pix, const float *wgt,
                              int32_t n_win, int32_t plane, int64_t n_pix, double *img, double *img2, void *work,
                              int64_t work_bytes, void *stream);
+int gh_arf_accumulate_binned_own(const float *logits, int64_t ldl, int64_t m, const int32_t *pix, const float *wgt,
+                                 int32_t n_win, int32_t plane, int64_t n_pix, double *img, double *img2, void *work,
+                                 int64_t work_bytes, void *stream);
 int gh_counts_accumulate(const int32_t *cls, const int32_t *pix, const float *wgt, int64_t m, int32_t n_win,
                          int32_t plane, double *img, double *img2, void *stream);
 

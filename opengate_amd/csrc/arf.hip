@@ -321,7 +321,7 @@ __global__ void __launch_bounds__(256) arf_accumulate_kernel(const float *__rest
 // at random (about 25 of them per ns over the chip, 0.9 10^6 pairs x 3 windows x 2 images 257 us), so
 // the pairs are first put in order of their pixel's bin (bin_count, bin_scatter: a counting sort
 // whose records hold the weighted probabilities), and a workgroup for each bin and window sums its
-// 4096 pixels in LDS and adds them to the images with plain loads and stores. Bins of 4096 pixels:
+// 4096 pixels in LDS and adds them to the images. Bins of 4096 pixels:
 // two workgroups a CU with both images, and a scattering workgroup's records still run together.
 constexpr int BIN_SHIFT = 12, BIN = 1 << BIN_SHIFT, MAX_BINS = 8192;
 constexpr int SORT_THREADS = 1024, SORT_PAIRS = 4096;  // pairs per sorting workgroup
@@ -421,7 +421,9 @@ __device__ __forceinline__ void lds_add_f64(double *p, double v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <int QUADS, bool SQUARED>
+// SHARED: others may add to the images meanwhile, as they may with the direct kernel, so each touched
+// pixel takes an atomic (10^6 pairs, 3 windows, squares: 64 heads 71 -> 81 us, 128 heads 86 -> 112).
+template <int QUADS, bool SQUARED, bool SHARED>
 __global__ void __launch_bounds__(512) bin_accumulate_kernel(BinWork W, int n_win, uint32_t n_pix, int plane,
                                                              double *img, double *img2) {
   __shared__ double sum[SQUARED ? 2 * BIN : BIN];
@@ -446,8 +448,13 @@ __global__ void __launch_bounds__(512) bin_accumulate_kernel(BinWork W, int n_wi
     if (s == 0.0 && s2 == 0.0) continue;
     const uint32_t head = q / (uint32_t)plane, rem = q - head * (uint32_t)plane;
     const int64_t idx = ((int64_t)head * n_win + k) * plane + rem;
-    img[idx] += s;
-    if (SQUARED) img2[idx] += s2;
+    if (SHARED) {
+      add_f64(img + idx, s);
+      if (SQUARED) add_f64(img2 + idx, s2);
+    } else {
+      img[idx] += s;
+      if (SQUARED) img2[idx] += s2;
+    }
   }
 }
 
@@ -555,7 +562,7 @@ int bin_quads(int32_t n_win) { return (n_win + 4) / 4; }
 
 int64_t bin_head_words(int64_t bins) { return (3 * bins + 1 + 3) / 4 * 4; }  // count, cursor, first
 
-template <int QUADS>
+template <int QUADS, bool SHARED>
 void launch_binned(const float *logits, int64_t ldl, int64_t m, const int32_t *pix, const float *wgt, int n_win,
                    int plane, int bins, uint32_t n_pix, BinWork W, double *img, double *img2, hipStream_t st) {
   const dim3 sort((unsigned)((m + SORT_PAIRS - 1) / SORT_PAIRS));
@@ -564,11 +571,30 @@ void launch_binned(const float *logits, int64_t ldl, int64_t m, const int32_t *p
   hipLaunchKernelGGL(bin_scatter_kernel<QUADS>, sort, dim3(SORT_THREADS), 0, st, logits, ldl, m, pix, wgt, n_win, bins,
                      n_pix, W);
   if (img2)
-    hipLaunchKernelGGL((bin_accumulate_kernel<QUADS, true>), dim3(bins, n_win), dim3(512), 0, st, W, n_win, n_pix,
-                       plane, img, img2);
+    hipLaunchKernelGGL((bin_accumulate_kernel<QUADS, true, SHARED>), dim3(bins, n_win), dim3(512), 0, st, W, n_win,
+                       n_pix, plane, img, img2);
   else
-    hipLaunchKernelGGL((bin_accumulate_kernel<QUADS, false>), dim3(bins, n_win), dim3(512), 0, st, W, n_win, n_pix,
-                       plane, img, img2);
+    hipLaunchKernelGGL((bin_accumulate_kernel<QUADS, false, SHARED>), dim3(bins, n_win), dim3(512), 0, st, W, n_win,
+                       n_pix, plane, img, img2);
+}
+
+template <bool SHARED>
+int accumulate_binned(const float *logits, int64_t ldl, int64_t m, const int32_t *pix, const float *wgt, int32_t n_win,
+                      int32_t plane, int64_t n_pix, double *img, double *img2, void *work, int64_t work_bytes,
+                      void *stream) {
+  if (!logits || !pix || !wgt || !img || !work || m < 0 || m > INT32_MAX || n_win <= 0 || n_win > MAX_WIN ||
+      ldl < n_win + 1 || plane <= 0 || n_pix <= 0 || n_pix > INT32_MAX || ((uintptr_t)work & 15) != 0)
+    return GH_EINVAL;
+  const int64_t bins = (n_pix + BIN - 1) / BIN;
+  if (bins > MAX_BINS || work_bytes < 4 * bin_head_words(bins) + 16 * bin_quads(n_win) * m) return GH_EINVAL;
+  if (m == 0) return GH_OK;
+  uint32_t *w = (uint32_t *)work;
+  const BinWork W{w, w + bins, w + 2 * bins, (float4 *)(w + bin_head_words(bins))};
+  const hipStream_t st = (hipStream_t)stream;
+  const auto launch = bin_quads(n_win) == 1 ? launch_binned<1, SHARED> :
+                      bin_quads(n_win) == 2 ? launch_binned<2, SHARED> : launch_binned<3, SHARED>;
+  launch(logits, ldl, m, pix, wgt, n_win, plane, (int)bins, (uint32_t)n_pix, W, img, img2, st);
+  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
 }
 
 }  // namespace
@@ -585,19 +611,13 @@ extern "C" int gh_arf_accumulate_workspace(int64_t m, int32_t n_win, int64_t n_p
 extern "C" int gh_arf_accumulate_binned(const float *logits, int64_t ldl, int64_t m, const int32_t *pix,
                                         const float *wgt, int32_t n_win, int32_t plane, int64_t n_pix, double *img,
                                         double *img2, void *work, int64_t work_bytes, void *stream) {
-  if (!logits || !pix || !wgt || !img || !work || m < 0 || m > INT32_MAX || n_win <= 0 || n_win > MAX_WIN ||
-      ldl < n_win + 1 || plane <= 0 || n_pix <= 0 || n_pix > INT32_MAX || ((uintptr_t)work & 15) != 0)
-    return GH_EINVAL;
-  const int64_t bins = (n_pix + BIN - 1) / BIN;
-  if (bins > MAX_BINS || work_bytes < 4 * bin_head_words(bins) + 16 * bin_quads(n_win) * m) return GH_EINVAL;
-  if (m == 0) return GH_OK;
-  uint32_t *w = (uint32_t *)work;
-  const BinWork W{w, w + bins, w + 2 * bins, (float4 *)(w + bin_head_words(bins))};
-  const hipStream_t st = (hipStream_t)stream;
-  const auto launch = bin_quads(n_win) == 1 ? launch_binned<1> :
-                      bin_quads(n_win) == 2 ? launch_binned<2> : launch_binned<3>;
-  launch(logits, ldl, m, pix, wgt, n_win, plane, (int)bins, (uint32_t)n_pix, W, img, img2, st);
-  return hipGetLastError() == hipSuccess ? GH_OK : GH_EHIP;
+  return accumulate_binned<true>(logits, ldl, m, pix, wgt, n_win, plane, n_pix, img, img2, work, work_bytes, stream);
+}
+
+extern "C" int gh_arf_accumulate_binned_own(const float *logits, int64_t ldl, int64_t m, const int32_t *pix,
+                                            const float *wgt, int32_t n_win, int32_t plane, int64_t n_pix, double *img,
+                                            double *img2, void *work, int64_t work_bytes, void *stream) {
+  return accumulate_binned<false>(logits, ldl, m, pix, wgt, n_win, plane, n_pix, img, img2, work, work_bytes, stream);
 }
 
 extern "C" int gh_counts_accumulate(const int32_t *cls, const int32_t *pix, const float *wgt, int64_t m, int32_t n_win,

@@ -336,8 +336,9 @@ class ArfModel:
         torch = _torch()
         return torch.softmax(self.mlp.forward(X, keep=False), 1)
 
-    def project(self, buf, m, img, img2=None, chunk=1 << 21, bufs=None):
-        """Add the window probabilities of the m pairs in buf into img [n_proj*n_win, ny, nx] (FP64)."""
+    def project(self, buf, m, img, img2=None, chunk=1 << 21, bufs=None, own=False):
+        """Add the window probabilities of the m pairs in buf into img [n_proj*n_win, ny, nx] (FP64).
+        own: nobody else adds to the images meanwhile (otherwise other streams may)."""
         torch = _torch()
         plane = img.shape[-1] * img.shape[-2]
         c = min(int(chunk), max(m, 1))
@@ -360,8 +361,8 @@ class ArfModel:
             pairs = (_ptr(Z), Z.shape[1], k, C.c_void_p(buf.pix.data_ptr() + 4 * s),
                      C.c_void_p(buf.wgt.data_ptr() + 4 * s), self.n_win, plane)
             if work is not None:
-                rc = self.lib.gh_arf_accumulate_binned(*pairs, n_pix, _ptr(img), _ptr(img2), _ptr(work), work.numel(),
-                                                       _stream())
+                add = self.lib.gh_arf_accumulate_binned_own if own else self.lib.gh_arf_accumulate_binned
+                rc = add(*pairs, n_pix, _ptr(img), _ptr(img2), _ptr(work), work.numel(), _stream())
             else:
                 rc = self.lib.gh_arf_accumulate(*pairs, _ptr(img), _ptr(img2), _stream())
             if rc != 0:
@@ -493,6 +494,7 @@ def project(rec, n, heads, arf=None, head_sim=None, seed=0, chunk=1 << 22, squar
         raise ValueError("learned and plain projections in one call need the same number of windows")
     n_win = arf.n_win if arf is not None else len(windows)
     shape = (heads.n_proj * n_win, heads.ny, heads.nx)
+    own = out is None  # the images of a previous call may have other users
     if out is None:
         out = {"pairs": 0, "t_pairs": 0.0, "t_arf": 0.0, "t_plain": 0.0}
         for name, on in (("arf", arf is not None), ("plain", head_sim is not None)):
@@ -520,7 +522,7 @@ def project(rec, n, heads, arf=None, head_sim=None, seed=0, chunk=1 << 22, squar
             continue
         if arf is not None:
             t = time.perf_counter()
-            arf.project(buf, m, out["arf"], out.get("arf2"), bufs=bufs)
+            arf.project(buf, m, out["arf"], out.get("arf2"), bufs=bufs, own=own)
             torch.cuda.synchronize()
             out["t_arf"] += time.perf_counter() - t
         if head_sim is not None and m:
