@@ -327,13 +327,17 @@ constexpr int BIN_SHIFT = 12, BIN = 1 << BIN_SHIFT, MAX_BINS = 8192;
 constexpr int SORT_THREADS = 1024, SORT_PAIRS = 4096;  // pairs per sorting workgroup
 
 // The direct kernel takes 0.044 ns for each atomic (pair, window, image); the binned ones 35 us for
-// their four launches, less than a tenth of that for each pair's terms, and the reading and writing
-// of the image lines that the pairs touch. Measured with 3 windows of 128 x 128, us direct / binned:
+// their four launches, the reading and writing of the image lines that the pairs touch, and 0.65 ns
+// for each pair of a bin, which one workgroup per window goes through (15 atomics' time; with few
+// bins most of the chip waits for them). Measured with 3 windows of 128 x 128, us direct / binned:
 // 16 heads with squares 128000 pairs 37 / 40, 256000 72 / 44, 10^6 267 / 61; 128 heads 128000
 // 37 / 60, 256000 72 / 64, 10^6 268 / 86; without squares 16 heads 256000 39 / 40, 10^6 144 / 57,
-// 128 heads 256000 39 / 50, 10^6 141 / 69. The line lies a little above where they meet.
+// 128 heads 256000 39 / 50, 10^6 141 / 69; 10^6 pairs with squares on one head of 64 x 64 (one bin)
+// 253 / 688, of 128 x 128 (4 bins) 263 / 202 and with one window 91 / 192, on two of those 92 / 111
+// and on four 92 / 70. The line lies a little above where they meet.
 bool binned_pays(int64_t m, int64_t n_win, int64_t n_pix, int64_t images) {
-  return m * n_win * images >= (1 << 20) + n_pix * n_win * images / 24;
+  const int64_t bins = (n_pix + BIN - 1) / BIN;
+  return m * n_win * images >= (1 << 20) + n_pix * n_win * images / 24 + 15 * m / bins;
 }
 
 struct BinWork {

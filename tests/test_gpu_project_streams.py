@@ -21,7 +21,7 @@ def _pairs(m, n_pix, seed):
 
 
 # pairs of a call: few (direct kernel), many (binned)
-@pytest.mark.parametrize("m", [3000, 400000])
+@pytest.mark.parametrize("m", [3000, 1000000])
 @pytest.mark.parametrize("squared", [True, False])
 def test_one_image_from_several_streams(m, squared):
     from opengate_amd.learn.arf import ArfModel
@@ -55,7 +55,7 @@ def test_own_images(squared):
     from opengate_amd.learn.arf import ArfModel
 
     print(f"[gpu case] own image, squared={squared}", flush=True)
-    m, heads, ny, nx = 400003, 7, 60, 70
+    m, heads, ny, nx = 1200003, 7, 60, 70
     arf = ArfModel(theta_max=math.radians(10.0), seed=4)
     buf = _pairs(m, heads * ny * nx, 9)
     out = []
