@@ -1675,6 +1675,22 @@ void staging_give(int device, std::vector<StagingBlock> &v) {
   v.clear();
 }
 
+// Where a kernel writes a destination that starts in pinned memory (`at`: its first byte): at the
+// device's address of it, if the last byte is of the same piece; otherwise nullptr, and the
+// runtime's own copy takes it.
+double *pinned_device_address(const HostCopy &c, const hipPointerAttribute_t &at) {
+  if (at.type != hipMemoryTypeHost || !at.devicePointer) return nullptr;
+  const size_t last = c.n * sizeof(double) - 1;
+  hipPointerAttribute_t end{};
+  if (hipPointerGetAttributes(&end, (const char *)c.dst + last) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const bool one_piece = end.type == hipMemoryTypeHost && end.device == at.device &&
+                         (const char *)end.devicePointer == (const char *)at.devicePointer + last;
+  return one_piece ? (double *)at.devicePointer : nullptr;
+}
+
 int copy_to_host(gh_ctx *ctx, const std::vector<HostCopy> &parts) {
   std::vector<HostCopy> blocks, direct, via_device;
   size_t total = 0;
@@ -1683,7 +1699,9 @@ int copy_to_host(gh_ctx *ctx, const std::vector<HostCopy> &parts) {
     const bool known = hipPointerGetAttributes(&at, c.dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
     if (!known) (void)hipGetLastError();
     if (known) {  // pinned, managed or device memory needs no staging
-      (c.step == 1 || at.type == hipMemoryTypeHost ? direct : via_device).push_back(c);
+      double *pinned = c.step == 1 ? c.dst : pinned_device_address(c, at);
+      if (pinned) direct.push_back({pinned, c.src, c.n, c.step});
+      else via_device.push_back(c);
       continue;
     }
     total += c.n * sizeof(double);
