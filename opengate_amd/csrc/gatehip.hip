@@ -116,7 +116,7 @@ struct Launch {
   int scatter_tries; // Compton / Rayleigh sampler tries per slow phase before a photon waits
   Phys P;
   unsigned long long *partial;    // [workgroup][RESULTS] counters and (as bits) energy sums
-  uint32_t copy_mask;             // tally copies - 1 (single-simulation launches: sims[] holds one entry each)
+  uint32_t copy_mask;             // tally copies - 1 (sims[] holds n_sims entries for each)
   int pair_ofs;                   // word of the dynamic LDS where the waves' pair buffers start, -1: none
 };
 
@@ -852,9 +852,9 @@ transport_kernel(Launch L) {
   const uint32_t qbase = threadIdx.x & ~63u;
 
   Hot hot;
-  // descriptor of simulation i (in the single-simulation forms the one with this workgroup's
-  // copy of the tallies)
-  auto sim = [&](int i) -> const SimDev & { return L.sims[BATCHED ? (uint32_t)i : blockIdx.x & L.copy_mask]; };
+  // descriptor of simulation i with this workgroup's copy of the tallies
+  const SimDev *sims = L.sims + (blockIdx.x & L.copy_mask) * (BATCHED ? (uint32_t)L.n_sims : 1u);
+  auto sim = [&](int i) -> const SimDev & { return sims[BATCHED ? (uint32_t)i : 0u]; };
   if (!BATCHED) hot.load(sim(0));
   if (!BATCHED) {
     const SimDev &s0 = sim(0);
@@ -1366,10 +1366,17 @@ transport_kernel(Launch L) {
 // workgroup, and this kernel folds them into the first and clears the others for the next run. For
 // water64 (2 x 64^3 values; its fold 12 us) 3e5 histories 205 -> 219 us, 1e6 365 -> 365, 3e6
 // 805 -> 705, 1e7 2335 -> 1935, 1e8 21950 -> 17610 (14800 are the requests themselves): from
-// COPY_MIN_SHARE histories a value on. (With copies a power of two apart 780, 2240, 20800.)
+// COPY_MIN_SHARE histories a value on. (With copies a power of two apart 780, 2240, 20800.) A launch
+// of several simulations works on one after the other, and its lanes add the two values of a voxel,
+// which lie in one piece, by themselves: 8 simulations of 2.5e6 histories in 16^3 voxels 9.2 -> 4.9 ms,
+// in 64^3 5.0 -> 4.3 (8.0 and 4.5 with the values in two pieces); 256 of 78000 4.24 -> 4.85, so a
+// simulation that shares its launch needs COPY_MIN_OF_MANY histories.
 constexpr int COPIES = 8;
 constexpr size_t COPY_MAX_VALUES = (size_t)4 << 20;
 constexpr size_t COPY_MIN_SHARE = 4;  // histories per value
+constexpr int COPY_MAX_SIMS = 256;    // of a launch: their descriptors are uploaded COPIES times
+constexpr uint64_t COPY_MIN_OF_MANY = 500000;  // histories of a simulation that shares its launch
+constexpr size_t COPY_MAX_BYTES = (size_t)1 << 30;  // of a context's copies
 // values from a copy to the next: a voxel's copies lie on different memory channels
 __host__ __device__ constexpr size_t copy_pitch(size_t n) { return (n + 511) / 512 * 512 + 512 + 32; }
 __global__ void __launch_bounds__(256) fold_copies_kernel(double *__restrict__ tally, double *__restrict__ copies,
@@ -1530,6 +1537,7 @@ struct gh_ctx {
   size_t lds1e_bytes = 0, lds2e_bytes = 0;  // the same with mu expanded per material
   // simulations
   std::vector<SimHost> sims;
+  size_t copy_bytes = 0;  // of their tally copies
   // run scratch
   // one upload per run, from pinned memory: queue counters, simulation descriptors, chunk offsets
   unsigned char *h_up = nullptr, *d_up = nullptr;
@@ -2195,6 +2203,7 @@ int gh_clear_simulations(gh_ctx *ctx) {
   HIPCHK(hipStreamSynchronize(ctx->stream));
   for (auto &s : ctx->sims) { free_all(s.owned); free_all(s.source_owned); }
   ctx->sims.clear();
+  ctx->copy_bytes = 0;
   return GH_OK;
 }
 
@@ -2382,6 +2391,9 @@ static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories) {
   for (const auto &t : h.tallies()) values += t.second;
   if (values > COPY_MAX_VALUES || n_histories < values * COPY_MIN_SHARE) return false;
   if (!h.copies.empty()) return true;
+  size_t need = 0;
+  for (const auto &t : h.tallies()) need += (COPIES - 1) * copy_pitch(t.second) * sizeof(double);
+  if (ctx->copy_bytes + need > COPY_MAX_BYTES) return false;
   std::vector<double *> fresh;
   for (const auto &t : h.tallies()) {
     const size_t bytes = (COPIES - 1) * copy_pitch(t.second) * sizeof(double);
@@ -2397,6 +2409,7 @@ static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories) {
   }
   for (double *q : fresh) h.owned.push_back(q);
   h.copies = std::move(fresh);
+  ctx->copy_bytes += need;
   return true;
 }
 
@@ -2443,16 +2456,24 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
   Launch L;
   L.n_sims = ns;
   L.copy_mask = 0;
-  if (ns == 1 && tally_copies(ctx, ctx->sims[0], n_histories[0])) {
-    const SimHost &h = ctx->sims[0];
-    const auto t = h.tallies();
-    devs.resize(COPIES, h.dev);
-    for (int c = 1; c < COPIES; ++c)
-      for (size_t k = 0; k < t.size(); ++k)
-        for (double **p : {&devs[c].edep, &devs[c].edep2, &devs[c].dose, &devs[c].dose2, &devs[c].counts})
-          if (*p && *p >= t[k].first && *p < t[k].first + t[k].second)
-            *p = h.copies[k] + (size_t)(c - 1) * copy_pitch(t[k].second) + (*p - t[k].first);
+  std::vector<SimHost *> copied;
+  for (int s = 0; s < (ns <= COPY_MAX_SIMS ? ns : 0); ++s)
+    if ((ns == 1 || n_histories[s] >= COPY_MIN_OF_MANY) && tally_copies(ctx, ctx->sims[s], n_histories[s]))
+      copied.push_back(&ctx->sims[s]);
+  if (!copied.empty()) {
     L.copy_mask = COPIES - 1;
+    devs.resize((size_t)COPIES * ns);
+    for (int c = 1; c < COPIES; ++c) {
+      std::copy(devs.begin(), devs.begin() + ns, devs.begin() + (size_t)c * ns);
+      for (const SimHost *h : copied) {
+        const auto t = h->tallies();
+        SimDev &d = devs[(size_t)c * ns + (h - ctx->sims.data())];
+        for (size_t k = 0; k < t.size(); ++k)
+          for (double **p : {&d.edep, &d.edep2, &d.dose, &d.dose2, &d.counts})
+            if (*p && *p >= t[k].first && *p < t[k].first + t[k].second)
+              *p = h->copies[k] + (size_t)(c - 1) * copy_pitch(t[k].second) + (*p - t[k].first);
+      }
+    }
   }
   L.seed = seed;
   L.max_iter = lp.refill_interval;
@@ -2593,12 +2614,11 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     void *args[] = {&L};
     HIPCHK(hipLaunchKernel(fn, dim3(lp.grid), dim3(lp.block), args, shmem, ctx->stream));
     HIPCHK(hipGetLastError());
-    if (L.copy_mask) {
-      const SimHost &h = ctx->sims[0];
-      const auto t = h.tallies();
+    for (const SimHost *h : copied) {
+      const auto t = h->tallies();
       for (size_t k = 0; k < t.size(); ++k) {
         const unsigned grid = (unsigned)std::min<size_t>((t[k].second + 255) / 256, 4096);
-        hipLaunchKernelGGL(fold_copies_kernel, dim3(grid), dim3(256), 0, ctx->stream, t[k].first, h.copies[k],
+        hipLaunchKernelGGL(fold_copies_kernel, dim3(grid), dim3(256), 0, ctx->stream, t[k].first, h->copies[k],
                            (int64_t)t[k].second);
       }
       HIPCHK(hipGetLastError());
