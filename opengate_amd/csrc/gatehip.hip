@@ -2624,12 +2624,12 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
       HIPCHK(hipGetLastError());
     }
   }
-  HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
   std::memset(ctx->h_result, 0, RESULTS * sizeof(unsigned long long));
   if (L.total_chunks > 0) {
     hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->d_partial, (int)lp.grid, ctx->h_result);
     HIPCHK(hipGetLastError());
   }
+  HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   unsigned long long c[N_COUNTERS];
   double e[N_ENERGIES];
