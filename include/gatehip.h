@@ -253,6 +253,10 @@ int gh_hu_to_labels(gh_ctx *ctx, const int16_t *hu, int64_t n_voxels, const doub
 int gh_hu_to_labels_f64(gh_ctx *ctx, const double *hu, int64_t n_voxels, const double *bins,
                         int32_t n_bins, const uint16_t *labels_sorted, uint16_t *out);
 
+/* out[i] = a[i] / b[i] by the division of the transport's scatter samplers (device arrays; no
+ * counterpart in the reference: lets tests compare its bits with the correctly rounded quotient). */
+int gh_quotient(const float *a, const float *b, int64_t n, float *out, void *stream);
+
 /* ---- dense-layer GEMM for the learned models (no reference counterpart: the reference
  * runs its GAN source and ARF networks through torch, gansources.py:512, arfactors.py:388).
  * C[M,N] = A[M,K] * B[K,N] in bf16 with FP32 accumulation on the matrix cores;

@@ -81,8 +81,9 @@ GH_DEV float u01(Rng &g) { return (float)((rng_next(g) >> 8) | 1u) * 0x1p-24f; }
 
 // a / b, correctly rounded, for normal operands whose quotient and remainder are normal too (a may
 // be zero): reciprocal, one Newton step, quotient and one remainder step (Markstein, "Computation of
-// elementary functions on the IBM RISC System/6000 processor", 1990; no difference from the general
-// division over all 2^23 divisors with 8192 dividends each). 6 instructions; the general one, which
+// elementary functions on the IBM RISC System/6000 processor", 1990; his proof takes a correctly
+// rounded reciprocal, which one step from the hardware's need not give: tests/test_gpu_quotient.py
+// compares all 2^23 divisor mantissas and the ranges used here). 6 instructions; the general one, which
 // also scales its operands, takes 10: in the scatter samplers ct256 of 5e8 histories 84.6 -> 83.9 ms,
 // water64 of 1e6 346 -> 336 us.
 GH_DEV float quotient(float a, float b) {
