@@ -604,10 +604,10 @@ int accumulate_binned(const float *logits, int64_t ldl, int64_t m, const int32_t
 }  // namespace
 
 extern "C" int gh_arf_accumulate_workspace(int64_t m, int32_t n_win, int64_t n_pix, int32_t squared, int64_t *bytes) {
-  if (!bytes || m < 0 || n_win <= 0 || n_win > MAX_WIN || n_pix <= 0 || n_pix > INT32_MAX) return GH_EINVAL;
+  if (!bytes || m < 0 || n_win <= 0 || n_win > MAX_WIN || n_pix < 0) return GH_EINVAL;
   const int64_t bins = (n_pix + BIN - 1) / BIN;
   *bytes = 0;
-  if (bins > MAX_BINS || m > INT32_MAX || !binned_pays(m, n_win, n_pix, squared ? 2 : 1)) return GH_OK;
+  if (bins == 0 || bins > MAX_BINS || m > INT32_MAX || !binned_pays(m, n_win, n_pix, squared ? 2 : 1)) return GH_OK;
   *bytes = 4 * bin_head_words(bins) + 16 * bin_quads(n_win) * m;
   return GH_OK;
 }

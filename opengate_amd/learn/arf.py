@@ -349,7 +349,8 @@ class ArfModel:
                     for _ in range(2)]
         n_pix = img.numel() // self.n_win
         need = C.c_int64(0)
-        if self.lib.gh_arf_accumulate_workspace(c, self.n_win, n_pix, int(img2 is not None), C.byref(need)) != 0:
+        if m > 0 and self.lib.gh_arf_accumulate_workspace(c, self.n_win, n_pix, int(img2 is not None),
+                                                          C.byref(need)) != 0:
             raise RuntimeError("gh_arf_accumulate_workspace failed")
         work = torch.empty(need.value, device=self.dev, dtype=torch.uint8) if need.value else None
         for s in range(0, m, c):
