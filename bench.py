@@ -16,7 +16,8 @@ Default workload ("headline"): the metric's own comparison, learned vs plain GPU
                          1e6 histories per run, GPU against the CPU restatement;
   roofline      the dominant kernel of the learned step (the fused generator forward,
                 MFMA-bound: FLOP per launch / its average duration from CUDA events on
-                the stream it runs on, against 2.5 PFLOP/s dense BF16);
+                the stream it runs on, in a pass of its own behind the timed steps, against
+                2.5 PFLOP/s dense BF16);
   cpu_baseline  the CPU restatement (oracle/transport_ref.c) on config 1, on the host's
                 CPUs (all of them the process may use), for a bounded sample.
 
@@ -491,7 +492,6 @@ def leg_exitplane(args):
     # ---- learned: generator + phantom, the same photon count per chunk
     ct.reset_tally(0)
     buf = [torch.empty(max(counts), device="cuda") for _ in range(8)]
-    events = []
     for k in range(n_warm):
         rec = gen.generate(counts[0], seed=55, first=k * counts[0], out=[b[:counts[0]] for b in buf])
         ct.set_source(0, phsp_source(rec))
@@ -505,7 +505,7 @@ def leg_exitplane(args):
     for m in counts:
         torch.cuda.synchronize()
         t = time.perf_counter()
-        rec = gen.generate(m, seed=5, first=done, out=[b[:m] for b in buf], events=events)
+        rec = gen.generate(m, seed=5, first=done, out=[b[:m] for b in buf])
         torch.cuda.synchronize()
         t_gen += time.perf_counter() - t
         if first_rec is None:
@@ -523,9 +523,14 @@ def leg_exitplane(args):
     dose = compare_dose(learned["edep"], plain["edep"], test2=learned["edep2"], ref2=plain["edep2"],
                         n_test=n_total, n_ref=n_total)
     gen_rate = n_total / t_gen
+    # the network's own launches, in a pass of its own: the timed steps make noise, network and
+    # photons in one call, as a user's do
+    events = []
+    gen.generate(counts[0], seed=5, out=[b[:counts[0]] for b in buf], events=events)
+    torch.cuda.synchronize()
     fwd_ms = sum(a.elapsed_time(b) for a, b in events)
     fwd_launches = len(events)
-    fwd_flops = gen.flops_per_photon() * n_total
+    fwd_flops = gen.flops_per_photon() * counts[0]
     fwd_tflops = fwd_flops / (fwd_ms * 1e-3) / 1e12
     ph_kms = sum(c["kernel_ms"] for c in ph_counters)
     ph_bytes = sum(algorithmic_bytes(c) for c in ph_counters)
@@ -573,7 +578,7 @@ def leg_exitplane(args):
                                        "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                        "frac": ph_bytes / (ph_kms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                                        "kernel_ms_per_launch": ph_kms / len(ph_counters)},
-        "time_split_s": {"generator": t_gen, "generator_forward_kernels": fwd_ms * 1e-3,
+        "time_split_s": {"generator": t_gen, "generator_forward_kernels": fwd_ms * 1e-3 * n_total / counts[0],
                          "phantom_transport_learned": t_ph2, "plain_upstream": t_up, "plain_phantom": t_ph},
     }
     col.close()
@@ -712,7 +717,7 @@ def bench_mlp(args):
         "warmup": 1, "ms_per_step": g["ms"], "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "bf16 (fp32 accumulate)", "data": "synthetic (random weights and inputs)",
         "config": {"workload": "MLP inference: exit-plane generator 8->256x5->6 and detector response "
-                               "3->128x3->4, 2^23 rows per call", "form": "gh_mlp_forward_bf16 vs gh_gemm_bf16",
+                               "3->128x3->4, 2^23 rows per call", "form": "gh_mlp_forward_packed_bf16 vs gh_gemm_bf16",
                    "networks": out},
         "roofline": {"bound": "mfma", "achieved": g["tflops"], "peak": 2500.0, "unit": "TFLOP/s",
                      "frac": g["tflops"] / 2500.0, "traffic": None},

@@ -302,7 +302,8 @@ int gh_mlp_forward_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers,
                         void *stream);
 
 /* The same with wt[l] in fragment order (see gh_adam_step_packed) and 16-byte aligned bias[l] of
- * the hidden layers. */
+ * the hidden layers: the faster one, which the package's own networks use; the form above is for
+ * callers who hold row-major weights. */
 int gh_mlp_forward_packed_bf16(const void *X, int64_t ldx, int64_t M, int32_t n_layers, int32_t k_in, int32_t hidden,
                                int32_t n_out, const void *const *wt, const float *const *bias, float *Z, int64_t ldz,
                                void *stream);
@@ -370,10 +371,16 @@ int gh_mlp_train_backward_bf16(const void *Xt, int64_t M, int32_t n_layers, int3
                                int32_t np, const void *const *w, const void *const *Y, const float *G, int64_t ldg,
                                float *dW, float *db, float *const *G32, void *ws, int64_t ws_bytes, void *stream);
 
-/* Column sums of `count` (at most 8) FP32 matrices of M rows in one fixed order of additions, that
- * of PyTorch's sum over the rows: G[k] M x n[k] with row pitch ld[k]; out[k]: n_pad[k] sums (a
- * power of two from 8 to 256, at least n[k]; those behind n[k] are zero). work: 256 sum(n_pad)
- * floats. M at most GH_COLUMN_SUMS_MAX_ROWS. */
+/* Column sums of `count` (at most 8) FP32 matrices of M rows in one fixed order of additions:
+ * G[k] M x n[k] with row pitch ld[k]; out[k]: n_pad[k] sums (a power of two from 8 to 256, at
+ * least n[k]; those behind n[k] are zero). work: 256 sum(n_pad) floats. M at most
+ * GH_COLUMN_SUMS_MAX_ROWS.
+ * The order: chain s of S = by ctas adds rows s, s + S, s + 2 S, ... in four running sums (the i-th
+ * row into sum i mod 4), then ((sum 0 + sum 1) + sum 2) + sum 3; chains c by + y of a group c add
+ * up by halves (y + by/2 onto y, then by/4, ...); with more than one group, totals y, y + by, ... of
+ * the groups one after the other, and those by halves again. by = 512 / n_pad, or 1 if M < 256 and
+ * M < 16 by; with rows = ceil(M / by) and g = ceil(rows / 16), ctas = 1 below 256 rows, else g up to
+ * 128, 128 up to 256, 256 beyond. (It gives the bits of sum(0) of PyTorch 2.10.0 for ROCm 7.0.) */
 #define GH_COLUMN_SUMS_MAX_ROWS 65536
 int gh_column_sums(const float *const *G, const int64_t *ld, const int32_t *n, const int32_t *n_pad, int32_t count,
                    int64_t M, float *const *out, float *work, int64_t work_floats, void *stream);

@@ -507,8 +507,9 @@ extern "C" int gh_spect_pairs(const float *const rec[8], int64_t n, const gh_spe
     }
   }
   if (n == 0) return GH_OK;
-  // as many workgroups as the chip holds at once: each then writes its pairs out few times
-  const dim3 grid(grid_for(n, 5));
+  // as many workgroups as the chip holds at once (27 KiB of LDS each, 34 with detector records):
+  // each then writes its pairs out few times
+  const dim3 grid(grid_for(n, det_rec ? 4 : 5));
   if (det_rec)
     hipLaunchKernelGGL(spect_pairs_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, rec[0], rec[1], rec[2],
                        rec[3], rec[4], rec[5], rec[6], rec[7], n, *det, angle_cs, o);

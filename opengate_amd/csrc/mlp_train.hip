@@ -372,12 +372,13 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // Sums over the rows of several FP32 matrices, in one fixed order of additions: workgroup c of
 // `ctas` and its thread row y of `by` add the rows s + S i, s = c by + y and S = by ctas, in
 // four running sums (i mod 4), then those, then the thread rows by halves, then the workgroups
-// (y, y + by, ... and the thread rows by halves again). This is the order in which PyTorch sums
-// the columns of a matrix of these widths, found by comparing bits over 1..70000 rows
-// (tests/test_gpu_column_sums.py holds it): fits divide by the size of nearly cancelled sums in
-// their first steps, so another order gives other weights. Its calls, one a layer, took 125 us for
-// 5 x 16384 x 256 and 32 for 3 x 5003 x 128; these two launches 23 and 15, the first bound by
-// reading 84 MB from behind the L2 (5.2 TB/s), the second by the one workgroup of its last layer.
+// (y, y + by, ... and the thread rows by halves again). This is the order in which PyTorch
+// 2.10.0 sums the columns of a matrix of these widths, found by comparing bits over 1..70000 rows
+// (tests/test_gpu_column_sums.py holds it; another version may sum in another order, this one does
+// not change): fits divide by the size of nearly cancelled sums in their first steps, so another
+// order gives other weights. PyTorch's calls, one a layer, took 125 us for 5 x 16384 x 256 and 32
+// for 3 x 5003 x 128; these two launches 23 and 15, the first bound by reading 84 MB from behind
+// the L2 (5.2 TB/s), the second by the one workgroup of its last layer.
 struct ColSum {
   const float *g;
   int64_t ld;
@@ -492,9 +493,9 @@ extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_lay
   hipStream_t st = (hipStream_t)stream;
   const int rt = row_tiles(M);
 #define GH_ROWS(H)                                                                  \
-  (rt == 1 ? launch_rows_forward<H, 1, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)       \
-           : (rt == 2 ? launch_rows_forward<H, 2, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st) \
-                      : launch_rows_forward<H, 4, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)))
+  (rt == 1 ? launch_rows_forward<H, 1, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)       \
+           : (rt == 2 ? launch_rows_forward<H, 2, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st) \
+                      : launch_rows_forward<H, 4, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)))
   return hidden == 256 ? GH_ROWS(256) : GH_ROWS(128);
 #undef GH_ROWS
 }

@@ -2,10 +2,8 @@
 
 The generator maps 8-D Gaussian noise to 6 values (E, x, y, u', v', w') through a
 6-layer dense network (width 256, BF16 weights, FP32 accumulation), evaluated and
-trained with the library's own kernels (gh_gaussian_bf16 for the noise, gh_gemm_bf16
-for every product of the training forward and backward passes, gh_mlp_forward_bf16 for
-generation (all six layers in one kernel), gh_exitplane_decode for the mapping back to
-photons). It replaces the upstream transport that produced the
+trained with the library's own kernels (gh_mlp_train_* for the training passes,
+gh_exitplane_generate for noise, network and the mapping back to photons in one call). It replaces the upstream transport that produced the
 exit-plane photons (the role of GANSource + GANSourceDefaultGenerator,
 sources/gansources.py:270-431,457-757).
 

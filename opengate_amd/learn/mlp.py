@@ -294,8 +294,8 @@ class MLP:
 
     def backward(self, grad_out, tensor_sums=False):
         """grad_out: dLoss/dOutput (M, out) FP32. Returns [dW...], [db...] (FP32, padded).
-        tensor_sums: take the bias gradients as column sums of the FP32 gradients in PyTorch's
-        order, the bits of the layer-by-layer path, instead of the kernels' own sums (2e-7 apart)."""
+        tensor_sums: take the bias gradients as column sums of the FP32 gradients in the order of
+        gh_column_sums (that of PyTorch 2.10.0's sum), the bits of the layer-by-layer path, instead of the kernels' own sums (2e-7 apart)."""
         torch = _torch()
         if self._zs is None:
             return self._backward_fused(grad_out, tensor_sums)
