@@ -840,9 +840,9 @@ int launch_rows(const __bf16 *X, int64_t ldx, int64_t M, const MlpArgs &a, const
                 int64_t ldz, hipStream_t st) {
   const MlpKeep keep{};
   switch (row_tiles(M)) {
-    case 1: return launch_rows_forward<H, 1, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
-    case 2: return launch_rows_forward<H, 2, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
-    default: return launch_rows_forward<H, 4, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+    case 1: return launch_rows_forward<H, 1, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+    case 2: return launch_rows_forward<H, 2, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
+    default: return launch_rows_forward<H, 4, 8, MODE>(X, ldx, M, a, keep, gen, Z, ldz, st);
   }
 }
 

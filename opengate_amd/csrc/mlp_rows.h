@@ -3,15 +3,15 @@
 //
 // What bounds it: a batch of 1e3..4e4 rows gives every CU one tile of 16..64 rows, so a layer
 // lasts 1-4 us and its weights (H x H bf16, 128 KiB at H = 256) come from L2 in that time. The
-// eight waves own H / 8 output columns each for all rows of the tile, so no two waves of a
-// workgroup read the same weights. A wave holds its weights as MFMA fragments in registers;
-// those of the next layer are loaded into them as this layer's steps are done with them. One
-// barrier per layer. The activations go through LDS in fragment order: 16-byte unit (row tile i,
-// k step ks, lane l) at ((i NK + ks) 64 + l) 16, lane l holding row l % 16 and
-// k = 32 ks + 8 (l / 16) + 0..7, so the reads and writes of a wave are consecutive (no bank
-// conflicts). Two activation buffers alternate. The MFMA sequence of an output element (k steps
-// of 32 in order, bias, ReLU, bf16 rounding) is that of the layer-by-layer GEMMs: bit-identical
-// results.
+// waves form CG column groups x 8 / CG row groups; at H = 256 (CG = 8) each owns 32 output
+// columns for all rows of the tile, so no two waves of a workgroup read the same weights. A
+// wave holds its weights as MFMA fragments in registers; those of the next layer are loaded
+// into them as this layer's steps are done with them. One barrier per layer. The
+// activations go through LDS in fragment order: 16-byte unit (row tile i, k step ks, lane l) at
+// ((i NK + ks) 64 + l) 16, lane l holding row l % 16 and k = 32 ks + 8 (l / 16) + 0..7, so the
+// reads and writes of a wave are consecutive (no bank conflicts). Two activation buffers
+// alternate. The MFMA sequence of an output element (k steps of 32 in order, bias, ReLU, bf16
+// rounding) is that of the layer-by-layer GEMMs: bit-identical results.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
@@ -154,29 +154,33 @@ __device__ __forceinline__ void rows_weights(bf16x8 (&w)[NK][CT], const __bf16 *
 
 // Forward through all layers. MODE: inference (Z: columns 0..n_out-1), training (also keeps the
 // activations), or noise -> photons (X and Z unused).
-template <int H, int RT, int MODE>
+template <int H, int RT, int CG, int MODE>
 __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_forward(const __bf16 *__restrict__ X, int64_t ldx, int64_t M,
                                                                 MlpArgs a, MlpKeep keep, MlpGenerate gen,
                                                                 float *__restrict__ Z, int64_t ldz) {
   constexpr bool KEEP = MODE == ROWS_KEEP, GENERATE = MODE == ROWS_GENERATE;
-  // CT column tiles per wave, all RT row tiles
-  constexpr int NK = H / 32, CT = H / 128, ROWS = 16 * RT;
+  // RW row tiles and CT column tiles per wave. (CG is 8 everywhere; with the row offset i0, then
+  // zero, folded away, the training forward at 16384 rows takes 19.4 us instead of 18.7: the
+  // addresses in registers leave the compiler a better order.)
+  constexpr int NK = H / 32, RG = 8 / CG, CT = H / 16 / CG, RW = RT / RG, ROWS = 16 * RT;
+  static_assert(RT % RG == 0, "the row groups share the tile's row tiles evenly");
   extern __shared__ __align__(16) unsigned char mlp_lds[];
   __bf16 *in = (__bf16 *)mlp_lds, *out = in + ROWS * H;
   float *s_bias = (float *)(mlp_lds + 2 * ROWS * H * sizeof(__bf16));  // [layer][H]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, g = lane >> 4;
-  const int n0 = wave * 16 * CT;
+  const int cg = wave % CG, i0 = wave / CG * RW;
+  const int n0 = cg * 16 * CT;
   const int64_t row0 = (int64_t)blockIdx.x * ROWS;
   const int L = a.n_layers;
   bf16x8 w0[CT], w[NK][CT];
   // weights of layer l >= 1: a hidden layer's column tiles, or the output layer's 16 columns
   // (past the end: the output layer again; a branch around the loads would make the compiler
   // wait for all of them in the path without)
-  auto tiles = [&](int l) { return a.wt[min(l, L - 1)] + (l < L - 1 ? wave * CT * NK * 512 : 0) + lane * 8; };
+  auto tiles = [&](int l) { return a.wt[min(l, L - 1)] + (l < L - 1 ? cg * CT * NK * 512 : 0) + lane * 8; };
   auto step = [&](int l) { return l < L - 1 ? NK * 512 : 0; };
 #pragma unroll
-  for (int j = 0; j < CT; ++j) w0[j] = *(const bf16x8 *)(a.wt[0] + ((wave * CT + j) * 64 + lane) * 8);
+  for (int j = 0; j < CT; ++j) w0[j] = *(const bf16x8 *)(a.wt[0] + ((cg * CT + j) * 64 + lane) * 8);
   for (int u = tid; u < ROWS * 4; u += ROW_THREADS) {
     const int r = u >> 2, q = (u & 3) * 8;
     const int64_t gr = row0 + r;
@@ -205,7 +209,7 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_forward(const __bf16 *__
     ((floatx4 *)s_bias)[u] = ((const floatx4 *)a.bias[u / (H / 4)])[u % (H / 4)];
   rows_weights<CT, NK>(w, tiles(1), step(1));
   __syncthreads();
-  floatx4 acc[RT][CT];
+  floatx4 acc[RW][CT];
   // bias, ReLU, bf16; into the other activation buffer and, in training, to memory
   auto finish = [&](int l) {
 #pragma unroll
@@ -213,29 +217,29 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_forward(const __bf16 *__
       const int c = n0 + j * 16 + g * 4;
       const floatx4 b = *(const floatx4 *)(s_bias + l * H + c);
 #pragma unroll
-      for (int i = 0; i < RT; ++i) {
+      for (int i = 0; i < RW; ++i) {
         bf16x4 v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (__bf16)fmaxf(acc[i][j][r] + b[r], 0.0f);
-        *(bf16x4 *)(out + rows_at<NK>(i, fr, c)) = v;
+        *(bf16x4 *)(out + rows_at<NK>(i0 + i, fr, c)) = v;
         if (KEEP) {
-          const int64_t row = row0 + i * 16 + fr;
+          const int64_t row = row0 + (i0 + i) * 16 + fr;
           if (row >= M)
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (__bf16)0.0f;
-          if (row < padded_rows(M)) *(bf16x4 *)(keep.y[l] + row0 * H + rows_at<NK>(i, fr, c)) = v;
+          if (row < padded_rows(M)) *(bf16x4 *)(keep.y[l] + row0 * H + rows_at<NK>(i0 + i, fr, c)) = v;
         }
       }
     }
     __syncthreads();
     __bf16 *t = in; in = out; out = t;
   };
-  rows_zero<RT, CT>(acc);
-  rows_mma0<RT, CT, NK>(acc, w0, in, lane);
+  rows_zero<RW, CT>(acc);
+  rows_mma0<RW, CT, NK>(acc, w0, in + i0 * NK * 512, lane);
   finish(0);
   for (int l = 1; l < L - 1; ++l) {
-    rows_zero<RT, CT>(acc);
-    rows_mma<RT, CT, NK>(acc, w, in, lane, tiles(l + 1), step(l + 1));
+    rows_zero<RW, CT>(acc);
+    rows_mma<RW, CT, NK>(acc, w, in + i0 * NK * 512, lane, tiles(l + 1), step(l + 1));
     finish(l);
   }
   // output layer: row tiles wave, wave + 8, ...
@@ -268,18 +272,18 @@ __global__ void __launch_bounds__(ROW_THREADS) mlp_rows_forward(const __bf16 *__
   }
 }
 
-template <int H, int RT, int MODE>
+template <int H, int RT, int CG, int MODE>
 int launch_rows_forward(const __bf16 *X, int64_t ldx, int64_t M, const MlpArgs &a, const MlpKeep &keep,
                         const MlpGenerate &gen, float *Z, int64_t ldz, hipStream_t st) {
   size_t extra = (a.n_layers - 1) * H * sizeof(float);
   if (MODE == ROWS_GENERATE) extra = extra > 16 * RT * 8 * sizeof(float) ? extra : 16 * RT * 8 * sizeof(float);
   const size_t lds = rows_lds_bytes<H, RT>() + extra;
-  const void *fn = (const void *)&mlp_rows_forward<H, RT, MODE>;
+  const void *fn = (const void *)&mlp_rows_forward<H, RT, CG, MODE>;
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return 2;  // GH_EHIP
   const dim3 grid((unsigned)(MODE == ROWS_KEEP ? row_grid(M, RT) : (M + 16 * RT - 1) / (16 * RT)));
-  hipLaunchKernelGGL((mlp_rows_forward<H, RT, MODE>), grid, dim3(ROW_THREADS), lds, st, X, ldx, M, a, keep, gen, Z,
+  hipLaunchKernelGGL((mlp_rows_forward<H, RT, CG, MODE>), grid, dim3(ROW_THREADS), lds, st, X, ldx, M, a, keep, gen, Z,
                      ldz);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }

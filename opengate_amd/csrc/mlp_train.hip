@@ -493,9 +493,9 @@ extern "C" int gh_mlp_train_forward_bf16(const void *X, int64_t M, int32_t n_lay
   hipStream_t st = (hipStream_t)stream;
   const int rt = row_tiles(M);
 #define GH_ROWS(H)                                                                  \
-  (rt == 1 ? launch_rows_forward<H, 1, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)       \
-           : (rt == 2 ? launch_rows_forward<H, 2, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st) \
-                      : launch_rows_forward<H, 4, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)))
+  (rt == 1 ? launch_rows_forward<H, 1, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)       \
+           : (rt == 2 ? launch_rows_forward<H, 2, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st) \
+                      : launch_rows_forward<H, 4, 8, ROWS_KEEP>(x, k_in, M, a, keep, {}, Z, ldz, st)))
   return hidden == 256 ? GH_ROWS(256) : GH_ROWS(128);
 #undef GH_ROWS
 }
