@@ -65,6 +65,7 @@ class MLP:
         self.lib = A.load_library()
         self.sizes = list(sizes)
         self.dev = torch.device(device)
+        self.f32 = torch.float32
         self.psizes = [pad8(s) for s in sizes]
         g = torch.Generator(device="cpu").manual_seed(seed)
         self.W, self.b = [], []
@@ -201,9 +202,10 @@ class MLP:
     def _fused_args(self):
         """Pointer arrays (bytes) of the forward weight copies and the biases; what was made for
         them stays referenced by the returned list."""
-        f32, hold, at = _torch().float32, [], []
-        for l in range(len(self.W)):
-            b = self.b[l]
+        if len(self.b) < len(self.W):
+            raise IndexError("a bias for every layer is needed")
+        f32, hold, at = self.f32, [], []
+        for b in self.b:
             p = b.data_ptr()
             if p & 15 or b.dtype is not f32 or not b.is_contiguous():
                 b = b.to(f32, copy=True).contiguous()
