@@ -2567,12 +2567,18 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     const uint64_t waves = (uint64_t)lp.grid * (uint64_t)(lp.block / 64);
     const uint64_t share = (total + waves - 1) / waves;
     lp.chunk = share <= 128 ? (int32_t)std::max<uint64_t>(4, (share + 3) & ~(uint64_t)3) : (share < 4096 ? 128 : 256);
-    // A recorder's slots come from one counter, one reservation every 12 ns: several simulations that
-    // record are worked on side by side, a quarter of a wave's share at a time (16 of 400000 histories
-    // 5.3 -> 2.8 ms, of 2e6 28.3 -> 12.6, of 2e7 241 -> 121)
+    // A recorder's slots come from one counter, one reservation (of a wave's photons that leave
+    // together) every 12 ns. So a short run that records has fuller waves instead of all of them, from
+    // 256 waves on (30000 histories 261 -> 136 us, 1e5 370 -> 233), and several simulations that record
+    // are worked on side by side, a quarter of a wave's share at a time (16 of 400000 histories 5.3 ->
+    // 2.8 ms, of 2e6 28.3 -> 12.6, of 2e7 241 -> 121).
     bool records = false;
     for (int s = 0; s < ns; ++s) records |= ctx->sims[s].dev.rec_count && n_histories[s] > 0;
-    if (ns > 1 && records) lp.chunk = std::max(lp.chunk, (int32_t)std::min<uint64_t>(share / 4 & ~(uint64_t)63, 1 << 16));
+    if (records) {
+      const uint64_t fuller = std::min<uint64_t>(total / 256 & ~(uint64_t)3, 64);
+      const uint64_t apart = ns > 1 ? std::min<uint64_t>(share / 4 & ~(uint64_t)63, 1 << 16) : 0;
+      lp.chunk = std::max(lp.chunk, (int32_t)std::max(fuller, apart));
+    }
   }
   for (int s = 0; s < ns; ++s) offs[s + 1] = offs[s] + (n_histories[s] + lp.chunk - 1) / lp.chunk;
   L.total_chunks = offs[ns];
