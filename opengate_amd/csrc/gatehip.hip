@@ -877,7 +877,9 @@ transport_kernel(Launch L) {
   float ev_edep = 0.0f;
   int mode = M_DEAD;
   int clab = 0;                  // material of a pending collision (kept from the step: no second
-                                 // global read); of one outside the phantom, its complement
+                                 // global read); negative outside the phantom: the complement
+                                 // of its material, or (batched form, where 13 more registers
+                                 // would spill) -1, and the material is read again
   int ntry = 0;                  // rejected tries of a pending Compton / Rayleigh sampling
 
   // wave-uniform work state
@@ -1062,7 +1064,7 @@ transport_kernel(Launch L) {
               ecache_set(ec, ph.E, maj_tab);
               if (meta & META_COLLIDE) {
                 mode = M_COLLIDE;
-                clab = ~s.world_mat;
+                clab = BATCHED ? -1 : ~s.world_mat;
               } else {
                 mode = M_STEP;
               }
@@ -1212,7 +1214,7 @@ transport_kernel(Launch L) {
       if (mode == M_WORLD && !kill) {
         mode = world_step(s, ph, rng, ec, iv);
         if (mode == M_DEAD) kill = true;
-        else if (mode == M_COLLIDE) clab = ~s.world_mat;
+        else if (mode == M_COLLIDE) clab = BATCHED ? -1 : ~s.world_mat;
       }
       // interaction: branching, then the process (photoelectric at once, the scattering
       // samplers in bounded tries); `fin` marks a finished interaction this pass
@@ -1220,7 +1222,7 @@ transport_kernel(Launch L) {
       bool comp = false;
       float x_dep = 0.0f;   // energy given to the medium at this interaction
       const bool in_world = clab < 0;
-      const int cmat = in_world ? ~clab : clab;
+      const int cmat = !in_world ? clab : (BATCHED ? max(s.world_mat, 0) : ~clab);
       const int crow = shared_rows ? mat_tab[cmat].row : cmat;  // table row of the interaction's material
       if (mode == M_COLLIDE && !kill) {
         const float r = u01(rng);
