@@ -1371,13 +1371,14 @@ transport_kernel(Launch L) {
 // COPY_MIN_SHARE histories a value on. (With copies a power of two apart 780, 2240, 20800.) A launch
 // of several simulations works on one after the other, and its lanes add the two values of a voxel,
 // which lie in one piece, by themselves: 8 simulations of 2.5e6 histories in 16^3 voxels 9.2 -> 4.9 ms,
-// in 64^3 5.0 -> 4.3 (8.0 and 4.5 with the values in two pieces); 256 of 78000 4.24 -> 4.85, so a
-// simulation that shares its launch needs COPY_MIN_OF_MANY histories.
+// in 64^3 5.0 -> 4.3 (8.0 and 4.5 with the values in two pieces); 256 of 78000 4.24 -> 4.85, 64 of
+// 600000 in 64^3 8.7 -> 9.9, so a simulation that shares its launch needs COPY_MIN_OF_MANY histories
+// and four a voxel.
 constexpr int COPIES = 8;
 constexpr size_t COPY_MAX_VALUES = (size_t)4 << 20;
 constexpr size_t COPY_MIN_SHARE = 4;  // histories per value
 constexpr int COPY_MAX_SIMS = 256;    // of a launch: their descriptors are uploaded COPIES times
-constexpr uint64_t COPY_MIN_OF_MANY = 500000;  // histories of a simulation that shares its launch
+constexpr size_t COPY_MIN_OF_MANY = 500000;  // histories of a simulation that shares its launch
 constexpr size_t COPY_MAX_BYTES = (size_t)1 << 30;  // of a context's copies
 // values from a copy to the next: a voxel's copies lie on different memory channels
 __host__ __device__ constexpr size_t copy_pitch(size_t n) { return (n + 511) / 512 * 512 + 512 + 32; }
@@ -2384,14 +2385,15 @@ int gh_reset_phsp(gh_ctx *ctx, int32_t sim_id) {
 }
 
 // Whether this run uses the copies of the tallies, which are there when it returns true.
-static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories) {
+static bool tally_copies(gh_ctx *ctx, SimHost &h, uint64_t n_histories, bool alone) {
   const SimDev &d = h.dev;
   if (d.pos_type != GH_POS_POINT) return false;
   for (int i = 0; i < 3; ++i)
     if (!(d.pos_mat[9 + i] >= 0.0f && d.pos_mat[9 + i] <= d.L[i])) return false;
   size_t values = 0;
   for (const auto &t : h.tallies()) values += t.second;
-  if (values > COPY_MAX_VALUES || n_histories < values * COPY_MIN_SHARE) return false;
+  const size_t least = alone ? values * COPY_MIN_SHARE : std::max(COPY_MIN_OF_MANY, 4 * h.n_tally);
+  if (values > COPY_MAX_VALUES || n_histories < least) return false;
   if (!h.copies.empty()) return true;
   size_t need = 0;
   for (const auto &t : h.tallies()) need += (COPIES - 1) * copy_pitch(t.second) * sizeof(double);
@@ -2460,8 +2462,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
   L.copy_mask = 0;
   std::vector<SimHost *> copied;
   for (int s = 0; s < (ns <= COPY_MAX_SIMS ? ns : 0); ++s)
-    if ((ns == 1 || n_histories[s] >= COPY_MIN_OF_MANY) && tally_copies(ctx, ctx->sims[s], n_histories[s]))
-      copied.push_back(&ctx->sims[s]);
+    if (tally_copies(ctx, ctx->sims[s], n_histories[s], ns == 1)) copied.push_back(&ctx->sims[s]);
   if (!copied.empty()) {
     L.copy_mask = COPIES - 1;
     devs.resize((size_t)COPIES * ns);
