@@ -2578,7 +2578,7 @@ int gh_run(gh_ctx *ctx, const uint64_t *n_histories, const uint64_t *first_histo
     bool records = false;
     for (int s = 0; s < ns; ++s) records |= ctx->sims[s].dev.rec_count && n_histories[s] > 0;
     if (records) {
-      const uint64_t fuller = std::min<uint64_t>(total / 256 & ~(uint64_t)3, 64);
+      const uint64_t fuller = std::min<uint64_t>(total / ns / 256 & ~(uint64_t)3, 64);
       const uint64_t apart = ns > 1 ? std::min<uint64_t>(share / 4 & ~(uint64_t)63, 1 << 16) : 0;
       lp.chunk = std::max(lp.chunk, (int32_t)std::max(fuller, apart));
     }
